@@ -139,7 +139,10 @@ def _s8_fp32(x: torch.Tensor, mode: str = "fp32") -> torch.Tensor:
     vb = v.reshape(-1, r, c)
     out = torch.empty_like(vb)
     _native.s8(vb, out, _native.S8_MODES[mode])
-    return (out.reshape(v.shape) * S8_MULTIPLIER).to(x.device)
+    out = out.reshape(v.shape)
+    if S8_MULTIPLIER != 1.0:  # the recipe's multiplier is 1: no pass for it
+        out = out * S8_MULTIPLIER
+    return out.to(x.device)
 
 
 _PARAM_DTYPES = (torch.float32, torch.bfloat16, torch.float16)
