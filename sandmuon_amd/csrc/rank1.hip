@@ -14,8 +14,8 @@
 //                      out = V1 + (rc u_i) rz_j
 //   mapback (order 1): V1 = X + (lc lz_i) t_j;  V2 = V1 + (rc u_i) rz_j;
 //                      out = (V2 li) ri
-// in three launches: column sums (threads over columns, rows walked in
-// order: coalesced), row sums (one wave per row), elementwise output.
+// in two launches: column sums (a block per 32 columns, 32 row groups),
+// then the rows (one wave per row: its sum, then its output).
 #include "common.h"
 
 #include <algorithm>
@@ -32,7 +32,6 @@ struct Rank1Args {
   const T *li, *lz, *lc;  // [batch][rows], [batch][rows], [batch]
   const T *ri, *rz, *rc;  // [batch][cols], [batch][cols], [batch]
   double *t;              // [batch][cols] column sums lz^T V
-  double *u;              // [batch][rows] row sums V1 rz
   int32_t order;
 };
 
@@ -50,59 +49,91 @@ __device__ __forceinline__ T r1_v1(const Rank1Args<T> &a, int64_t b, int64_t i, 
   return r1_v0(a, b, i, j) + (a.lc[b] * a.lz[b * a.rows + i]) * t;
 }
 
-// t[b][j] = sum_i lz_i V0_ij; grid (ceil(cols / 256), batch).
+// t[b][j] = sum_i lz_i V0_ij: a block takes kColTile columns, its kColRows
+// row groups every kColRows-th row each, kColUnroll loads in flight per
+// thread, then the groups in order through LDS.  Bound by latency at helper
+// sizes: a thread's chain is rows / kColRows terms (one chain of all rows
+// per column: 173 us for [4, 640, 1280], this one 11).
+// grid (ceil(cols / kColTile), batch), block kColTile x kColRows.
+constexpr int kColTile = 32, kColRows = 32, kColUnroll = 4;
 template <typename T>
-__global__ void __launch_bounds__(256) rank1_colsum_kernel(Rank1Args<T> a) {
+__global__ void __launch_bounds__(kColTile * kColRows) rank1_colsum_kernel(Rank1Args<T> a) {
+  __shared__ double part[kColRows][kColTile];
   const int64_t b = blockIdx.y;
-  const int64_t j = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (j >= a.cols) return;
+  const int lane = threadIdx.x % kColTile, grp = threadIdx.x / kColTile;
+  const int64_t j = static_cast<int64_t>(blockIdx.x) * kColTile + lane;
   double s = 0.0;
-  for (int64_t i = 0; i < a.rows; ++i)
-    s += static_cast<double>(a.lz[b * a.rows + i]) * static_cast<double>(r1_v0(a, b, i, j));
-  a.t[b * a.cols + j] = s;
+  if (j < a.cols)
+    for (int64_t i0 = grp; i0 < a.rows; i0 += kColRows * kColUnroll) {
+      double lz[kColUnroll], v[kColUnroll];
+#pragma unroll
+      for (int u = 0; u < kColUnroll; ++u) {
+        const int64_t i = i0 + kColRows * u;
+        const bool in = i < a.rows;
+        lz[u] = in ? static_cast<double>(a.lz[b * a.rows + i]) : 0.0;
+        v[u] = in ? static_cast<double>(r1_v0(a, b, i, j)) : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < kColUnroll; ++u)
+        if (i0 + kColRows * u < a.rows) s += lz[u] * v[u];
+    }
+  part[grp][lane] = s;
+  __syncthreads();
+  if (grp == 0 && j < a.cols) {
+    for (int g = 1; g < kColRows; ++g) s += part[g][lane];
+    a.t[b * a.cols + j] = s;
+  }
 }
 
-// u[b][i] = sum_j V1_ij rz_j, one wave per row; grid (ceil(rows / 4), batch).
+// One wave per row: u_i = sum_j V1_ij rz_j (FP64), then the output of the
+// row, which it reads a second time from cache; kRowUnroll loads in flight
+// per lane.  (Row sums and an output pass with a thread per element as two
+// launches: 12 + 12 us for [4, 640, 1280].)  grid (ceil(rows / 4), batch).
+constexpr int kRowUnroll = 4;
 template <typename T>
-__global__ void __launch_bounds__(256) rank1_rowsum_kernel(Rank1Args<T> a) {
+__global__ void __launch_bounds__(256) rank1_row_kernel(Rank1Args<T> a) {
   const int64_t b = blockIdx.y;
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (i >= a.rows) return;  // wave-uniform
   double s = 0.0;
-  for (int64_t j = lane; j < a.cols; j += 64)
-    s += static_cast<double>(r1_v1(a, b, i, j)) * static_cast<double>(a.rz[b * a.cols + j]);
-  s = wave_sum(s);
-  if (lane == 0) a.u[b * a.rows + i] = s;
-}
-
-// Elementwise output; grid (ceil(rows * cols / 256), batch).
-template <typename T>
-__global__ void __launch_bounds__(256) rank1_out_kernel(Rank1Args<T> a) {
-  const int64_t b = blockIdx.y;
-  const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (e >= a.rows * a.cols) return;
-  const int64_t i = e / a.cols, j = e % a.cols;
-  const T u = static_cast<T>(a.u[b * a.rows + i]);
-  T v = r1_v1(a, b, i, j) + (a.rc[b] * u) * a.rz[b * a.cols + j];
-  if (a.order == 1) v = (v * a.li[b * a.rows + i]) * a.ri[b * a.cols + j];
-  a.out[b * a.rows * a.cols + e] = v;
+  for (int64_t j0 = lane; j0 < a.cols; j0 += 64 * kRowUnroll) {
+    double v[kRowUnroll], rz[kRowUnroll];
+#pragma unroll
+    for (int u = 0; u < kRowUnroll; ++u) {
+      const int64_t j = j0 + 64 * u;
+      const bool in = j < a.cols;
+      v[u] = in ? static_cast<double>(r1_v1(a, b, i, j)) : 0.0;
+      rz[u] = in ? static_cast<double>(a.rz[b * a.cols + j]) : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < kRowUnroll; ++u)
+      if (j0 + 64 * u < a.cols) s += v[u] * rz[u];
+  }
+  const T u = static_cast<T>(wave_sum(s));
+  const T cu = a.rc[b] * u, li = a.li[b * a.rows + i];
+  T *out = a.out + (b * a.rows + i) * a.cols;
+  for (int64_t j0 = lane; j0 < a.cols; j0 += 64 * kRowUnroll) {
+#pragma unroll
+    for (int q = 0; q < kRowUnroll; ++q) {
+      const int64_t j = j0 + 64 * q;
+      if (j >= a.cols) continue;
+      T v = r1_v1(a, b, i, j) + cu * a.rz[b * a.cols + j];
+      if (a.order == 1) v = (v * li) * a.ri[b * a.cols + j];
+      out[j] = v;
+    }
+  }
 }
 
 template <typename T>
 static int launch_rank1(const Rank1Args<T> &a, int64_t batch, hipStream_t st) {
   const unsigned nb = static_cast<unsigned>(batch);
-  hipLaunchKernelGGL(rank1_colsum_kernel<T>, dim3(static_cast<unsigned>(ceil_div(a.cols, 256)), nb), dim3(256), 0,
-                     st, a);
+  hipLaunchKernelGGL(rank1_colsum_kernel<T>, dim3(static_cast<unsigned>(ceil_div(a.cols, kColTile)), nb),
+                     dim3(kColTile * kColRows), 0, st, a);
   int rc = check_launch("rank1_apply column sums");
   if (rc) return rc;
-  hipLaunchKernelGGL(rank1_rowsum_kernel<T>, dim3(static_cast<unsigned>(ceil_div(a.rows, 4)), nb), dim3(256), 0, st,
-                     a);
-  rc = check_launch("rank1_apply row sums");
-  if (rc) return rc;
-  hipLaunchKernelGGL(rank1_out_kernel<T>, dim3(static_cast<unsigned>(ceil_div(a.rows * a.cols, 256)), nb), dim3(256),
-                     0, st, a);
-  return check_launch("rank1_apply output");
+  hipLaunchKernelGGL(rank1_row_kernel<T>, dim3(static_cast<unsigned>(ceil_div(a.rows, 4)), nb), dim3(256), 0, st, a);
+  return check_launch("rank1_apply rows");
 }
 
 // ---------------------------------------------------- inverse sqrt ---
@@ -220,18 +251,18 @@ extern "C" int smx_rank1_apply(int dtype, const void *x, void *out, int64_t batc
   SMX_REQUIRE(out != x, SMX_EINVAL, "rank1_apply: out must not alias x");
   if (batch == 0) return SMX_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  double *t = work, *u = work + batch * cols;
+  double *t = work;
   if (dtype == SMX_F32) {
     Rank1Args<float> a{static_cast<const float *>(x), static_cast<float *>(out), rows, cols,
                        static_cast<const float *>(li), static_cast<const float *>(lz), static_cast<const float *>(lc),
                        static_cast<const float *>(ri), static_cast<const float *>(rz), static_cast<const float *>(rc),
-                       t, u, order};
+                       t, order};
     return launch_rank1(a, batch, st);
   }
   Rank1Args<double> a{static_cast<const double *>(x), static_cast<double *>(out), rows, cols,
                       static_cast<const double *>(li), static_cast<const double *>(lz),
                       static_cast<const double *>(lc), static_cast<const double *>(ri),
-                      static_cast<const double *>(rz), static_cast<const double *>(rc), t, u, order};
+                      static_cast<const double *>(rz), static_cast<const double *>(rc), t, order};
   return launch_rank1(a, batch, st);
 }
 

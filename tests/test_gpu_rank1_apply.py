@@ -1,0 +1,32 @@
+"""smx_rank1_apply at the edges of its column tiles (32), row groups (32, four
+rows in flight) and row loops (64 columns, four in flight), against the same
+formula in float64.  The bound: FP64 sums, so an element carries the few
+FP32 roundings of its own expression (eps32 = 6e-8 each)."""
+import pytest
+import torch
+
+from oracle import sandmuon_oracle as O
+from sandmuon_amd.optimizer import rank1_mapback, rank1_whiten
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-6), (torch.float64, 1e-13)])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 2, 33), (2, 31, 32), (1, 33, 65), (2, 128, 255), (1, 129, 257),
+                                   (1, 300, 1025), (70, 5, 7)])
+def test_rank1_apply_edges(device, dtype, tol, shape):
+    b, r, c = shape
+    g = torch.Generator().manual_seed(b + 10 * r + 100 * c)
+    x = torch.randn(shape, generator=g, dtype=dtype)
+    fac = lambda n: (torch.rand(b, n, generator=g, dtype=dtype) + .5, torch.randn(b, n, generator=g, dtype=dtype) * .3,
+                     -torch.rand(b, generator=g, dtype=dtype) * .5)
+    left, right = fac(r), fac(c)
+    up = lambda f: tuple(t.double() for t in f)
+    got = rank1_whiten(x.to(device), left, right)
+    want = O.rank1_whiten(x.double(), up(left), up(right))
+    assert got.dtype == dtype and (got.cpu().double() - want).norm() <= tol * want.norm()
+    got = rank1_mapback(x.to(device), left, right).cpu().double()
+    for k in range(b):
+        one = lambda f: tuple(t[k].double() for t in f)
+        want = O.rank1_mapback(x[k].double(), one(left), one(right))
+        assert (got[k] - want).norm() <= tol * want.norm()
