@@ -57,8 +57,14 @@ enum smx_status {
 enum smx_dtype { SMX_F32 = 0, SMX_BF16 = 1, SMX_F16 = 2, SMX_F64 = 3 };
 
 /* Arithmetic of the S8 polar map.
- * SMX_S8_FP32: every product on FP32 MFMA (v_mfma_f32_32x32x2_f32), FP32
- *   intermediates.  Restates sandmuon/optimizer.py:69-93.
+ * SMX_S8_FP32: FP32 accuracy, restating sandmuon/optimizer.py:69-93: every
+ *   product as three FP16 MFMAs on hi/lo splits (hi*lo + lo*hi + hi*hi,
+ *   v_mfma_f32_32x32x16_f16, FP32 accumulation); every operand is scaled by
+ *   a power of two into FP16's range and held as the FP16 hi/lo pair (22
+ *   significant bits).  Against FP64 it is as close as FP32 MFMAs on FP32
+ *   operands, which round the accumulator eight times as often; those
+ *   (v_mfma_f32_32x32x2_f32) still run in a matrix step that has 16-bit
+ *   parameters, whose bits it keeps.
  * SMX_S8_COMP_BF16: every product as three BF16 MFMAs on hi/lo splits
  *   (hi*lo + lo*hi + hi*hi, FP32 accumulation); intermediates are stored as
  *   the BF16 hi/lo pair.  The compensated-product scheme of
@@ -382,7 +388,8 @@ int smx_s8(const float *x, float *out, int64_t batch, int64_t rows,
  * padded columns exceed their padded rows)
  * and the MFMA FLOPs the launch (or run) issues (tiles computed x
  * 2*256*256*K, x3 in SMX_S8_COMP_BF16 mode, plus the square phase's
- * one-hot MFMAs).  It returns the number of records or a negative status.
+ * one-hot MFMAs; SMX_S8_FP32 counts one product per element pair, a third
+ * of what it issues).  It returns the number of records or a negative status.
  * The recorder is process-wide, not thread-safe.
  * ------------------------------------------------------------------ */
 int smx_s8_timing(int32_t enable);

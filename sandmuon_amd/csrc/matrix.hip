@@ -1327,6 +1327,8 @@ extern "C" int smx_matrix_step(const smx_matrix_desc *descs, int32_t n, int mode
     if (!plan_s8(r.data(), c.data(), fl.get(), m, mode, static_cast<char *>(workspace), plan, cls.data(),
                  slot.data()))
       return fail(SMX_EINVAL, "matrix_step: internal shape grouping error");
+    plan.layout.keep_bits = std::any_of(g.begin(), g.end(), [&](int32_t i) { return descs[i].param_dtype != SMX_F32; });
+    s8_choose_pairs(plan.layout);
     MatJob *table = reinterpret_cast<MatJob *>(static_cast<char *>(workspace) + plan.bytes);
     // Table order (one whiten launch each): parameters kept as they are,
     // except those of the next bucket; parameters kept as they are whose

@@ -88,6 +88,13 @@ struct S8Layout {
   int32_t n_classes;
   int32_t mode;
   int32_t rowsums;  // the stage-5 apply writes the mapback row-sum partials (matrix step)
+  // Matrices of 16-bit parameters: the arithmetic is not replaced by one that
+  // agrees to rounding only (FP16 pairs in the place of FP32 MFMAs).  Where an
+  // update is rounded to 8 or 11 bits, a last-place difference of the
+  // direction moves single weights by a whole last place, so such runs keep
+  // the bits they had.
+  int32_t keep_bits;
+  int32_t pairs;  // SMX_S8_FP32 on FP16 pairs (s8_choose_pairs)
 };
 
 __host__ __device__ inline int64_t sym_tiles(int64_t t) { return t * (t + 1) / 2; }
@@ -158,6 +165,16 @@ __device__ __forceinline__ uint16_t bf16_lo_bits(float v) {
   return bf16_bits(v - static_cast<float>(static_cast<__bf16>(v)));
 }
 
+// The same halves in FP16 (v scaled into FP16's range).
+__device__ __forceinline__ uint16_t f16_bits(float v) { return __builtin_bit_cast(uint16_t, static_cast<_Float16>(v)); }
+__device__ __forceinline__ uint16_t f16_lo_bits(float v) {
+  return f16_bits(v - static_cast<float>(static_cast<_Float16>(v)));
+}
+template <bool F16>
+__device__ __forceinline__ uint16_t hi_bits(float v) { return F16 ? f16_bits(v) : bf16_bits(v); }
+template <bool F16>
+__device__ __forceinline__ uint16_t lo_bits(float v) { return F16 ? f16_lo_bits(v) : bf16_lo_bits(v); }
+
 // Operand-form stores at the FP32 element index idx (tiled_index of the
 // element; the elements of one store lie in one 16-element group).
 __device__ __forceinline__ void put_operand(float *base, int64_t idx, float v, bool planes) {
@@ -196,16 +213,17 @@ __device__ __forceinline__ void put_operand4(float *base, int64_t idx, const flo
 typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
 typedef float f32x4v __attribute__((ext_vector_type(4)));
+template <bool F16 = false>
 __device__ __forceinline__ void put_operand4_paired(SMX_GLOBAL float *base, int64_t idx, const float (&v)[4],
                                                     bool planes, bool pair) {
   if (!planes) {
     *reinterpret_cast<SMX_GLOBAL f32x4v *>(base + idx) = f32x4v{v[0], v[1], v[2], v[3]};
     return;
   }
-  const uint32_t h0 = bf16_bits(v[0]) | (uint32_t(bf16_bits(v[1])) << 16);
-  const uint32_t h1 = bf16_bits(v[2]) | (uint32_t(bf16_bits(v[3])) << 16);
-  const uint32_t l0 = bf16_lo_bits(v[0]) | (uint32_t(bf16_lo_bits(v[1])) << 16);
-  const uint32_t l1 = bf16_lo_bits(v[2]) | (uint32_t(bf16_lo_bits(v[3])) << 16);
+  const uint32_t h0 = hi_bits<F16>(v[0]) | (uint32_t(hi_bits<F16>(v[1])) << 16);
+  const uint32_t h1 = hi_bits<F16>(v[2]) | (uint32_t(hi_bits<F16>(v[3])) << 16);
+  const uint32_t l0 = lo_bits<F16>(v[0]) | (uint32_t(lo_bits<F16>(v[1])) << 16);
+  const uint32_t l1 = lo_bits<F16>(v[2]) | (uint32_t(lo_bits<F16>(v[3])) << 16);
   const bool odd = (threadIdx.x & 1) != 0;
   // the partner's hi (to an even lane) or lo (to an odd lane)
   const uint32_t x0 = dpp_mov<0xB1>(odd ? h0 : l0), x1 = dpp_mov<0xB1>(odd ? h1 : l1);
@@ -221,25 +239,6 @@ __device__ __forceinline__ void put_operand4_paired(SMX_GLOBAL float *base, int6
   }
 }
 
-// Eight consecutive elements starting at idx (idx % 8 == 0): one 16-byte
-// store per BF16 half, or two for FP32.
-__device__ __forceinline__ void put_operand8(float *base, int64_t idx, const float (&v)[8], bool planes) {
-  if (planes) {
-    uint32_t hw[4], lw[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      hw[e] = bf16_bits(v[2 * e]) | (static_cast<uint32_t>(bf16_bits(v[2 * e + 1])) << 16);
-      lw[e] = bf16_lo_bits(v[2 * e]) | (static_cast<uint32_t>(bf16_lo_bits(v[2 * e + 1])) << 16);
-    }
-    uint16_t *h = reinterpret_cast<uint16_t *>(base) + plane_hi(idx);
-    *reinterpret_cast<uint4 *>(h) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
-    *reinterpret_cast<uint4 *>(h + 16) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
-  } else {
-    *reinterpret_cast<float4 *>(base + idx) = make_float4(v[0], v[1], v[2], v[3]);
-    *reinterpret_cast<float4 *>(base + idx + 4) = make_float4(v[4], v[5], v[6], v[7]);
-  }
-}
-
 // Host-side planning of a set of matrices into classes.
 struct S8Plan {
   S8Layout layout;
@@ -251,6 +250,11 @@ struct S8Plan {
 // class/slot of each matrix.  Returns false if more than kMaxClasses shapes.
 bool plan_s8(const int64_t *r, const int64_t *c, const bool *flips, int32_t n, int mode,
              char *base, S8Plan &plan, int32_t *cls_of, int32_t *slot_of);
+
+// Sets `pairs`, and the classes' iteration form under it.  To be called once
+// a layout's keep_bits is set, before its results are located
+// (S8Mat::result).
+void s8_choose_pairs(S8Layout &layout);
 
 // Run the five S8 stages on a planned layout whose x0 and input norms
 // (cst()[kCstFro]) are filled.  The result of each matrix is in S8Mat::result().

@@ -40,7 +40,17 @@
 // epilogue reads G.
 //
 // Arithmetic modes:
-//   SMX_S8_FP32       v_mfma_f32_32x32x2_f32 on FP32 operands.
+//   SMX_S8_FP32       v_mfma_f32_32x32x2_f32 on FP32 operands (S8Layout::
+//                     keep_bits: the matrices of 16-bit parameters), or as
+//                     kS8Pair: every operand, scaled by a power of two into
+//                     FP16's range (kExpX ...), an FP16 pair hi + lo of 22
+//                     significant bits in the place of FP32's 24; acc +=
+//                     lo*hi + hi*lo + hi*hi with v_mfma_f32_32x32x16_f16 and
+//                     FP32 accumulation.  One rounding of the accumulator
+//                     per 16 products instead of one per two makes the map
+//                     no further from FP64 than the FP32 MFMAs, at a fifth
+//                     of their matrix cycles (36 matrices of 768 x 768:
+//                     2755 -> 1175 us a call; error 4.4e-6 -> 2.4e-6).
 //   SMX_S8_COMP_BF16  every operand is stored by its producer as BF16 hi +
 //                     lo (put_operand); acc += hi*lo + lo*hi + hi*hi with
 //                     v_mfma_f32_32x32x16_bf16 (the compensated product of
@@ -129,8 +139,13 @@ constexpr int kMaxSeg = 2 * kMaxClasses;
 //              code would otherwise outgrow the instruction cache).
 constexpr int kS8HiOnly = 3;
 constexpr int kS8F16 = 4;
+//   kS8Pair    SMX_S8_FP32 on FP16 pairs (above).
 constexpr int kS8CompMix = 5;
+constexpr int kS8Pair = 6;
 __host__ __device__ constexpr bool is_comp(int m) { return m == SMX_S8_COMP_BF16 || m == kS8CompMix; }
+// Operands split into a hi and a lo plane, three products per K: BF16 pairs
+// (is_comp) or FP16 pairs (kS8Pair).
+__host__ __device__ constexpr bool is_split(int m) { return is_comp(m) || m == kS8Pair; }
 // Bit k-1 set: stage k of SMX_S8_COMP_BF16 is compensated.
 static int g_comp_mask = 0x1f;
 
@@ -140,10 +155,32 @@ __host__ __device__ constexpr int form_of(int gemm_mode) {
   return gemm_mode == SMX_S8_FP32 ? kFormF32 : gemm_mode == kS8F16 ? kFormF16 : kFormPlanes;
 }
 
+// Binary exponents of the kS8Pair operands: an FP16 pair of v holds v 2^e.
+// Over the whole input interval of the map (singular values of the stage-1
+// operand at most 1/1.35 of the Schatten scale) the spectral norms, which
+// bound every entry, are at most 2.0 for X, 3.97 for G, 11.07 for P1 and 4.11
+// for the later P, 3.45 for T and 45.4 for Q, so no value reaches the FP16
+// maximum of 65504, and the lo half keeps 11 more bits of every value above
+// 2^-(13 + e) (below that, an absolute 2^-(25 + e)).  X0 holds V 2^k with
+// ||V|| 2^k in [2^14, 2^15) (s8_exp0).  The products fold their operands'
+// exponents into the epilogue's scale: exact.
+constexpr int kExpX = 14, kExpG = 13, kExpP = 12, kExpT = 13, kExpQ = 10;
+static_assert(kExpT == kExpG, "P G -> T and T P -> G have one scale");
+__host__ __device__ constexpr float pow2f(int e) {
+  float v = 1.f;
+  for (int i = 0; i < (e < 0 ? -e : e); ++i) v *= e < 0 ? 0.5f : 2.f;
+  return v;
+}
+__device__ __forceinline__ int s8_exp0(double fro2) {
+  int e = 0;
+  if (fro2 > 0.0 && fro2 < 1e300) frexp(sqrt(fro2), &e);  // ||V|| in [2^(e-1), 2^e)
+  return fro2 > 0.0 ? 15 - e : 0;
+}
+
 // The MFMA mode of one product of the map (phase, stage and, for SYM and
 // APPLY, its SegOp) under the run's public `mode` and compensation mask.
 __host__ __device__ constexpr int gemm_mode(int mode, int mask, int phase, int stage, int op, bool gs) {
-  return mode == SMX_S8_FP32 ? SMX_S8_FP32
+  return mode == SMX_S8_FP32 || mode == kS8Pair ? mode
          : mode == SMX_S8_COMP_BF16 ? (((mask >> (stage - 1)) & 1) ? SMX_S8_COMP_BF16 : kS8HiOnly)
          : (stage <= 2 || gs) ? kS8CompMix
                               : kS8F16;
@@ -248,6 +285,7 @@ struct StageArgs {
   int32_t mask;      // compensated stages of SMX_S8_COMP_BF16 (bit k-1: stage k)
   float a, b, c;
   float b_over_c;
+  float ah, bh_over_c;  // the same polynomial in H = G - I (kS8Pair, X-space): a + b + c and (b + 2 c) / c
 };
 
 // A K-contiguous GEMM operand with rows of `ld` elements: FP32, or BF16
@@ -457,6 +495,8 @@ template <>
 struct AFrag<kS8F16> : AFrag<SMX_S8_COMP_BF16> {};  // h: K 0-15, l: K 16-31 (FP16 bits)
 template <>
 struct AFrag<kS8CompMix> : AFrag<SMX_S8_COMP_BF16> {};
+template <>
+struct AFrag<kS8Pair> : AFrag<SMX_S8_COMP_BF16> {};  // FP16 bits
 template <int MODE>
 struct BFrags;
 template <>
@@ -473,11 +513,13 @@ template <>
 struct BFrags<kS8F16> : BFrags<SMX_S8_COMP_BF16> {};
 template <>
 struct BFrags<kS8CompMix> : BFrags<SMX_S8_COMP_BF16> {};
+template <>
+struct BFrags<kS8Pair> : BFrags<SMX_S8_COMP_BF16> {};  // FP16 bits
 
 // Both 16-byte chunks of a row's K slice are read (the lo plane, or FP16's
 // second 16 K).
 template <int MODE>
-constexpr bool two_chunks() { return is_comp(MODE) || MODE == kS8F16; }
+constexpr bool two_chunks() { return is_split(MODE) || MODE == kS8F16; }
 
 // LDS -> registers: A row block i, and the four B column blocks, of one
 // stage.  Lane (r, h) takes K = 8h .. 8h+7 of its row: chunks h (hi) and
@@ -598,7 +640,7 @@ __device__ __forceinline__ void load_b_km(const char *st, int wn, BFrags<MODE> &
 #pragma unroll
     for (int j = 0; j < kSubN; ++j) {
 #pragma unroll
-      for (int pl = 0; pl < (is_comp(MODE) ? 2 : 1); ++pl) {
+      for (int pl = 0; pl < (is_split(MODE) ? 2 : 1); ++pl) {
         lds_char *p = q[pl] + (kOpA + 2 * j * 1024);
         const i16x4 lo = read_tr16(p), hi = read_tr16(p + 4 * 64);
         const bf16x8 v = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -642,6 +684,17 @@ __device__ __forceinline__ void mma_row(const AFrag<MODE> &a, const BFrags<MODE>
   } else if constexpr (MODE == kS8HiOnly) {
 #pragma unroll
     for (int j = 0; j < kSubN; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], a.h, acc[j], 0, 0, 0);
+  } else if constexpr (MODE == kS8Pair) {
+    // The same on FP16 pairs (lo*lo, 2^-24 of the product, is left out).
+#pragma unroll
+    for (int j = 0; j < kSubN; ++j)
+      acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.l[j]), as_f16(a.h), acc[j], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < kSubN; ++j)
+      acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.h[j]), as_f16(a.l), acc[j], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < kSubN; ++j)
+      acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.h[j]), as_f16(a.h), acc[j], 0, 0, 0);
   } else if constexpr (MODE == kS8F16) {
     // K 0-15, then K 16-31 of the stage.
 #pragma unroll
@@ -672,7 +725,7 @@ __device__ __forceinline__ AFrag<MODE> one_hot(float s, int r0) {
   const int lane = threadIdx.x & 63;
   const int e = (lane & 31) - r0 - 8 * (lane >> 5);  // position of k = row - R in this lane's 8
   AFrag<MODE> f;
-  if constexpr (MODE == kS8F16) {
+  if constexpr (MODE == kS8F16 || MODE == kS8Pair) {
     // s as the FP16 pair hi + lo (22 bits), hi in h, lo in l.
     const _Float16 sh = static_cast<_Float16>(s);
     const _Float16 sl = static_cast<_Float16>(s - static_cast<float>(sh));
@@ -701,8 +754,8 @@ __device__ __forceinline__ AFrag<MODE> one_hot(float s, int r0) {
   return f;
 }
 
-// acc[i] += s G over the rows of the one-hot window stage: the compensated
-// recipe's three products of the (hi, lo) scalar and B planes; a plain BF16
+// acc[i] += s G over the rows of the one-hot window stage: the split
+// operands' three products of the (hi, lo) scalar and B planes; a plain BF16
 // stage the scalar's hi and lo against B's hi plane (a BF16 scalar alone
 // would misscale the linear term of P by up to 2^-9); FP16 the scalar's hi
 // and lo against the stage's first 16 K (rows r0 = 0 .. 15 of the block)
@@ -1074,6 +1127,14 @@ s8_stage_kernel(StageArgs args) {
   float *x_out = odd ? M.x1() : M.x0();
 
   f32x16 acc[kSubM][kSubN];
+  // What the epilogue multiplies by; kPair: with the exponents of the FP16
+  // pairs (kExpX ...) folded in.
+  constexpr bool kPair = MODE == kS8Pair;
+  // X-space pairs: from stage 2 on the Gram is stored as H = G - I and P is
+  // formed from it.  The iterate's singular values approach 1, so H is small
+  // where G is not: neither the rounding of a diagonal near 1 nor the
+  // cancellation of a + b G + c G^2 there reaches P.
+  const bool shift = kPair && stage != 1 && !K.gs;
   float scale = 1.f;
   float *sym_out = nullptr;  // SYM: the product's destination
   // Gram space (see the header): a segment's first Q sits in qa; Q' = P Q
@@ -1093,12 +1154,15 @@ s8_stage_kernel(StageArgs args) {
         scale = sc.ok ? 1.0f / (sc.s * sc.s) : 0.f;
       }
     }
+    if constexpr (kPair) scale *= pow2f(-kExpP);  // P G -> T, T P -> G
     gemm_tile<MODE, Gm, false, false, MODE == kS8CompMix>(Opnd{A, K.rp}, Opnd{B, K.rp}, K.rp, tm * Gm::kTileM,
                                                          tn * kTileN, 0.f, smem, acc);
   } else if constexpr (PHASE == kGram) {
     if (stage == 1) {
       const double f = M.cst()[kCstFro];
-      scale = f > 0.0 ? static_cast<float>(1.0 / f) : 0.f;
+      scale = f > 0.0 ? static_cast<float>(kPair ? ldexp(1.0 / f, kExpG - 2 * s8_exp0(f)) : 1.0 / f) : 0.f;
+    } else if constexpr (kPair) {
+      scale = pow2f(kExpG - 2 * kExpX);
     }
     // A Gram-space class takes its stage-3 Gram of X2 from x1.
     const Opnd X{K.gs && stage == 3 ? M.x1() : x_in, K.cp};
@@ -1109,11 +1173,14 @@ s8_stage_kernel(StageArgs args) {
     // the operand bases in vector registers)
     constexpr bool kUB = true;
     if (stage == 1) {
+      if constexpr (kPair) scale = pow2f(-2 * kExpG);
       gemm_tile<MODE, Gm, false, false, kUB>(G, G, K.rp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, acc);
     } else {
       // acc = G G + (b/c) G; the epilogue forms P = c acc + a I.
-      scale = args.c;
-      gemm_tile<MODE, Gm, true, false, kUB>(G, G, K.rp, tm * Gm::kTileM, tn * kTileN, args.b_over_c, smem, acc);
+      scale = kPair ? args.c * pow2f(kExpP - 2 * kExpG) : args.c;
+      gemm_tile<MODE, Gm, true, false, kUB>(G, G, K.rp, tm * Gm::kTileM, tn * kTileN,
+                                            kPair ? (shift ? args.bh_over_c : args.b_over_c) * pow2f(kExpG)
+                                                  : args.b_over_c, smem, acc);
     }
   } else {
     // X-space: X' = P X (stage 1: X' = P1 V / (||V|| s)).  Gram space:
@@ -1122,7 +1189,14 @@ s8_stage_kernel(StageArgs args) {
     const bool gq = op == kOpApplyQ, mid = op == kOpApplyMid, fin = op == kOpApplyFinal;
     if (stage == 1 || mid) {
       const Stage1Scalars sc = stage1_scalars(M, args.sq_geo, &bcast);
-      scale = sc.ok ? static_cast<float>(1.0 / (sqrt(sc.fro2) * static_cast<double>(sc.s))) : 0.f;
+      const double inv = sc.ok ? 1.0 / (sqrt(sc.fro2) * static_cast<double>(sc.s)) : 0.0;
+      scale = static_cast<float>(kPair ? ldexp(inv, kExpX - (mid ? kExpQ : kExpP) - s8_exp0(sc.fro2)) : inv);
+    } else if constexpr (kPair) {
+      // Q2 and Q4 are products of two P (a segment's first Q is its P);
+      // the stage-5 results are FP32 without an exponent.
+      scale = gq ? (stage == 5 ? pow2f(-kExpP) : pow2f(kExpQ - 2 * kExpP))
+              : fin ? pow2f(-kExpQ - kExpX)
+              : stage == 5 ? pow2f(-kExpP - kExpX) : pow2f(-kExpP);
     }
     const float *A = mid ? M.qb() : fin ? M.qa() : M.p();
     const Opnd B = gq ? Opnd{q_in, K.rp} : Opnd{mid ? M.x0() : fin ? M.x1() : x_in, K.cp};
@@ -1183,7 +1257,9 @@ s8_stage_kernel(StageArgs args) {
   // FP32: the mapback's and the stand-alone map's input).
   const bool tiled_t = !(PHASE == kApply && last && (ref.op == kOpApplyX || ref.op == kOpApplyFinal));
   const bool tiled_m = PHASE != kApply;
-  const bool eye = PHASE == kSquare && stage != 1;  // add a I on the diagonal
+  // add eye_a on the diagonal: a I of P, or -I of H (shift)
+  const bool eye = (PHASE == kSquare && stage != 1) || (PHASE == kGram && shift);
+  const float eye_a = !kPair ? args.a : PHASE == kGram ? -pow2f(kExpG) : (shift ? args.ah : args.a) * pow2f(kExpP);
   // the wave's staging block of a transposed output: [column][row]
   float *const U = reinterpret_cast<float *>(smem) + wave * 2 * kEpBlock;
   float sq_local = 0.f;
@@ -1271,7 +1347,7 @@ s8_stage_kernel(StageArgs args) {
       if (eye)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (gr == gc0 + ec4 + e && gr < K.r) w[e] += args.a;
+          if (gr == gc0 + ec4 + e && gr < K.r) w[e] += eye_a;
       uint32_t b[2];
 #pragma unroll
       for (int e = 0; e < 2; ++e)
@@ -1296,12 +1372,12 @@ s8_stage_kernel(StageArgs args) {
       if (eye)
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-          if (gr == gc0 + ec8 + e && gr < K.r) w[e] += args.a;
+          if (gr == gc0 + ec8 + e && gr < K.r) w[e] += eye_a;
       uint32_t b[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const uint16_t x0 = lo_plane ? bf16_lo_bits(w[2 * e]) : bf16_bits(w[2 * e]);
-        const uint16_t x1 = lo_plane ? bf16_lo_bits(w[2 * e + 1]) : bf16_bits(w[2 * e + 1]);
+        const uint16_t x0 = lo_plane ? lo_bits<kPair>(w[2 * e]) : hi_bits<kPair>(w[2 * e]);
+        const uint16_t x1 = lo_plane ? lo_bits<kPair>(w[2 * e + 1]) : hi_bits<kPair>(w[2 * e + 1]);
         b[e] = x0 | (static_cast<uint32_t>(x1) << 16);
       }
       *reinterpret_cast<uint4 *>(out) = make_uint4(b[0], b[1], b[2], b[3]);
@@ -1311,7 +1387,7 @@ s8_stage_kernel(StageArgs args) {
       if (eye)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (gr == gc0 + ec4 + e && gr < K.r) w[e] += args.a;
+          if (gr == gc0 + ec4 + e && gr < K.r) w[e] += eye_a;
       *reinterpret_cast<float4 *>(out) = make_float4(w[0], w[1], w[2], w[3]);
       if (acc_r) accum4(w, gc0 + ec4, r);
     }
@@ -1352,8 +1428,8 @@ s8_stage_kernel(StageArgs args) {
         uint32_t h[4], l[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          h[e] = bf16_bits(w[8 * g + 2 * e]) | (static_cast<uint32_t>(bf16_bits(w[8 * g + 2 * e + 1])) << 16);
-          l[e] = bf16_lo_bits(w[8 * g + 2 * e]) | (static_cast<uint32_t>(bf16_lo_bits(w[8 * g + 2 * e + 1])) << 16);
+          h[e] = hi_bits<kPair>(w[8 * g + 2 * e]) | (static_cast<uint32_t>(hi_bits<kPair>(w[8 * g + 2 * e + 1])) << 16);
+          l[e] = lo_bits<kPair>(w[8 * g + 2 * e]) | (static_cast<uint32_t>(lo_bits<kPair>(w[8 * g + 2 * e + 1])) << 16);
         }
         *reinterpret_cast<uint4 *>(out + base + 1024 * g) = make_uint4(h[0], h[1], h[2], h[3]);
         *reinterpret_cast<uint4 *>(out + base + 1024 * g + 32) = make_uint4(l[0], l[1], l[2], l[3]);
@@ -1396,7 +1472,7 @@ s8_stage_kernel(StageArgs args) {
         if (eye)
 #pragma unroll
           for (int e = 0; e < 16; ++e)
-            if (gr == cb + col16(e) && gr < K.r) w[e] += args.a;
+            if (gr == cb + col16(e) && gr < K.r) w[e] += eye_a;
         put_direct(fm_c, w, gr, cb, dst_t, ld_t, tiled_t);
         if (rs_on) {
           // a and z of the lane's columns, then the row's two lanes (lh)
@@ -1486,7 +1562,7 @@ __host__ __device__ inline int64_t poly_blocks_per_matrix(const S8Class &k) {
 template <int MODE>
 __global__ void __launch_bounds__(256) s8_poly1_kernel(StageArgs args) {
   __shared__ double bcast;
-  constexpr bool PL = MODE == SMX_S8_COMP_BF16;
+  constexpr bool kPair = MODE == kS8Pair, PL = MODE == SMX_S8_COMP_BF16 || kPair;
   const TileRef ref = tile_of(args);
   const S8Class &K = *ref.k;
   const int64_t tpm = poly_blocks_per_matrix(K);
@@ -1519,6 +1595,8 @@ __global__ void __launch_bounds__(256) s8_poly1_kernel(StageArgs args) {
   const Stage1Scalars sc = stage1_scalars(M, args.sq_geo, &bcast);
   const float s2 = sc.s * sc.s;
   const float is2 = sc.ok ? 1.0f / s2 : 0.f, is4 = sc.ok ? 1.0f / (s2 * s2) : 0.f;
+  // FP16 pairs: G holds 2^kExpG G, P1 goes out as 2^kExpP P1
+  constexpr float kOut = kPair ? pow2f(kExpP) : 1.f, kOutG = kPair ? pow2f(kExpP - kExpG) : 1.f;
 #pragma unroll
   for (int k = 0; k < kPolyUnits; ++k) {
     const float w[4] = {w4[k].x, w4[k].y, w4[k].z, w4[k].w};
@@ -1527,8 +1605,13 @@ __global__ void __launch_bounds__(256) s8_poly1_kernel(StageArgs args) {
       const uint32_t hw[2] = {gh[k].x, gh[k].y}, lw[2] = {gl[k].x, gl[k].y};
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
-        g[2 * e] = __uint_as_float(hw[e] << 16) + __uint_as_float(lw[e] << 16);
-        g[2 * e + 1] = __uint_as_float(hw[e] & 0xffff0000u) + __uint_as_float(lw[e] & 0xffff0000u);
+        if constexpr (kPair) {
+          g[2 * e] = f16_bits_to_f32(hw[e] & 0xffff) + f16_bits_to_f32(lw[e] & 0xffff);
+          g[2 * e + 1] = f16_bits_to_f32(hw[e] >> 16) + f16_bits_to_f32(lw[e] >> 16);
+        } else {
+          g[2 * e] = __uint_as_float(hw[e] << 16) + __uint_as_float(lw[e] << 16);
+          g[2 * e + 1] = __uint_as_float(hw[e] & 0xffff0000u) + __uint_as_float(lw[e] & 0xffff0000u);
+        }
       }
     } else {
       g[0] = __uint_as_float(gh[k].x); g[1] = __uint_as_float(gh[k].y);
@@ -1541,9 +1624,41 @@ __global__ void __launch_bounds__(256) s8_poly1_kernel(StageArgs args) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float eye = (row == col + e && row < K.r) ? args.a : 0.f;
-      v[e] = (eye + (args.b * g[e]) * is2) + (args.c * w[e]) * is4;
+      v[e] = (eye * kOut + (args.b * g[e] * kOutG) * is2) + (args.c * w[e] * kOut) * is4;
     }
-    put_operand4_paired(Pout, grp[k] * 16 + 4 * qt, v, PL, true);
+    put_operand4_paired<kPair>(Pout, grp[k] * 16 + 4 * qt, v, PL, true);
+  }
+}
+
+// kS8Pair: the FP32 iterate X0 that the whiten or the load left becomes
+// FP16 pairs of V 2^k, in place (a group is 64 bytes in both forms).  Only
+// here is ||V|| known, and with it the exponent; 8 bytes per element at the
+// copy rate.  Blocks and lanes as s8_poly1_kernel, over the iterate's groups.
+__host__ __device__ inline int64_t pair_blocks_per_matrix(const S8Class &k) {
+  return k.rp * k.cp / 16 / kPolyChunk;
+}
+
+__global__ void __launch_bounds__(256) s8_pair0_kernel(StageArgs args) {
+  const TileRef ref = tile_of(args);
+  const S8Class &K = *ref.k;
+  const int64_t tpm = pair_blocks_per_matrix(K);
+  if (ref.L >= tpm * ref.cnt) return;
+  const S8Mat M{K, ref.slot0 + static_cast<int>(ref.L / tpm)};
+  const int64_t g0 = (ref.L % tpm) * kPolyChunk;
+  const int qt = threadIdx.x & 3;
+  SMX_GLOBAL float *X = (SMX_GLOBAL float *)M.x0();
+  f32x4v x[kPolyUnits];
+  int64_t idx[kPolyUnits];
+#pragma unroll
+  for (int k = 0; k < kPolyUnits; ++k) {
+    idx[k] = (g0 + (threadIdx.x + 256 * k) / 4) * 16 + 4 * qt;
+    x[k] = *reinterpret_cast<const SMX_GLOBAL f32x4v *>(X + idx[k]);
+  }
+  const int e0 = s8_exp0(M.cst()[kCstFro]);
+#pragma unroll
+  for (int k = 0; k < kPolyUnits; ++k) {
+    const float v[4] = {ldexpf(x[k].x, e0), ldexpf(x[k].y, e0), ldexpf(x[k].z, e0), ldexpf(x[k].w, e0)};
+    put_operand4_paired<true>(X, idx[k], v, true, true);
   }
 }
 
@@ -1659,6 +1774,8 @@ static double launch_flops(int mode, int phase, int stage, int geo, const S8Layo
   const double prod = is_comp(mode) ? 3.0 : 1.0;
   const int tm = geo == kGeoS ? 128 : 256, tn = geo == kGeoL ? 256 : 128, waves = geo == kGeoL ? 8 : 4;
   const int sub_m = tm / 64;
+  // (kS8Pair counts one product per element pair, as the FP32 MFMAs whose
+  // place it takes issue; it is carried out as three FP16 ones.)
   const double onehot = is_comp(mode) ? 6.0 * sub_m : mode == kS8HiOnly ? 4.0 * sub_m
                         : mode == kS8F16 ? 4.0 * sub_m : 2.0 * sub_m;
   double f = 0.0;
@@ -1757,6 +1874,8 @@ static int launch_phase(const S8Layout &Lay, const SlotSet &set, int stage, int 
     a.b = static_cast<float>(co[1]);
     a.c = static_cast<float>(co[2]);
     a.b_over_c = static_cast<float>(co[1] / co[2]);
+    a.ah = static_cast<float>(co[0] + co[1] + co[2]);
+    a.bh_over_c = static_cast<float>((co[1] + 2.0 * co[2]) / co[2]);
     if (static_cast<int>(segs.size()) > kMaxSeg) return fail(SMX_EINVAL, "s8: too many launch segments");
     if (PHASE != kPoly1)
       for (const Seg &sg : segs)
@@ -1784,7 +1903,9 @@ static int launch_phase(const S8Layout &Lay, const SlotSet &set, int stage, int 
     int rc = timing_begin(st, slot, false);
     if (rc) return rc;
     if constexpr (PHASE == kPoly1) {
-      if (mode != SMX_S8_FP32)
+      if (mode == kS8Pair)
+        hipLaunchKernelGGL(s8_poly1_kernel<kS8Pair>, dim3(off), dim3(256), 0, st, a);
+      else if (mode != SMX_S8_FP32)
         hipLaunchKernelGGL(s8_poly1_kernel<SMX_S8_COMP_BF16>, dim3(off), dim3(256), 0, st, a);
       else
         hipLaunchKernelGGL(s8_poly1_kernel<SMX_S8_FP32>, dim3(off), dim3(256), 0, st, a);
@@ -1794,6 +1915,7 @@ static int launch_phase(const S8Layout &Lay, const SlotSet &set, int stage, int 
       else if (mode == kS8CompMix) launch_stage<kS8CompMix, PHASE>(geo, off, a, st);
       else if (mode == kS8HiOnly) launch_stage<kS8HiOnly, PHASE>(geo, off, a, st);
       else if (mode == kS8F16) launch_stage<kS8F16, PHASE>(geo, off, a, st);
+      else if (mode == kS8Pair) launch_stage<kS8Pair, PHASE>(geo, off, a, st);
       else launch_stage<SMX_S8_FP32, PHASE>(geo, off, a, st);
       rc = check_launch(PHASE == kGram ? "s8 gram" : PHASE == kSquare ? "s8 square" : PHASE == kSym ? "s8 sym"
                                                                                                   : "s8 apply");
@@ -1882,9 +2004,33 @@ static int fork_stream(ForkStream *&out) {
 // one record for the run, on the caller's stream.
 constexpr int kSplitCount = 2 * kChains;
 
-int run_s8_stages(const S8Layout &Lay, hipStream_t st) {
+// The FP16 pairs of every X0 of a kS8Pair run, before its chains fork.
+static int run_s8_pair0(const S8Layout &Lay, hipStream_t st) {
+  StageArgs a{};
+  a.L = Lay;
+  int32_t off = 0;
+  for (int i = 0; i < Lay.n_classes; ++i) {
+    const S8Class &k = Lay.cls[i];
+    if (!k.count) continue;
+    a.seg_off[a.n_seg] = off;
+    a.seg_cls[a.n_seg] = i;
+    a.seg_cnt[a.n_seg++] = k.count;
+    off += static_cast<int32_t>(round_up(pair_blocks_per_matrix(k) * k.count, 8));
+  }
+  a.seg_off[a.n_seg] = off;
+  if (off == 0) return SMX_OK;
+  hipLaunchKernelGGL(s8_pair0_kernel, dim3(off), dim3(256), 0, st, a);
+  return check_launch("s8 input pairs");
+}
+
+int run_s8_stages(const S8Layout &layout, hipStream_t st) {
   int slot = -1;
   int rc = timing_begin(st, slot, true);
+  S8Layout Lay = layout;
+  if (Lay.pairs) {
+    Lay.mode = kS8Pair;
+    if (!rc) rc = run_s8_pair0(Lay, st);
+  }
   if (rc) return rc;
   std::vector<int> order;
   for (int i = 0; i < Lay.n_classes; ++i)
@@ -1946,6 +2092,22 @@ int run_s8_stages(const S8Layout &Lay, hipStream_t st) {
   }
   if (rc) return rc;
   return timing_end(slot, st, kSpan, flops);
+}
+
+// SMX_S8_FP32 runs on FP16 pairs (kS8Pair) unless the bits of FP32 MFMAs are
+// kept, or a matrix of up to 32 rows is wider than 256: the pairs' 22 bits
+// cost more there than the longer accumulation of FP32 MFMAs (16 x 700: error
+// 7.2e-6 against 4.2e-6).  Small Gram-space classes then iterate in X-space,
+// where P comes from H = G - I: the r x r products of Gram space carry G
+// itself (100 x 1100: 5.9e-6 against FP32's 5.5e-6, X-space 3.4e-6), and a
+// short run takes fewer launches so (15 of 23).  From about 160 rows on
+// both are at or below FP32's error.
+void s8_choose_pairs(S8Layout &L) {
+  L.pairs = L.mode == SMX_S8_FP32 && !L.keep_bits;
+  for (int i = 0; i < L.n_classes; ++i)
+    if (L.cls[i].r <= 32 && L.cls[i].gs) L.pairs = 0;
+  for (int i = 0; i < L.n_classes && L.pairs; ++i)
+    if (L.cls[i].r <= 160) L.cls[i].gs = 0;
 }
 
 bool plan_s8(const int64_t *r, const int64_t *c, const bool *flips, int32_t n, int mode, char *base,

@@ -147,6 +147,7 @@ extern "C" int smx_s8(const float *x, float *out, int64_t batch, int64_t rows, i
   S8Plan plan;
   plan_single(batch, rows, cols, mode, static_cast<char *>(workspace), plan);
   SMX_REQUIRE(workspace_bytes >= plan.bytes, SMX_EWORKSPACE, "s8: workspace too small");
+  s8_choose_pairs(plan.layout);
   hipStream_t st = static_cast<hipStream_t>(stream);
   S8IoArgs a{};
   a.k = plan.layout.cls[0];

@@ -15,7 +15,7 @@ results):
 * ``s8_mode`` selects the arithmetic of the S8 products: "comp_bf16"
   (compensated BF16 MFMA in all five stages), "mixed" (compensated BF16
   stages 1-2, FP16 MFMA stages 3-5: about 1e-3 from the FP32 map at a
-  quarter less S8 time) or "fp32" (FP32 MFMA);
+  quarter less S8 time) or "fp32" (FP32 accuracy: FP16 pairs of 22 bits);
 * ``hook_batch_bytes``: the hooks queue their inputs and take the
   statistics of the queue in one launch once it holds this many bytes (and
   at step(), state_dict() and close()); 0 launches in every hook call.  The
@@ -133,7 +133,7 @@ def _graft_direction(value: torch.Tensor, output_rows: int) -> torch.Tensor:
 
 
 def _s8_fp32(x: torch.Tensor, mode: str = "fp32") -> torch.Tensor:
-    """S8 polar map on [..., rows, cols] (sandmuon/optimizer.py:69-93), FP32 MFMA by default."""
+    """S8 polar map on [..., rows, cols] (sandmuon/optimizer.py:69-93), at FP32 accuracy by default."""
     v = _to_gpu_f32(x)
     r, c = v.shape[-2], v.shape[-1]
     vb = v.reshape(-1, r, c)
