@@ -72,7 +72,6 @@ struct S8Class {
   float *u;            // [count][cp] per param-row rank-one coefficient
   double *fro;         // [count][parts] whiten: per-block partial sums (two kinds)
   double *mb;          // [count][parts] mapback: per-block partial sums of U^2
-  double *sch;         // [count][sym_tiles(tiles_s)] Schatten partials (one per upper-triangle Gram tile)
   double *cst;         // [count][kCst] per-matrix scalars (see the kCst* indices)
   // Matrix step only (S8Layout::rowsums): the A factor diagonal and the
   // rank-one vector (NULL without one) of each slot's matrix, and the
@@ -119,7 +118,10 @@ struct S8Mat {
   __host__ __device__ float *u() const { return kp()->u + slot * kp()->cp; }
   __host__ __device__ double *fro() const { return kp()->fro + static_cast<int64_t>(slot) * kp()->parts; }
   __host__ __device__ double *mb() const { return kp()->mb + static_cast<int64_t>(slot) * kp()->parts; }
-  __host__ __device__ double *sch() const { return kp()->sch + slot * sym_tiles(kp()->tiles_s); }
+  // Schatten partials, one per tile of the stage-1 square (at most parts of
+  // them): in the place of the whiten's (or load's), which the matrix's
+  // total has consumed.
+  __host__ __device__ double *sch() const { return fro(); }
   __host__ __device__ double *cst() const { return kp()->cst + kCst * static_cast<int64_t>(slot); }
   __host__ __device__ const float *acol() const { return kp()->colv[2 * slot]; }
   __host__ __device__ const float *zcol() const { return kp()->colv[2 * slot + 1]; }

@@ -237,9 +237,14 @@ constexpr int kBK = 16;             // K per pipeline stage
 // (its 256 A rows serve 256 B rows: cfg5 S8 7% faster).  A round of the
 // device's block slots does the same work in M and L; the host picks the
 // geometry per launch (pick_geo).
-enum TileGeo { kGeoM = 0, kGeoS = 1, kGeoL = 2 };
+//   kGeoT  64 x 64, 4 waves of 64 x 64 that each take a quarter of K
+//          (gemm_tile_split), two blocks per CU: for launches that leave
+//          CUs idle, where the length of a tile's chain of K stages is the
+//          launch's time.
+enum TileGeo { kGeoM = 0, kGeoS = 1, kGeoL = 2, kGeoT = 3 };
 template <int TM, int TN>
 struct Geo {
+  static constexpr bool kSplitK = false;
   static constexpr int kTileM = TM, kTileN = TN;
   static constexpr int kSubM = TM / 64;             // 32x32 MFMA row tiles per wave
   static constexpr int kWavesN = TN / (32 * kSubN);
@@ -260,6 +265,23 @@ struct Geo {
   static constexpr int kWavesPerEU = TM == 128 ? 3 : 2;
   static constexpr int kGeo = TN == 256 ? kGeoL : TM == 128 ? kGeoS : kGeoM;
 };
+template <>
+struct Geo<64, 64> {
+  static constexpr bool kSplitK = true;
+  static constexpr int kTileM = 64, kTileN = 64;
+  static constexpr int kSubM = 2, kWavesN = 1;  // a wave covers the whole tile
+  static constexpr int kWaves = 4;
+  static constexpr int kThreads = 64 * kWaves;
+  static constexpr int kOpA = 0;                   // only a K-major B goes through LDS
+  static constexpr int kLoadsB = 4;                // 1 KB pieces of a K-major stage
+  static constexpr int kBufBytes = 2 * 4096;       // per wave: two K-major stages
+  static constexpr int kAccBytes = 64 * 64 * 4;    // per wave: its partial sums of the tile
+  static constexpr int kRingBytes = kWaves * kAccBytes;
+  static constexpr int kKmRow = 64 * 4, kKmRowH = 64 * 2;
+  static constexpr int kWavesPerEU = 2;
+  static constexpr int kGeo = kGeoT;
+};
+using GeoT = Geo<64, 64>;
 using GeoM = Geo<256, 128>;
 using GeoS = Geo<128, 128>;
 using GeoL = Geo<256, 256>;
@@ -285,7 +307,7 @@ struct StageArgs {
   int32_t mask;      // compensated stages of SMX_S8_COMP_BF16 (bit k-1: stage k)
   float a, b, c;
   float b_over_c;
-  float ah, bh_over_c;  // the same polynomial in H = G - I (kS8Pair, X-space): a + b + c and (b + 2 c) / c
+  float ah, bh, bh_over_c;  // the same polynomial in H = G - I (kS8Pair, X-space): a + b + c, b + 2 c and (b + 2 c) / c
 };
 
 // A K-contiguous GEMM operand with rows of `ld` elements: FP32, or BF16
@@ -962,6 +984,145 @@ __device__ __forceinline__ void gemm_tile(const Opnd &A_in, const Opnd &B_in, in
   block_barrier();
 }
 
+// The same product for a 64 x 64 tile whose K is split over the block's four
+// waves (kGeoT).  Each wave keeps its whole 64 x 64 partial and loads its
+// fragments of row-major operands straight from memory, kDeep K stages
+// ahead (their 16-byte chunks are what a lane's MFMA takes, and nothing is
+// shared between waves); a K-major B goes through a wave-private LDS
+// buffer for its transposed reads.  No barrier inside the K loop.  Then the
+// partials are added through LDS in wave order, and waves 0 and 1 hold the
+// tile's 32 x 32 blocks: blocks (w, 0) and (w, 1), or, by_col, (0, w) and
+// (1, w), in acc[0][0] and acc[0][1].  Bound by latency: a launch of a
+// single 768 x 768 matrix takes 48 K stages as one chain of 21 blocks in
+// 128 x 128 tiles, here 12 in 84 blocks.
+constexpr int kDeep = 4;
+template <int MODE, bool BKM>
+__device__ __forceinline__ void gemm_tile_split(const Opnd &A_in, const Opnd &B_in, int64_t K, int64_t arow0,
+                                                int64_t brow0, char *smem, bool by_col, f32x16 (&acc)[2][kSubN]) {
+  using G = GeoT;
+  constexpr bool F16 = MODE == kS8F16;
+  constexpr int kU = F16 ? 2 : 1;  // elements per 4-byte unit
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int lr = lane & 31, lh = lane >> 5;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < kSubN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  // K is a multiple of 256 (128 pairs of FP16): nk is a multiple of 4 (2).
+  const int nk = static_cast<int>(K / (kBK * kU)) / G::kWaves;
+  const int64_t k0 = static_cast<int64_t>(wave) * nk * kBK;  // 4-byte units
+  const Opnd A{uniform_ptr(A_in.p), A_in.ld / kU}, B{uniform_ptr(B_in.p), B_in.ld / kU};
+  const SMX_GLOBAL char *ap = (const SMX_GLOBAL char *)A.p + 64 * k0;
+  const SMX_GLOBAL char *bp = (const SMX_GLOBAL char *)B.p + (BKM ? 4 * k0 * B.ld * kU : 64 * k0);
+  const int64_t bstep = BKM ? 4 * static_cast<int64_t>(kBK) * B.ld * kU : 64 * kBK;  // bytes of a K stage
+  // Row r of a 32-row block: its 16-row piece, its 64 bytes, chunk lh.
+  auto row_off = [&](int64_t row0, int r, int64_t ld) {
+    return static_cast<uint32_t>(((row0 >> 4) + (r >> 4)) * (ld >> 4) * 1024 + (r & 15) * 64 + 16 * lh);
+  };
+  uint32_t ao[2], bo[4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) ao[i] = row_off(arow0, 32 * i + lr, A.ld);
+  if constexpr (BKM) {
+    const auto t = tile_offsets_km<G::kLoadsB, F16 ? G::kKmRowH : G::kKmRow, F16 ? kKmSwzH : kKmSwzT>(B.ld, brow0 / kU, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bo[i] = t.v[i];
+  } else {
+#pragma unroll
+    for (int j = 0; j < kSubN; ++j) bo[j] = row_off(brow0, 32 * j + sw23(lr), B.ld);
+  }
+  const BkmLane bl = F16 ? bkm_lane_f16(0) : bkm_lane(0);
+  char *const buf = smem + wave * G::kBufBytes;
+  struct Stage {
+    AFrag<MODE> a[2];
+    bf16x8 b[4];  // row-major: hi and lo of each column block; K-major: the lane's chunk of each piece
+  } st[kDeep];
+  auto chunk = [](const SMX_GLOBAL char *p) { return *reinterpret_cast<const SMX_GLOBAL bf16x8 *>(p); };
+  auto load = [&](int kt, Stage &s) {
+    const SMX_GLOBAL char *a = ap + static_cast<int64_t>(64 * kBK) * kt, *b = bp + bstep * kt;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      s.a[i].h = chunk(a + ao[i]);
+      if constexpr (two_chunks<MODE>()) s.a[i].l = chunk(a + ao[i] + 32);
+    }
+    if constexpr (BKM) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s.b[i] = chunk(b + bo[i]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < kSubN; ++j) {
+        s.b[2 * j] = chunk(b + bo[j]);
+        if constexpr (two_chunks<MODE>()) s.b[2 * j + 1] = chunk(b + bo[j] + 32);
+      }
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < kDeep; ++u)
+    if (u < nk) load(u, st[u]);
+  for (int kt = 0; kt < nk; kt += kDeep) {
+    static_for<kDeep>([&](auto u_c) {
+      constexpr int u = decltype(u_c)::value;
+      if (u >= 2 && kt + u >= nk) return;  // nk is even
+      Stage &s = st[u];
+      BFrags<MODE> bf;
+      if constexpr (BKM) {
+        char *slot = buf + (u & 1) * 4096;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<bf16x8 *>(slot + i * 1024 + lane * 16) = s.b[i];
+        // (the wave's own writes: LDS keeps a wave's order)
+        asm volatile("" ::: "memory");
+        load_b_km<MODE, G>(slot, 0, bf, bl);
+      } else {
+#pragma unroll
+        for (int j = 0; j < kSubN; ++j) {
+          bf.h[j] = s.b[2 * j];
+          if constexpr (two_chunks<MODE>()) bf.l[j] = s.b[2 * j + 1];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) mma_row<MODE>(s.a[i], bf, acc[i]);
+      if (kt + u + kDeep < nk) load(kt + u + kDeep, s);
+    });
+  }
+  // Partials to LDS, [wave][block][register quad][lane], and the sums.
+  __syncthreads();
+  f32x4 *const part = reinterpret_cast<f32x4 *>(smem);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < kSubN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        part[((wave * 4 + 2 * i + j) * 4 + q) * 64 + lane] =
+            f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+  __syncthreads();
+  if (wave < 2) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int blk = by_col ? 2 * b + wave : 2 * wave + b;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        f32x4 v = part[(blk * 4 + q) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < G::kWaves; ++w) v += part[((w * 4 + blk) * 4 + q) * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[0][b][4 * q + e] = v[e];
+      }
+    }
+  }
+  __syncthreads();
+}
+
+// One product of a tile in geometry G: gemm_tile or, for kGeoT,
+// gemm_tile_split (whose epilogue adds the square's G term from memory).
+template <int MODE, class G, bool ACCG, bool BKM, bool UB = false>
+__device__ __forceinline__ void gemm_any(const Opnd &A, const Opnd &B, int64_t K, int64_t arow0, int64_t brow0,
+                                         float sel_s, char *smem, bool by_col, f32x16 (&acc)[G::kSubM][kSubN]) {
+  if constexpr (G::kSplitK) gemm_tile_split<MODE, BKM>(A, B, K, arow0, brow0, smem, by_col, acc);
+  else gemm_tile<MODE, G, ACCG, BKM, UB>(A, B, K, arow0, brow0, sel_s, smem, acc);
+}
+
 // ---------------------------------------------------------- scalars ---
 // Sum of a small FP64 partial array by wave 0; result broadcast.
 __device__ double sum_parts(const double *p, int n, double *bcast) {
@@ -987,9 +1148,10 @@ struct Stage1Scalars {
 };
 // Tiles of a symmetric r x r result (Gram, square, SYM) in a geometry: the
 // upper-triangle 256 x 256 blocks (kGeoL), each as two 128-column halves
-// (kGeoM), or the upper-triangle 128 x 128 tiles (kGeoS).
+// (kGeoM), or the upper-triangle 128 x 128 tiles (kGeoS), each as four
+// quadrants (kGeoT).
 __host__ __device__ inline int64_t square_tiles(const S8Class &k, int geo) {
-  return geo == kGeoS ? sym_tiles(k.tiles_s) : geo == kGeoL ? sym_tiles(k.tiles_m) : 2 * sym_tiles(k.tiles_m);
+  return geo == kGeoT ? 4 * sym_tiles(k.tiles_s) : geo == kGeoS ? sym_tiles(k.tiles_s) : geo == kGeoL ? sym_tiles(k.tiles_m) : 2 * sym_tiles(k.tiles_m);
 }
 
 __device__ Stage1Scalars stage1_scalars(const S8Mat &M, int sq_geo, double *bcast) {
@@ -1030,7 +1192,7 @@ constexpr bool epilogue_fits() {
   // per wave two staging blocks; the apply adds the tile's a and z vectors
   return (G::kWaves * 2 * kEpBlock + 2 * (G::kTileM > G::kTileN ? G::kTileM : G::kTileN)) * 4 <= G::kRingBytes;
 }
-static_assert(epilogue_fits<GeoM>() && epilogue_fits<GeoS>() && epilogue_fits<GeoL>(),
+static_assert(epilogue_fits<GeoM>() && epilogue_fits<GeoS>() && epilogue_fits<GeoL>() && epilogue_fits<GeoT>(),
               "epilogue staging and the row-sum column vectors must fit in the operand ring");
 
 __device__ __forceinline__ void ep_read8(const float *s, int row, int col, float (&w)[8]) {
@@ -1046,12 +1208,15 @@ __device__ __forceinline__ void ep_read8(const float *s, int row, int col, float
 // their symmetric result (square_tiles): 256 x 256 tiles are its
 // upper-triangle blocks (tn >= tm, row by row); 256 x 128 tiles the
 // halves of those blocks (tix = 2 * block index + half); 128 x 128 tiles
-// its upper-triangle 128 x 128 tiles.  A diagonal block or tile is
+// its upper-triangle 128 x 128 tiles; 64 x 64 tiles the quadrants of
+// those (tix = 4 * tile index + quadrant).  A diagonal block or tile is
 // computed whole; an off-diagonal one also writes its mirror.
 __host__ __device__ inline int64_t phase_tiles(const S8Class &k, int phase, int geo, int op = -1) {
-  if (phase == kApply)
-    return static_cast<int64_t>(geo == kGeoS ? k.tiles_s : k.tiles_m) *
-           ((op == kOpApplyQ ? k.rp : k.cp) / (geo == kGeoL ? 256 : 128));
+  if (phase == kApply) {
+    const int64_t n = op == kOpApplyQ ? k.rp : k.cp;
+    if (geo == kGeoT) return (k.rp / 64) * (n / 64);
+    return static_cast<int64_t>(geo == kGeoS ? k.tiles_s : k.tiles_m) * (n / (geo == kGeoL ? 256 : 128));
+  }
   return square_tiles(k, geo);
 }
 
@@ -1078,7 +1243,7 @@ s8_stage_kernel(StageArgs args) {
     // a column block of X and cycle through P's row blocks, so each X block
     // is fetched once (0.54 GB per cfg4 apply launch against 0.77 GB
     // row-major; the launch time is the same).
-    const int64_t nrow = Gm::kGeo == kGeoS ? K.tiles_s : K.tiles_m;  // row tiles
+    const int64_t nrow = Gm::kSplitK ? K.rp / 64 : Gm::kGeo == kGeoS ? K.tiles_s : K.tiles_m;  // row tiles
     tn = tix / nrow;
     tm = tix % nrow;
   } else if constexpr (Gm::kGeo == kGeoM) {
@@ -1090,11 +1255,15 @@ s8_stage_kernel(StageArgs args) {
     diag = tb == tm;
   } else {
     const int64_t nt = Gm::kGeo == kGeoL ? K.tiles_m : K.tiles_s;  // tiles per row and column
-    int64_t rem = tix;
+    int64_t rem = Gm::kSplitK ? tix >> 2 : tix;
     tm = 0;
     while (rem >= nt - tm) { rem -= nt - tm; ++tm; }
     tn = tm + rem;
     diag = tn == tm;
+    if constexpr (Gm::kSplitK) {
+      tm = 2 * tm + ((tix >> 1) & 1);
+      tn = 2 * tn + (tix & 1);
+    }
   }
   const S8Mat M{K, slot};
   const int stage = args.stage;
@@ -1135,6 +1304,9 @@ s8_stage_kernel(StageArgs args) {
   // where G is not: neither the rounding of a diagonal near 1 nor the
   // cancellation of a + b G + c G^2 there reaches P.
   const bool shift = kPair && stage != 1 && !K.gs;
+  // kGeoT: the wave's two blocks below each other instead of side by side,
+  // where the row sums run down the tile's rows (a transposed parameter).
+  const bool by_col = Gm::kSplitK && PHASE == kApply && M.flip();
   float scale = 1.f;
   float *sym_out = nullptr;  // SYM: the product's destination
   // Gram space (see the header): a segment's first Q sits in qa; Q' = P Q
@@ -1155,8 +1327,8 @@ s8_stage_kernel(StageArgs args) {
       }
     }
     if constexpr (kPair) scale *= pow2f(-kExpP);  // P G -> T, T P -> G
-    gemm_tile<MODE, Gm, false, false, MODE == kS8CompMix>(Opnd{A, K.rp}, Opnd{B, K.rp}, K.rp, tm * Gm::kTileM,
-                                                         tn * kTileN, 0.f, smem, acc);
+    gemm_any<MODE, Gm, false, false, MODE == kS8CompMix>(Opnd{A, K.rp}, Opnd{B, K.rp}, K.rp, tm * Gm::kTileM,
+                                                         tn * kTileN, 0.f, smem, by_col, acc);
   } else if constexpr (PHASE == kGram) {
     if (stage == 1) {
       const double f = M.cst()[kCstFro];
@@ -1166,7 +1338,7 @@ s8_stage_kernel(StageArgs args) {
     }
     // A Gram-space class takes its stage-3 Gram of X2 from x1.
     const Opnd X{K.gs && stage == 3 ? M.x1() : x_in, K.cp};
-    gemm_tile<MODE, Gm, false, false>(X, X, K.cp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, acc);
+    gemm_any<MODE, Gm, false, false>(X, X, K.cp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, by_col, acc);
   } else if constexpr (PHASE == kSquare) {
     const Opnd G{M.g(), K.rp};
     // (the square kernels run at the VGPR budget, where the compiler keeps
@@ -1174,13 +1346,13 @@ s8_stage_kernel(StageArgs args) {
     constexpr bool kUB = true;
     if (stage == 1) {
       if constexpr (kPair) scale = pow2f(-2 * kExpG);
-      gemm_tile<MODE, Gm, false, false, kUB>(G, G, K.rp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, acc);
+      gemm_any<MODE, Gm, false, false, kUB>(G, G, K.rp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, by_col, acc);
     } else {
       // acc = G G + (b/c) G; the epilogue forms P = c acc + a I.
       scale = kPair ? args.c * pow2f(kExpP - 2 * kExpG) : args.c;
-      gemm_tile<MODE, Gm, true, false, kUB>(G, G, K.rp, tm * Gm::kTileM, tn * kTileN,
+      gemm_any<MODE, Gm, true, false, kUB>(G, G, K.rp, tm * Gm::kTileM, tn * kTileN,
                                             kPair ? (shift ? args.bh_over_c : args.b_over_c) * pow2f(kExpG)
-                                                  : args.b_over_c, smem, acc);
+                                                  : args.b_over_c, smem, by_col, acc);
     }
   } else {
     // X-space: X' = P X (stage 1: X' = P1 V / (||V|| s)).  Gram space:
@@ -1201,7 +1373,7 @@ s8_stage_kernel(StageArgs args) {
     const float *A = mid ? M.qb() : fin ? M.qa() : M.p();
     const Opnd B = gq ? Opnd{q_in, K.rp} : Opnd{mid ? M.x0() : fin ? M.x1() : x_in, K.cp};
     // B = X (or Q) rows k (K-major), columns of the tile.
-    gemm_tile<MODE, Gm, false, true>(Opnd{A, K.rp}, B, K.rp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, acc);
+    gemm_any<MODE, Gm, false, true>(Opnd{A, K.rp}, B, K.rp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, by_col, acc);
   }
 
   // ------------------------------------------------------- epilogue ---
@@ -1219,7 +1391,9 @@ s8_stage_kernel(StageArgs args) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wm = wave / Gm::kWavesN, wn = wave % Gm::kWavesN;
   const int lr = lane & 31, lh = lane >> 5;
-  const int64_t R0 = tm * Gm::kTileM + wm * (32 * kSubM), C0 = tn * kTileN + wn * (32 * kSubN);
+  // The wave's blocks: kSubM x kSubN from (R0, C0); kGeoT two (waves 0, 1).
+  const int64_t R0 = tm * Gm::kTileM + (Gm::kSplitK ? (by_col ? 0 : 32 * wave) : wm * (32 * kSubM));
+  const int64_t C0 = tn * kTileN + (Gm::kSplitK ? (by_col ? 32 * wave : 0) : wn * (32 * kSubN));
   const bool last = stage == 5;
   float *dst_t, *dst_m;
   int64_t ld_t, ld_m;
@@ -1446,6 +1620,36 @@ s8_stage_kernel(StageArgs args) {
       }
     }
   };
+  // kGeoT's square: b G of the lane's 16 values of row gr, columns cb +
+  // col16(e), in the scale of P (the K loop has just read them).  In place
+  // of the one-hot MFMAs, whose code is longer than a launch this short can
+  // fetch: 14.5 -> 11 us per launch of one 512 x 512 matrix.
+  auto add_bg = [&](float (&w)[16], int64_t gr, int64_t cb) {
+    const SMX_GLOBAL char *gp = (const SMX_GLOBAL char *)M.g();
+    constexpr bool F16 = MODE == kS8F16;
+    const int64_t base = (gr & ~int64_t{15}) * ((F16 ? 2 : 4) * K.rp) + ((gr & 15) << 6) + (F16 ? 32 : 64) * cb + 16 * lh;
+    const float b = kPair ? (shift ? args.bh : args.b) * pow2f(kExpP - kExpG) : args.b;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const uint4 h = __builtin_bit_cast(uint4, *reinterpret_cast<const SMX_GLOBAL u32x4v *>(gp + base + (F16 ? 32 : 1024) * q));
+      const uint4 l = !is_split(MODE) ? make_uint4(0, 0, 0, 0)
+                          : __builtin_bit_cast(uint4, *reinterpret_cast<const SMX_GLOBAL u32x4v *>(gp + base + 1024 * q + 32));
+      const uint32_t hw[4] = {h.x, h.y, h.z, h.w}, lw[4] = {l.x, l.y, l.z, l.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float g0, g1;
+        if constexpr (kPair || F16) {
+          g0 = f16_bits_to_f32(hw[e] & 0xffff) + f16_bits_to_f32(lw[e] & 0xffff);
+          g1 = f16_bits_to_f32(hw[e] >> 16) + f16_bits_to_f32(lw[e] >> 16);
+        } else {
+          g0 = __uint_as_float(hw[e] << 16) + __uint_as_float(lw[e] << 16);
+          g1 = __uint_as_float(hw[e] & 0xffff0000u) + __uint_as_float(lw[e] & 0xffff0000u);
+        }
+        w[8 * q + 2 * e] = fmaf(b, g0, w[8 * q + 2 * e]);
+        w[8 * q + 2 * e + 1] = fmaf(b, g1, w[8 * q + 2 * e + 1]);
+      }
+    }
+  };
   // The block loop, specialised for the output form (one copy per form the
   // launch's mode can produce, so that each keeps only its own registers).
   auto epilogue = [&](auto fm_c) {
@@ -1457,17 +1661,22 @@ s8_stage_kernel(StageArgs args) {
     float rsd[3] = {0.f, 0.f, 0.f};
     // (expanded at compile time: a rolled block loop indexes acc at run
     // time, which moves every accumulator of the kernel to scratch memory)
-    static_for<kSubM * kSubN>([&](auto blk_c) {
+    static_for<Gm::kSplitK ? 2 : kSubM * kSubN>([&](auto blk_c) {
       constexpr int blk = decltype(blk_c)::value, i = blk / kSubN, j = blk % kSubN;
-      const int64_t gr = R0 + i * 32 + lr, cb = C0 + j * 32;
+      const int64_t rb = R0 + (Gm::kSplitK && by_col ? blk : i) * 32;
+      const int64_t gr = rb + lr, cb = C0 + (Gm::kSplitK && by_col ? 0 : j) * 32;
       float w[16];
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         w[e] = acc[i][j][e] * scale;
         // stage 1's FP32 G2: its squared entries feed the Schatten scale
         if constexpr (PHASE == kSquare && (FM == kFormF32 || FM == kFormAny)) sq_local = fmaf(w[e], w[e], sq_local);
-        if (do_m) U[col16(e) * kEpStride + lr] = w[e];
       }
+      if constexpr (PHASE == kSquare && Gm::kSplitK)
+        if (stage != 1) add_bg(w, gr, cb);
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (do_m) U[col16(e) * kEpStride + lr] = w[e];
       if (do_t) {
         if (eye)
 #pragma unroll
@@ -1507,8 +1716,10 @@ s8_stage_kernel(StageArgs args) {
         for (int q = 0; q < 4; ++q) {
           const int row = er + 8 * q;
           const int64_t gm = cb + row;
-          put_row(fm_c, U, row, gm, R0 + i * 32, dst_m, ld_m, tiled_m, rs[j][q], rs_on);
-          if (rs_on && (i + 1) % (kStripM / 32) == 0) emit(gm, (R0 + 32 * (i + 1) - kStripM) / kStripM, rs[j][q]);
+          float(&r)[3] = rs[Gm::kSplitK ? 0 : j][q];
+          put_row(fm_c, U, row, gm, rb, dst_m, ld_m, tiled_m, r, rs_on);
+          if (rs_on && (Gm::kSplitK ? blk == 1 : (i + 1) % (kStripM / 32) == 0))
+            emit(gm, (rb + 32 - kStripM) / kStripM, r);
         }
       }
       // Keep the scheduler from hoisting every accumulator read to the top
@@ -1518,12 +1729,14 @@ s8_stage_kernel(StageArgs args) {
   };
   // Only the forms this launch kind can produce are compiled (the host
   // checks every launch's forms against the same table, form_compiled).
+  const bool owns = !Gm::kSplitK || wave < 2;  // the wave holds blocks of the tile
   constexpr bool kPlanes = form_compiled(MODE, PHASE, kFormPlanes);
   constexpr bool kF16 = form_compiled(MODE, PHASE, kFormF16);
   constexpr bool kF32 = form_compiled(MODE, PHASE, kFormF32);
   if constexpr (PHASE == kSquare && kPlanes && kF32 && !kF16) {
     // one loop for both forms, as compact as a kernel of one form
-    epilogue(std::integral_constant<int, kFormAny>{});
+    if (owns) epilogue(std::integral_constant<int, kFormAny>{});
+  } else if (!owns) {
   } else if (kPlanes && form == kFormPlanes) {
     if constexpr (kPlanes) epilogue(std::integral_constant<int, kFormPlanes>{});
   } else if (kF16 && form == kFormF16) {
@@ -1772,8 +1985,11 @@ static double launch_flops(int mode, int phase, int stage, int geo, const S8Layo
                            const std::vector<Seg> &segs) {
   if (phase == kPoly1) return 0.0;
   const double prod = is_comp(mode) ? 3.0 : 1.0;
-  const int tm = geo == kGeoS ? 128 : 256, tn = geo == kGeoL ? 256 : 128, waves = geo == kGeoL ? 8 : 4;
-  const int sub_m = tm / 64;
+  const int tm = geo == kGeoT ? 64 : geo == kGeoS ? 128 : 256, tn = geo == kGeoT ? 64 : geo == kGeoL ? 256 : 128;
+  // waves that issue the one-hot MFMAs of a tile, 32 sub_m rows each (kGeoT,
+  // which adds that term from memory, counts as many)
+  const int waves = geo == kGeoT ? 1 : geo == kGeoL ? 8 : 4;
+  const int sub_m = geo == kGeoT ? 2 : tm / 64;
   // (kS8Pair counts one product per element pair, as the FP32 MFMAs whose
   // place it takes issue; it is carried out as three FP16 ones.)
   const double onehot = is_comp(mode) ? 6.0 * sub_m : mode == kS8HiOnly ? 4.0 * sub_m
@@ -1799,43 +2015,49 @@ static int64_t device_cus() {
   return cus[dev];
 }
 
-// The tile geometry of one launch over `segs`.  256 x 256 tiles when the
-// launch has at least 1.5 of them per CU: those blocks move a third fewer
-// operand bytes per MFMA (cfg5 S8 7% faster).  With fewer, each CU holds
-// one or two blocks of the launch and nothing of it to overlap a block's
-// prologue and epilogue with (cfg4 Gram, square and SYM launches 15-60%
-// slower; with tiled operands the cfg4 applies, 0.6-2.2 tiles per CU, are
-// 1-2% faster as 256 x 128 tiles, two blocks per CU).  Otherwise 128 x 128
-// tiles when they take fewer rounds of the CUs' block slots (three per CU,
-// a round counted 0.9 of one of two 256 x 128 blocks per CU), else
-// 256 x 128 (the cfg4 applies take 128 x 128 tiles: S8 runs 2% shorter
-// than with 256 x 128).
+// The tile geometry of one launch over `segs`.  64 x 64 tiles with K split
+// over the block's waves (kGeoT) up to three per CU: such a launch takes
+// the time of one tile's chain, a quarter as long there.  (One 512 x 512
+// matrix 261 -> 183 us, two of 768 x 3072 in an MLP step 1446 -> 1310 us,
+// four of 640 x 1280 in a direction 635 -> 520; with up to six tiles per
+// CU, half of 36 768 x 768 matrices 1235 -> 1620 us.)  It adds in another
+// order than the other geometries, so not where those bits are kept
+// (S8Layout::keep_bits), nor on FP32 MFMAs.  256 x 256 tiles when
+// the launch has at least 1.5 of them per CU: those blocks move a third
+// fewer operand bytes per MFMA (cfg5 S8 7% faster).  With fewer, each CU
+// holds one or two blocks of the launch and nothing of it to overlap a
+// block's prologue and epilogue with (cfg4 Gram, square and SYM launches
+// 15-60% slower; with tiled operands the cfg4 applies, 0.6-2.2 tiles per
+// CU, are 1-2% faster as 256 x 128 tiles, two blocks per CU).  Otherwise
+// 128 x 128 tiles when they take fewer rounds of the CUs' block slots
+// (three per CU, a round counted 0.9 of one of two 256 x 128 blocks per
+// CU), else 256 x 128 (the cfg4 applies take 128 x 128 tiles: S8 runs 2%
+// shorter than with 256 x 128).
 static int pick_geo(const S8Layout &Lay, int phase, const std::vector<Seg> &segs) {
   if (g_tile_policy == 1) return kGeoL;
   const int64_t cus = device_cus();
-  int64_t tiles[3] = {0, 0, 0};
+  int64_t tiles[4] = {0, 0, 0, 0};
   for (const Seg &sg : segs) {
     const S8Class &k = Lay.cls[sg.cls];
     const int64_t cnt = sg.hi - sg.lo;
-    for (int g = 0; g < 3; ++g) tiles[g] += cnt * phase_tiles(k, phase, g, sg.op);
+    for (int g = 0; g < 4; ++g) tiles[g] += cnt * phase_tiles(k, phase, g, sg.op);
   }
-  {
-    static int thr_apply = getenv("SMX_XL_APPLY") ? atoi(getenv("SMX_XL_APPLY")) : 15;
-    static int thr_other = getenv("SMX_XL_OTHER") ? atoi(getenv("SMX_XL_OTHER")) : 15;
-    const int thr = phase == kApply ? thr_apply : thr_other;
-    if (g_tile_policy == 0 && 10 * tiles[kGeoL] >= thr * cus) return kGeoL;
-  }
-  {
-    const double r_m = static_cast<double>(ceil_div(tiles[kGeoM], 2 * cus));
-    const double r_s = static_cast<double>(ceil_div(tiles[kGeoS], 3 * cus));
-    if (0.9 * r_s < r_m) return kGeoS;
-  }
-  return kGeoM;
+  if (g_tile_policy == 0 && !Lay.keep_bits && Lay.mode != SMX_S8_FP32 && tiles[kGeoT] <= 3 * cus)
+    return kGeoT;
+  if (g_tile_policy == 0 && 2 * tiles[kGeoL] >= 3 * cus) return kGeoL;
+  const double r_m = static_cast<double>(ceil_div(tiles[kGeoM], 2 * cus));
+  const double r_s = static_cast<double>(ceil_div(tiles[kGeoS], 3 * cus));
+  return 0.9 * r_s < r_m ? kGeoS : kGeoM;
 }
 
 // One phase launch of a stage kernel in geometry `geo`.
 template <int MODE, int PHASE>
 static void launch_stage(int geo, int32_t blocks, const StageArgs &a, hipStream_t st) {
+  if (geo == kGeoT) {
+    if constexpr (MODE != SMX_S8_FP32)
+      hipLaunchKernelGGL((s8_stage_kernel<MODE, PHASE, 64, 64>), dim3(blocks), dim3(GeoT::kThreads), 0, st, a);
+    return;
+  }
   if (geo == kGeoS) {
     hipLaunchKernelGGL((s8_stage_kernel<MODE, PHASE, 128, 128>), dim3(blocks), dim3(GeoS::kThreads), 0, st, a);
     return;
@@ -1875,6 +2097,7 @@ static int launch_phase(const S8Layout &Lay, const SlotSet &set, int stage, int 
     a.c = static_cast<float>(co[2]);
     a.b_over_c = static_cast<float>(co[1] / co[2]);
     a.ah = static_cast<float>(co[0] + co[1] + co[2]);
+    a.bh = static_cast<float>(co[1] + 2.0 * co[2]);
     a.bh_over_c = static_cast<float>((co[1] + 2.0 * co[2]) / co[2]);
     if (static_cast<int>(segs.size()) > kMaxSeg) return fail(SMX_EINVAL, "s8: too many launch segments");
     if (PHASE != kPoly1)
@@ -2170,7 +2393,6 @@ bool plan_s8(const int64_t *r, const int64_t *c, const bool *flips, int32_t n, i
     C.u = reinterpret_cast<float *>(take(static_cast<size_t>(C.count) * C.cp * sizeof(float)));
     C.fro = reinterpret_cast<double *>(take(static_cast<size_t>(C.count) * C.parts * sizeof(double)));
     C.mb = reinterpret_cast<double *>(take(static_cast<size_t>(C.count) * C.parts * sizeof(double)));
-    C.sch = reinterpret_cast<double *>(take(static_cast<size_t>(C.count) * sym_tiles(C.tiles_s) * sizeof(double)));
     C.cst = reinterpret_cast<double *>(take(static_cast<size_t>(C.count) * kCst * sizeof(double)));
     C.colv = reinterpret_cast<const float **>(take(static_cast<size_t>(C.count) * 2 * sizeof(float *)));
     C.mrp = reinterpret_cast<float *>(take(static_cast<size_t>(C.count) * 3 * (C.rp * C.cp / kStripT) * sizeof(float)));
