@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import struct
 import threading
 from ctypes import c_double, c_float, c_int, c_int32, c_int64, c_size_t, c_void_p
 from pathlib import Path
@@ -60,6 +61,26 @@ class MatrixDesc(ctypes.Structure):
                 ("inv_row", c_void_p), ("inv_col", c_void_p), ("z", c_void_p), ("kappa", c_void_p),
                 ("rows", c_int64), ("cols", c_int64), ("lr", c_double), ("momentum_beta", c_double),
                 ("grad_dtype", c_int32), ("param_dtype", c_int32)]
+
+
+# The descriptors' bytes, field by field in order (native alignment; the
+# layouts above): one pack_into fills a descriptor of a table at a fifth of
+# the cost of a ctypes constructor with keywords.
+STATS_PACK = struct.Struct("3Q3q2i")
+FINISH_PACK = struct.Struct("9Q2q4i")
+ADAMW_PACK = struct.Struct("4Q2q2f2i")
+MATRIX_PACK = struct.Struct("7Q2q2d2i")
+assert [STATS_PACK.size, FINISH_PACK.size, ADAMW_PACK.size, MATRIX_PACK.size] == \
+    [ctypes.sizeof(d) for d in (StatsDesc, FinishDesc, AdamwDesc, MatrixDesc)]
+
+
+def table(desc, packed: bytearray):
+    """A descriptor table (a ctypes array of `desc`) over its packed bytes."""
+    return (desc * (len(packed) // ctypes.sizeof(desc))).from_buffer(packed)
+
+
+def _table_of(desc, descs):
+    return descs if isinstance(descs, ctypes.Array) else (desc * len(descs))(*descs)
 
 
 # name -> (restype, argtypes); every symbol include/sandmuon_amd.h declares.
@@ -238,15 +259,18 @@ def stats_slot_rows(rows: int, n_slots: int) -> int:
 def stats_accumulate_batch(entries, stream: int) -> None:
     """One launch over several hook inputs: entries of (rows2d, slots_sq,
     slots_first) whose slot rows are pairwise distinct."""
-    descs = (StatsDesc * len(entries))()
-    for d, (rows2d, sq, fs) in zip(descs, entries):
-        d.x, d.slots_sq, d.slots_first = rows2d.data_ptr(), sq.data_ptr(), ptr(fs)
-        d.rows, d.cols, d.row_stride = rows2d.shape[0], rows2d.shape[1], rows2d.stride(0)
-        d.dtype, d.n_slots = dtype_code(rows2d.dtype), sq.shape[0]
-    rc = lib().smx_stats_accumulate_batch(descs, len(entries), stream)
+    size = STATS_PACK.size
+    packed = bytearray(size * len(entries))
+    for k, (rows2d, sq, fs) in enumerate(entries):
+        rows, cols = rows2d.shape
+        STATS_PACK.pack_into(packed, k * size, rows2d.data_ptr(), sq.data_ptr(), 0 if fs is None else fs.data_ptr(),
+                             rows, cols, rows2d.stride(0), dtype_code(rows2d.dtype), sq.shape[0])
+    rc = lib().smx_stats_accumulate_batch(table(StatsDesc, packed), len(entries), stream)
     _check(rc, "smx_stats_accumulate_batch")
-    for rows2d, _, _ in entries:
-        _record_use(rows2d, stream)
+    if entries:
+        s = torch_stream(stream, entries[0][0].device)  # (a launch's inputs are on one device)
+        for rows2d, _, _ in entries:
+            rows2d.record_stream(s)
 
 
 def stats_cast(rows2d: torch.Tensor, slots_sq: torch.Tensor, slots_first: Optional[torch.Tensor],
@@ -354,9 +378,9 @@ class DescriptorStage:
     def take(self, nbytes: int):
         if nbytes > self.size:
             self._grow(nbytes)
-        free = [i for i, sl in enumerate(self.slots) if sl[1] is None or sl[1].query()]
-        slot = self.slots.pop(free[0] if free else 0)
-        if not free:
+        free = next((i for i, sl in enumerate(self.slots) if sl[1] is None or sl[1].query()), None)
+        slot = self.slots.pop(free or 0)
+        if free is None:
             slot[1].synchronize()
         self.slots.append(slot)  # most recent use last
         return slot
@@ -373,7 +397,7 @@ def stats_finish(descs: Sequence[FinishDesc], beta: float, device: torch.device,
     descriptors, or one of each for the whole table through `stage`."""
     if not descs:
         return
-    arr = (FinishDesc * len(descs))(*descs)
+    arr = _table_of(FinishDesc, descs)
     if stage is None or len(descs) <= FINISH_BATCH or torch.cuda.is_current_stream_capturing():
         _check(lib().smx_stats_finish(arr, len(descs), beta, stream_of(device)), "smx_stats_finish")
         return
@@ -390,7 +414,7 @@ def adamw(descs: Sequence[AdamwDesc], total: int, lr: float, beta1: float, beta2
     for the whole table through `stage`."""
     if not descs:
         return
-    arr = (AdamwDesc * len(descs))(*descs)
+    arr = _table_of(AdamwDesc, descs)
     if stage is None or len(descs) <= ADAMW_BATCH or torch.cuda.is_current_stream_capturing():
         _check(lib().smx_adamw(arr, len(descs), total, lr, beta1, beta2, eps, weight_decay, stream_of(device)),
                "smx_adamw")
@@ -403,6 +427,11 @@ def adamw(descs: Sequence[AdamwDesc], total: int, lr: float, beta1: float, beta2
 
 
 def matrix_step_workspace_bytes(shapes: Sequence[tuple], mode: int) -> int:
+    return _matrix_step_workspace_bytes(tuple(shapes), mode)
+
+
+@functools.lru_cache(maxsize=64)
+def _matrix_step_workspace_bytes(shapes: tuple, mode: int) -> int:
     n = len(shapes)
     rows = (c_int64 * n)(*[s[0] for s in shapes])
     cols = (c_int64 * n)(*[s[1] for s in shapes])
@@ -412,7 +441,7 @@ def matrix_step_workspace_bytes(shapes: Sequence[tuple], mode: int) -> int:
 def matrix_step(descs: Sequence[MatrixDesc], mode: int, workspace: torch.Tensor) -> None:
     if not descs:
         return
-    arr = (MatrixDesc * len(descs))(*descs)
+    arr = _table_of(MatrixDesc, descs)
     _check(lib().smx_matrix_step(arr, len(descs), mode, workspace.data_ptr(), workspace.numel(),
                                  stream_of(workspace.device)), "smx_matrix_step")
 

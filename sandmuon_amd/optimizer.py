@@ -189,6 +189,12 @@ def _require_f32(t: torch.Tensor, n: int, device, what: str) -> torch.Tensor:
     return t
 
 
+def _is_f32(t, n: int, device) -> bool:
+    """Whether _require_f32 takes t."""
+    return (isinstance(t, torch.Tensor) and t.dtype is torch.float32 and t.numel() == n and t.is_contiguous() and
+            t.device == device)
+
+
 def _like(t: torch.Tensor, parameter: torch.Tensor, dtype: Optional[torch.dtype] = None) -> torch.Tensor:
     """t (same shape as `parameter`) with the parameter's strides: as it is
     when they already match, else copied into the parameter's layout."""
@@ -573,31 +579,31 @@ class DiagonalWeightedPE(Optimizer):
             raise RuntimeError(f"Missing or mismatched cotangent statistics: {self.parameter_names[id(parameter)]}; "
                                f"expected {expected_count}, got {state.get('b_count', 0)}")
 
-    def _finish_desc(self, parameter, side: str, count: int, out: Dict[str, torch.Tensor]) -> _native.FinishDesc:
+    def _pack_finish(self, packed: bytearray, k: int, parameter, side: str, count: int, inv: int, z: int = 0,
+                     kappa: int = 0) -> None:
+        """Packs finish descriptor k: the vector's sums, slot rows and EMA,
+        and the device pointers its factors go to."""
         state = self.state[parameter]
-        total = state[f"{side}_sum"]
+        device = parameter.device
         n = parameter.shape[1] if side == "a" else parameter.shape[0]
         rank1 = side == "a" and self.rank_one_a
+        sum_key, ema_key = ("a_sum", "a_ema") if side == "a" else ("b_sum", "b_ema")
+        total = state[sum_key]
         sq, fs = self._slot_pair(parameter, side, n, total.device, rank1)
-        ema_key = f"{side}_ema"
         first = ema_key not in state
         if first:
             state[ema_key] = torch.empty(n, dtype=torch.float32, device=total.device)
             if rank1:
                 state["a_mean_ema"] = torch.empty(n, dtype=torch.float32, device=total.device)
-        name = self.parameter_names[id(parameter)]
-        keys = [f"{side}_sum", ema_key] + (["a_first_sum", "a_mean_ema"] if rank1 else [])
-        for key in keys:
-            _require_f32(state[key], n, parameter.device, f"{key} of {name}")
+        for key in (sum_key, ema_key) + (("a_first_sum", "a_mean_ema") if rank1 else ()):
+            if not _is_f32(state[key], n, device):
+                _require_f32(state[key], n, device, f"{key} of {self.parameter_names[id(parameter)]}")
         kind = _KIND_B if side == "b" else (_KIND_RANK1_A if rank1 else _KIND_DIAG_A)
-        d = _native.FinishDesc(sum_sq=total.data_ptr(), slots_sq=sq.data_ptr(), ema=state[ema_key].data_ptr(),
-                               inv=out["inv"].data_ptr(), n=n, count=int(count), n_slots=self._take_slot_rows(sq),
-                               kind=kind, first=int(first))
-        if rank1:
-            d.sum_first, d.slots_first = state["a_first_sum"].data_ptr(), fs.data_ptr()
-            d.mean_ema = state["a_mean_ema"].data_ptr()
-            d.z, d.kappa = out["z"].data_ptr(), out["kappa"].data_ptr()
-        return d
+        _native.FINISH_PACK.pack_into(
+            packed, k * _native.FINISH_PACK.size, total.data_ptr(), sq.data_ptr(),
+            state["a_first_sum"].data_ptr() if rank1 else 0, fs.data_ptr() if rank1 else 0,
+            state[ema_key].data_ptr(), state["a_mean_ema"].data_ptr() if rank1 else 0, inv, z, kappa,
+            n, int(count), self._take_slot_rows(sq), kind, int(first), 0)
 
     def _descriptor_stage(self, device) -> "_native.DescriptorStage":
         if self._stage is None or self._stage.device != device:
@@ -647,74 +653,68 @@ class DiagonalWeightedPE(Optimizer):
 
     def _matrix_update(self, items, a_counts) -> None:
         device = items[0][0].device
-        sources = []
-        seen = set()
-        for parameter, source, _ in items:
-            if id(source) not in seen:
-                seen.add(id(source))
-                sources.append(source)
-        # One flat buffer for every factor of this step; each vector starts on
-        # a 16-byte boundary (the kernels' vector loads).
-        sizes, lengths = [], []
+        sources = list({id(source): source for _, source, _ in items}.values())
+        # One flat buffer for every factor of this step (inv, and z and kappa
+        # of a rank-one source); each vector starts on a 16-byte boundary (the
+        # kernels' vector loads).  Its pointers: (inv, z, kappa) per vector.
+        at, a_at, b_at = 0, [], []
         for s in sources:
-            d = self.state[s]["a_sum"].numel()
-            lengths += [d, d, 1] if self.rank_one_a else [d]
+            n = -(-s.shape[1] // 4) * 4
+            a_at.append((at, at + n, at + 2 * n))
+            at += 2 * n + 4 if self.rank_one_a else n
         for parameter, _, _ in items:
-            lengths.append(parameter.shape[0])
-        sizes = [-(-n // 4) * 4 for n in lengths]
-        flat = torch.empty(sum(sizes), dtype=torch.float32, device=device)
-        views = iter(v[:n] for v, n in zip(torch.split(flat, sizes), lengths))
-        a_out, b_out, descs = {}, {}, []
-        for s in sources:
-            out = {"inv": next(views)}
-            if self.rank_one_a:
-                out["z"], out["kappa"] = next(views), next(views)
+            b_at.append(at)
+            at += -(-parameter.shape[0] // 4) * 4
+        flat = torch.empty(at, dtype=torch.float32, device=device)
+        base = flat.data_ptr()
+        packed = bytearray(_native.FINISH_PACK.size * (len(sources) + len(items)))
+        a_out, k = {}, 0
+        for s, (inv, z, kappa) in zip(sources, a_at):
+            out = (base + 4 * inv, base + 4 * z, base + 4 * kappa) if self.rank_one_a else (base + 4 * inv, 0, 0)
             a_out[id(s)] = out
-            descs.append(self._finish_desc(s, "a", a_counts[id(s)], out))
-        for parameter, source, _ in items:
-            out = {"inv": next(views)}
-            b_out[id(parameter)] = out
-            descs.append(self._finish_desc(parameter, "b", a_counts[id(source)], out))
-        _native.stats_finish(descs, self.statistic_beta, device, self._descriptor_stage(device))
+            self._pack_finish(packed, k, s, "a", a_counts[id(s)], *out)
+            k += 1
+        for (parameter, source, _), inv in zip(items, b_at):
+            self._pack_finish(packed, k, parameter, "b", a_counts[id(source)], base + 4 * inv)
+            k += 1
+        _native.stats_finish(_native.table(_native.FinishDesc, packed), self.statistic_beta, device,
+                             self._descriptor_stage(device))
         for s in sources:
             self.state[s]["a_count"] = 0
-        for parameter, _, _ in items:
-            self.state[parameter]["b_count"] = 0
 
         # Converted or re-laid-out gradients are temporaries: they must stay
         # alive until the launch that reads them is enqueued (the allocator
         # would hand a freed one to the next temporary of this loop).
-        mdescs, shapes, keep = [], [], []
-        for parameter, source, group in items:
+        size = _native.MATRIX_PACK.size
+        packed, shapes, keep = bytearray(size * len(items)), [], []
+        for k, (parameter, source, group) in enumerate(items):
             state = self.state[parameter]
-            _check_layout(parameter, self.parameter_names[id(parameter)], True)
-            if "momentum_buffer" not in state:
-                state["momentum_buffer"] = torch.zeros_like(parameter, dtype=torch.float32)
-            elif not state["momentum_buffer"].is_contiguous() or state["momentum_buffer"].dtype != torch.float32:
-                state["momentum_buffer"] = state["momentum_buffer"].to(torch.float32).contiguous()
+            state["b_count"] = 0
+            if not parameter.is_contiguous():
+                _check_layout(parameter, self.parameter_names[id(parameter)], True)
+            momentum = state.get("momentum_buffer")
+            if momentum is None:
+                momentum = state["momentum_buffer"] = torch.zeros_like(parameter, dtype=torch.float32)
+            elif not momentum.is_contiguous() or momentum.dtype != torch.float32:
+                momentum = state["momentum_buffer"] = momentum.to(torch.float32).contiguous()
             grad = parameter.grad
             if grad.dtype not in _PARAM_DTYPES:
                 grad = grad.float()
             grad = grad.contiguous()
             keep.append(grad)
-            a = a_out[id(source)]
-            md = _native.MatrixDesc(param=parameter.data_ptr(), grad=grad.data_ptr(),
-                                    momentum=state["momentum_buffer"].data_ptr(),
-                                    inv_row=b_out[id(parameter)]["inv"].data_ptr(), inv_col=a["inv"].data_ptr(),
-                                    rows=parameter.shape[0], cols=parameter.shape[1], lr=float(group["lr"]),
-                                    momentum_beta=self._momentum(group),
-                                    grad_dtype=_native.dtype_code(grad.dtype),
-                                    param_dtype=_native.dtype_code(parameter.dtype))
-            if self.rank_one_a:
-                md.z, md.kappa = a["z"].data_ptr(), a["kappa"].data_ptr()
-            mdescs.append(md)
-            shapes.append(tuple(parameter.shape))
+            inv, z, kappa = a_out[id(source)]
+            rows, cols = parameter.shape
+            _native.MATRIX_PACK.pack_into(
+                packed, k * size, parameter.data_ptr(), grad.data_ptr(), momentum.data_ptr(), base + 4 * b_at[k], inv,
+                z, kappa, rows, cols, float(group["lr"]), self._momentum(group), _native.dtype_code(grad.dtype),
+                _native.dtype_code(parameter.dtype))
+            shapes.append((rows, cols))
         mode = _native.S8_MODES[self.s8_mode]
         need = _native.matrix_step_workspace_bytes(shapes, mode)
         if self._workspace is None or self._workspace.numel() < need or self._workspace.device != device:
             self._workspace = None
             self._workspace = torch.empty(need, dtype=torch.uint8, device=device)
-        _native.matrix_step(mdescs, mode, self._workspace)
+        _native.matrix_step(_native.table(_native.MatrixDesc, packed), mode, self._workspace)
         del keep
 
     def _auxiliary_update(self, items) -> None:
@@ -724,34 +724,41 @@ class DiagonalWeightedPE(Optimizer):
         for entries in by_group.values():
             group = entries[0][1]
             b1, b2 = group["adamw_betas"]
-            descs, offset, keep = [], 0, []
+            size = _native.ADAMW_PACK.size
+            packed, offset, keep, bias = bytearray(size * len(entries)), 0, [], {}
             device = entries[0][0].device
-            for parameter, _ in entries:
+            for k, (parameter, _) in enumerate(entries):
                 state = self.state[parameter]
                 # The kernel walks parameter, gradient and state flat, so all
                 # of them take the parameter's layout.
-                _check_layout(parameter, "an auxiliary parameter", False)
+                flat = parameter.is_contiguous()
+                if not flat:
+                    _check_layout(parameter, "an auxiliary parameter", False)
                 if "exp_avg" not in state:
                     state["exp_avg"] = torch.zeros_like(parameter, dtype=torch.float32)
                     state["exp_avg_sq"] = torch.zeros_like(parameter, dtype=torch.float32)
                     state["step"] = 0
                 for key in ("exp_avg", "exp_avg_sq"):
-                    state[key] = _like(state[key], parameter, torch.float32)
-                state["step"] = int(state["step"]) + 1
+                    t = state[key]
+                    if not (flat and t.is_contiguous() and t.dtype is torch.float32 and t.shape == parameter.shape):
+                        state[key] = _like(t, parameter, torch.float32)
+                step = state["step"] = int(state["step"]) + 1
+                if step not in bias:
+                    bias[step] = 1 - b1 ** step, 1 - b2 ** step
                 grad = parameter.grad
                 if grad.dtype not in _PARAM_DTYPES:
                     grad = grad.float()
-                grad = _like(grad, parameter)
+                if not (flat and grad.is_contiguous()):
+                    grad = _like(grad, parameter)
                 keep.append(grad)  # alive until the launch below is enqueued
                 n = parameter.numel()
-                descs.append(_native.AdamwDesc(
-                    param=parameter.data_ptr(), grad=grad.data_ptr(), exp_avg=state["exp_avg"].data_ptr(),
-                    exp_avg_sq=state["exp_avg_sq"].data_ptr(), n=n, offset=offset,
-                    bias1=1 - b1 ** state["step"], bias2=1 - b2 ** state["step"],
-                    grad_dtype=_native.dtype_code(grad.dtype), param_dtype=_native.dtype_code(parameter.dtype)))
+                _native.ADAMW_PACK.pack_into(
+                    packed, k * size, parameter.data_ptr(), grad.data_ptr(), state["exp_avg"].data_ptr(),
+                    state["exp_avg_sq"].data_ptr(), n, offset, *bias[step], _native.dtype_code(grad.dtype),
+                    _native.dtype_code(parameter.dtype))
                 offset += n
             lr = group["lr"] * group["adamw_lr_ratio"]
-            _native.adamw(descs, offset, lr, b1, b2, group["adamw_eps"], group["weight_decay"], device,
+            _native.adamw(_native.table(_native.AdamwDesc, packed), offset, lr, b1, b2, group["adamw_eps"], group["weight_decay"], device,
                           self._descriptor_stage(device))
             del keep
 
