@@ -385,7 +385,8 @@ int smx_s8(const float *x, float *out, int64_t batch, int64_t rows,
  * duration (ms), phase (0 Gram, 1 square, 2 apply, 3 stage-1 polynomial,
  * 4 a whole S8 run, first launch to last, 5 the symmetric r x r products
  * of Gram-space classes, which are iterated on r x r matrices when their
- * padded columns exceed their padded rows)
+ * padded columns exceed their padded rows, 6 matrices small enough to run
+ * whole in one block each)
  * and the MFMA FLOPs the launch (or run) issues (tiles computed x
  * 2*256*256*K, x3 in SMX_S8_COMP_BF16 mode, plus the square phase's
  * one-hot MFMAs; SMX_S8_FP32 counts one product per element pair, a third

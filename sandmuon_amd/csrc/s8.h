@@ -253,6 +253,12 @@ struct S8Plan {
 bool plan_s8(const int64_t *r, const int64_t *c, const bool *flips, int32_t n, int mode,
              char *base, S8Plan &plan, int32_t *cls_of, int32_t *slot_of);
 
+// Whether a class's matrices run whole in one block's LDS (s8_small.hip).
+bool s8_small(const S8Class &k);
+// Runs every small class of the layout, a launch per number of row tiles;
+// adds its MFMA FLOPs.
+int run_s8_small(const S8Layout &layout, hipStream_t st, double &flops);
+
 // Sets `pairs`, and the classes' iteration form under it.  To be called once
 // a layout's keep_bits is set, before its results are located
 // (S8Mat::result).

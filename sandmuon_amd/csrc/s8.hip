@@ -112,7 +112,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-enum Phase { kGram = 0, kSquare = 1, kApply = 2, kPoly1 = 3, kSpan = 4, kSym = 5 };  // kSpan: timing record of a whole S8 run
+enum Phase { kGram = 0, kSquare = 1, kApply = 2, kPoly1 = 3, kSpan = 4, kSym = 5, kSmall = 6 };  // kSpan: timing record of a whole S8 run
 // SYM products of a Gram-space class (per segment of a SYM launch).
 // The product of a segment of a SYM or APPLY launch: PG / TP of a
 // Gram-space class (SYM); X' = P X of an X-space class, Q' = P Q and the
@@ -2227,14 +2227,14 @@ static int fork_stream(ForkStream *&out) {
 // one record for the run, on the caller's stream.
 constexpr int kSplitCount = 2 * kChains;
 
-// The FP16 pairs of every X0 of a kS8Pair run, before its chains fork.
-static int run_s8_pair0(const S8Layout &Lay, hipStream_t st) {
+// The FP16 pairs of the X0 of a kS8Pair run's chains, before they fork.
+static int run_s8_pair0(const S8Layout &Lay, bool small, hipStream_t st) {
   StageArgs a{};
   a.L = Lay;
   int32_t off = 0;
   for (int i = 0; i < Lay.n_classes; ++i) {
     const S8Class &k = Lay.cls[i];
-    if (!k.count) continue;
+    if (!k.count || (small && s8_small(k))) continue;
     a.seg_off[a.n_seg] = off;
     a.seg_cls[a.n_seg] = i;
     a.seg_cnt[a.n_seg++] = k.count;
@@ -2250,14 +2250,17 @@ int run_s8_stages(const S8Layout &layout, hipStream_t st) {
   int slot = -1;
   int rc = timing_begin(st, slot, true);
   S8Layout Lay = layout;
+  // Small classes run whole in one block each, except where bits are kept, or
+  // a tile geometry or a compensation mask is forced (test aids).
+  const bool small = g_tile_policy == 0 && g_comp_mask == 0x1f && !Lay.keep_bits;
   if (Lay.pairs) {
     Lay.mode = kS8Pair;
-    if (!rc) rc = run_s8_pair0(Lay, st);
+    if (!rc) rc = run_s8_pair0(Lay, small, st);
   }
   if (rc) return rc;
   std::vector<int> order;
   for (int i = 0; i < Lay.n_classes; ++i)
-    if (Lay.cls[i].count) order.push_back(i);
+    if (Lay.cls[i].count && !(small && s8_small(Lay.cls[i]))) order.push_back(i);
   auto work = [&](int i, int n) {
     const S8Class &k = Lay.cls[i];
     return static_cast<double>(n) * k.rp * k.rp * k.cp;
@@ -2286,12 +2289,24 @@ int run_s8_stages(const S8Layout &layout, hipStream_t st) {
       load[t] += work(i, c);
     }
   }
-  int chains = 0;  // chains with work (the first always has some)
+  int chains = 0;  // chains with work
   for (int t = 0; t < kChains; ++t)
     if (!set[t].empty()) chains = t + 1;
   double flops = 0.0;
+  auto run_small = [&]() {
+    bool any = false;
+    for (int i = 0; i < Lay.n_classes; ++i) any = any || (Lay.cls[i].count && s8_small(Lay.cls[i]));
+    if (!small || !any) return static_cast<int>(SMX_OK);
+    int rec = -1;
+    double f = 0.0;
+    int e = timing_begin(st, rec, false);
+    if (!e) e = run_s8_small(layout, st, f);
+    flops += f;
+    return e ? e : timing_end(rec, st, kSmall, f);
+  };
   if (chains <= 1) {
-    for (int stage = 1; stage <= 5 && !rc; ++stage) rc = run_s8_set_stage(Lay, set[0], stage, st, flops);
+    for (int stage = 1; stage <= 5 && !rc && chains; ++stage) rc = run_s8_set_stage(Lay, set[0], stage, st, flops);
+    if (!rc) rc = run_small();
   } else {
     // Only enqueues happen under the lock.
     std::lock_guard<std::mutex> lock(g_fork_lock);
@@ -2306,6 +2321,7 @@ int run_s8_stages(const S8Layout &layout, hipStream_t st) {
     for (int stage = 1; stage <= 5 && !rc; ++stage)
       for (int t = chains - 1; t >= 0 && !rc; --t)
         if (!set[t].empty()) rc = run_s8_set_stage(Lay, set[t], stage, t ? f->aux[t - 1] : st, flops);
+    if (!rc) rc = run_small();  // beside the second chain
     // Join even after a failed launch, so the caller's stream never runs
     // ahead of work already on the other streams.
     for (int t = 1; f && t < chains; ++t)
@@ -2328,7 +2344,7 @@ int run_s8_stages(const S8Layout &layout, hipStream_t st) {
 void s8_choose_pairs(S8Layout &L) {
   L.pairs = L.mode == SMX_S8_FP32 && !L.keep_bits;
   for (int i = 0; i < L.n_classes; ++i)
-    if (L.cls[i].r <= 32 && L.cls[i].gs) L.pairs = 0;
+    if (L.cls[i].r <= 32 && L.cls[i].gs && !s8_small(L.cls[i])) L.pairs = 0;
   for (int i = 0; i < L.n_classes && L.pairs; ++i)
     if (L.cls[i].r <= 160) L.cls[i].gs = 0;
 }
