@@ -65,6 +65,32 @@ __device__ __forceinline__ float gelu_erf(float x) {
   return __fmul_rn(__fmul_rn(x, 0.5f), __fadd_rn(1.0f, e));
 }
 
+// The bf16 GELU as a table.  A bf16 input has 2^16 values: those of magnitude
+// 2^-9 up to 16 are looked up (13 binades of 128 values and a sign: 6.5 KB
+// of LDS, filled by the block with gelu_erf itself); below, GELU(x) rounds to
+// x / 2 (erf(x / sqrt 2) < 2^-9 moves x / 2 by less than half a last place),
+// which is one off the exponent of a normal value; the rest (magnitudes of
+// 16 and more, infinities, NaN, zero and the smallest normals) go through
+// gelu_erf.  The erf is some 45 vector instructions per element, which bound
+// the kernel: [16384, 3072] took 70 us that way and 55 this way, for 36 of
+// HBM time.
+constexpr int kGeluLo = 118 << 7, kGeluHi = 131 << 7;  // bf16 magnitude bits: 2^-9, 16
+constexpr int kGeluHalf = kGeluHi - kGeluLo;           // values per sign
+__device__ __forceinline__ uint16_t gelu_bf16_erf(uint32_t b) {
+  return f32_to_bf16_bits(gelu_erf(bf16_bits_to_f32(static_cast<uint16_t>(b))));
+}
+__device__ __forceinline__ void gelu_table_fill(uint16_t *table) {
+  for (int i = threadIdx.x; i < 2 * kGeluHalf; i += kStatsThreads)
+    table[i] = gelu_bf16_erf(i < kGeluHalf ? kGeluLo + i : 0x8000 + kGeluLo + i - kGeluHalf);
+}
+__device__ __forceinline__ uint32_t gelu_lookup(uint32_t b, const uint16_t *table) {
+  const int a = static_cast<int>(b & 0x7fffu);
+  const int i = min(max(a - kGeluLo, 0), kGeluHalf - 1) + (b & 0x8000u ? kGeluHalf : 0);
+  uint32_t g = a < kGeluLo ? b - 0x80u : table[i];
+  if (a >= kGeluHi || a < 0x100) g = gelu_bf16_erf(b);
+  return g;
+}
+
 // Element access of one lane's VEC consecutive channels: `raw` loads their
 // bits (16 bytes for the vector forms, one element otherwise) and `cvt`
 // widens them to FP32.  Keeping the raw bits in registers until they are
@@ -180,7 +206,7 @@ static_assert(sizeof(StatsPack) <= 4000, "StatsPack is passed by value in the ke
 // the transformed values a later read of the output would load.
 template <int DT, int VEC, int CT, int U, int MODE, int CAST, int XF>
 __device__ __forceinline__ void stats_tile(const StatsJob &J, int64_t tile, int64_t chunk, float *red,
-                                           const InMap &m = InMap{}) {
+                                           const InMap &m = InMap{}, const uint16_t *gelu_table = nullptr) {
   using E = Elems<DT, VEC>;
   using Raw = typename E::Raw;
   constexpr bool FIRST = MODE != kSqOnly && MODE != kSqDefer;
@@ -229,8 +255,19 @@ __device__ __forceinline__ void stats_tile(const StatsJob &J, int64_t tile, int6
         *reinterpret_cast<uint4 *>(o) = q;
       }
       float v[VEC];
-      E::cvt(q, v);
-      if constexpr (XF == kXfGelu) {
+      if constexpr (XF == kXfGelu && DT == SMX_BF16) {
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+        uint32_t o[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          o[k] = gelu_lookup(w[k] & 0xffffu, gelu_table) | (gelu_lookup(w[k] >> 16, gelu_table) << 16);
+        const uint4 g = make_uint4(o[0], o[1], o[2], o[3]);
+        *reinterpret_cast<uint4 *>(static_cast<uint16_t *>(J.cast_out) + row * J.out_stride + col0) = g;
+        E::cvt(g, v);
+      } else {
+        E::cvt(q, v);
+      }
+      if constexpr (XF == kXfGelu && DT != SMX_BF16) {
 #pragma unroll
         for (int k = 0; k < VEC; ++k) {
           float g = gelu_erf(v[k]);
@@ -238,8 +275,7 @@ __device__ __forceinline__ void stats_tile(const StatsJob &J, int64_t tile, int6
           // (torch rounds its FP32 result): the compiler would otherwise fold
           // the last multiply into a mixed FMA that rounds to f16 once.
           asm volatile("" : "+v"(g));
-          if constexpr (DT == SMX_BF16) v[k] = bf16_bits_to_f32(f32_to_bf16_bits(g));
-          else v[k] = f16_bits_to_f32(__builtin_bit_cast(uint16_t, static_cast<_Float16>(g)));
+          v[k] = f16_bits_to_f32(__builtin_bit_cast(uint16_t, static_cast<_Float16>(g)));
         }
         store_cast<DT, VEC>(J.cast_out, row * J.out_stride + col0, v);
       }
@@ -352,9 +388,11 @@ constexpr int64_t kStatsMinChunkRows = 512;
 // register budget).
 template <int FORM, int MODE, int CAST, int XF>
 __device__ __forceinline__ void run_tile(const StatsJob &J, int64_t tile, int64_t chunk, float *red,
-                                         const InMap &m = InMap{}) {
+                                         const InMap &m = InMap{}, const uint16_t *gelu_table = nullptr) {
   using F = FormTraits<FORM>;
-  stats_tile<F::DT, F::VEC, F::CT, XF == kXfGelu ? 2 : F::U, MODE, CAST, XF>(J, tile, chunk, red, m);
+  // (the f16 GELU, bound by its erf, keeps two loads per batch)
+  constexpr int U = XF == kXfGelu && F::DT != SMX_BF16 ? 2 : F::U;
+  stats_tile<F::DT, F::VEC, F::CT, U, MODE, CAST, XF>(J, tile, chunk, red, m, gelu_table);
 }
 
 // The job of block b of a launch: block_begin grows with the job index, so
@@ -416,12 +454,17 @@ __global__ void __launch_bounds__(kStatsThreads) stats_gelu_kernel(StatsPack pac
   const StatsJob J = pack.job[stats_job_of(pack, b)];
   const int64_t local = b - J.block_begin;
   const int64_t tile = local % J.tiles, chunk = local / J.tiles;
+  __shared__ uint16_t table[2 * kGeluHalf];
+  if (J.code / (kStatsModes * 3 * kStatsXforms) == kBf16V8) {
+    gelu_table_fill(table);
+    __syncthreads();
+  }
 #define SMX_STATS_GELU(FORM)                                                                   \
   case stats_code(FORM, kSqDefer, 0, kXfGelu):                                                 \
-    run_tile<FORM, kSqDefer, 0, kXfGelu>(J, tile, chunk, red);                                 \
+    run_tile<FORM, kSqDefer, 0, kXfGelu>(J, tile, chunk, red, InMap{}, table);                 \
     break;                                                                                     \
   case stats_code(FORM, kSqFirstDefer, 0, kXfGelu):                                            \
-    run_tile<FORM, kSqFirstDefer, 0, kXfGelu>(J, tile, chunk, red);                            \
+    run_tile<FORM, kSqFirstDefer, 0, kXfGelu>(J, tile, chunk, red, InMap{}, table);            \
     break;
   switch (J.code) {
     SMX_STATS_GELU(kBf16V8)
