@@ -431,6 +431,14 @@ int smx_rank1_apply(int dtype, const void *x, void *out, int64_t batch,
                     const void *rz, const void *rc, int order, double *work,
                     void *stream);
 
+/* smx_rank1_apply with factors that serve the whole batch: shared bit 0 for
+ * the left one (li/lz of [rows], lc one element), bit 1 for the right one. */
+int smx_rank1_apply_shared(int dtype, const void *x, void *out, int64_t batch,
+                           int64_t rows, int64_t cols, const void *li,
+                           const void *lz, const void *lc, const void *ri,
+                           const void *rz, const void *rc, int shared,
+                           int order, double *work, void *stream);
+
 int smx_graft(const float *x, float *out, int64_t n, int64_t output_rows,
               double *work, int32_t work_len, void *stream);
 

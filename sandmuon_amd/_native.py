@@ -122,6 +122,8 @@ SIGNATURES = {
                                  c_void_p]),
     "smx_rank1_apply": (c_int, [c_int, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p,
                                 c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p]),
+    "smx_rank1_apply_shared": (c_int, [c_int, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p,
+                                       c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p]),
     "smx_graft": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_int32, c_void_p]),
     "smx_s8_comp_stages": (c_int, [c_int32]),
     "smx_s8_comp_mask": (c_int, [c_int32]),
@@ -500,14 +502,16 @@ def inverse_sqrt(kind: int, second: torch.Tensor, mean: Optional[torch.Tensor], 
 
 def rank1_apply(x: torch.Tensor, out: torch.Tensor, left, right, order: int) -> None:
     """x, out: contiguous [batch, rows, cols]; left/right: (inv, z, coef) of
-    shapes [batch, n], [batch, n], [batch], all of x's dtype."""
+    shapes [batch, n], [batch, n], [batch], or [n], [n], [1] for the whole
+    batch, all of x's dtype."""
     b, r, c = x.shape
     li, lz, lc = left
     ri, rz, rc_ = right
     work = torch.empty(max(b * (r + c), 1), dtype=torch.float64, device=x.device)
-    rc = lib().smx_rank1_apply(helper_dtype_code(x.dtype), x.data_ptr(), out.data_ptr(), b, r, c, li.data_ptr(),
-                               lz.data_ptr(), lc.data_ptr(), ri.data_ptr(), rz.data_ptr(), rc_.data_ptr(), order,
-                               work.data_ptr(), stream_of(x.device))
+    shared = (1 if li.dim() == 1 else 0) | (2 if ri.dim() == 1 else 0)
+    rc = lib().smx_rank1_apply_shared(helper_dtype_code(x.dtype), x.data_ptr(), out.data_ptr(), b, r, c,
+                                      li.data_ptr(), lz.data_ptr(), lc.data_ptr(), ri.data_ptr(), rz.data_ptr(),
+                                      rc_.data_ptr(), shared, order, work.data_ptr(), stream_of(x.device))
     _check(rc, "smx_rank1_apply")
 
 

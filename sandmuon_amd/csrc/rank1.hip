@@ -15,7 +15,7 @@
 //   mapback (order 1): V1 = X + (lc lz_i) t_j;  V2 = V1 + (rc u_i) rz_j;
 //                      out = (V2 li) ri
 // in two launches: column sums (a block per 32 columns, 32 row groups),
-// then the rows (one wave per row: its sum, then its output).
+// then the rows (one or four waves each: their sums, then their output).
 #include "common.h"
 
 #include <algorithm>
@@ -29,24 +29,18 @@ struct Rank1Args {
   const T *x;
   T *out;
   int64_t rows, cols;
-  const T *li, *lz, *lc;  // [batch][rows], [batch][rows], [batch]
-  const T *ri, *rz, *rc;  // [batch][cols], [batch][cols], [batch]
+  const T *li, *lz, *lc;  // [batch or 1][rows], [batch or 1][rows], [batch or 1]
+  const T *ri, *rz, *rc;  // [batch or 1][cols], [batch or 1][cols], [batch or 1]
   double *t;              // [batch][cols] column sums lz^T V
   int32_t order;
+  int64_t lb, rb;         // 1, or 0 where one left (right) factor serves the whole batch
 };
 
 // The first-stage value V0 (whiten) or X (mapback) of element (i, j).
 template <typename T>
 __device__ __forceinline__ T r1_v0(const Rank1Args<T> &a, int64_t b, int64_t i, int64_t j) {
   const T x = a.x[(b * a.rows + i) * a.cols + j];
-  return a.order == 0 ? (x * a.li[b * a.rows + i]) * a.ri[b * a.cols + j] : x;
-}
-
-// V1 of element (i, j): V0 + (lc lz_i) t_j.
-template <typename T>
-__device__ __forceinline__ T r1_v1(const Rank1Args<T> &a, int64_t b, int64_t i, int64_t j) {
-  const T t = static_cast<T>(a.t[b * a.cols + j]);
-  return r1_v0(a, b, i, j) + (a.lc[b] * a.lz[b * a.rows + i]) * t;
+  return a.order == 0 ? (x * a.li[a.lb * b * a.rows + i]) * a.ri[a.rb * b * a.cols + j] : x;
 }
 
 // t[b][j] = sum_i lz_i V0_ij: a block takes kColTile columns, its kColRows
@@ -70,7 +64,7 @@ __global__ void __launch_bounds__(kColTile * kColRows) rank1_colsum_kernel(Rank1
       for (int u = 0; u < kColUnroll; ++u) {
         const int64_t i = i0 + kColRows * u;
         const bool in = i < a.rows;
-        lz[u] = in ? static_cast<double>(a.lz[b * a.rows + i]) : 0.0;
+        lz[u] = in ? static_cast<double>(a.lz[a.lb * b * a.rows + i]) : 0.0;
         v[u] = in ? static_cast<double>(r1_v0(a, b, i, j)) : 0.0;
       }
 #pragma unroll
@@ -85,42 +79,61 @@ __global__ void __launch_bounds__(kColTile * kColRows) rank1_colsum_kernel(Rank1
   }
 }
 
-// One wave per row: u_i = sum_j V1_ij rz_j (FP64), then the output of the
-// row, which it reads a second time from cache; kRowUnroll loads in flight
-// per lane.  (Row sums and an output pass with a thread per element as two
-// launches: 12 + 12 us for [4, 640, 1280].)  grid (ceil(rows / 4), batch).
-constexpr int kRowUnroll = 4;
-template <typename T>
+// A row by kW waves: u_i = sum_j V1_ij rz_j (FP64), then the row's output,
+// from registers where the row is one round of kRowUnroll columns per lane
+// and else from a second read.  Bound by latency at helper sizes: four waves
+// per row give a CU 40 waves for [4, 640, 1280] (11 us), where one wave per
+// row left it at 10 with five rounds in series (22 us).
+// grid (ceil(rows kW / 4), batch), block 256.
+constexpr int kRowUnroll = 8;
+template <typename T, int kW>
 __global__ void __launch_bounds__(256) rank1_row_kernel(Rank1Args<T> a) {
+  __shared__ double part[4];
+  constexpr int kLanes = 64 * kW, kRound = kLanes * kRowUnroll;
   const int64_t b = blockIdx.y;
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (i >= a.rows) return;  // wave-uniform
-  double s = 0.0;
-  for (int64_t j0 = lane; j0 < a.cols; j0 += 64 * kRowUnroll) {
-    double v[kRowUnroll], rz[kRowUnroll];
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * (4 / kW) + threadIdx.x / kLanes;
+  if (i >= a.rows) return;  // uniform over the row's waves
+  const int lane = threadIdx.x % kLanes;
+  const T li = a.li[a.lb * b * a.rows + i];
+  const T cl = a.lc[a.lb * b] * a.lz[a.lb * b * a.rows + i];
+  const T *x = a.x + (b * a.rows + i) * a.cols;
+  T *out = a.out + (b * a.rows + i) * a.cols;
+  const T *ri = a.ri + a.rb * b * a.cols, *rz = a.rz + a.rb * b * a.cols;
+  const double *t = a.t + b * a.cols;
+  const bool whiten = a.order == 0;
+  T v[kRowUnroll], r[kRowUnroll], z[kRowUnroll];  // V1, ri and rz of the lane's columns of one round
+  auto load = [&](int64_t j0) {
+    T c[kRowUnroll];
 #pragma unroll
     for (int u = 0; u < kRowUnroll; ++u) {
-      const int64_t j = j0 + 64 * u;
+      const int64_t j = j0 + kLanes * u;
       const bool in = j < a.cols;
-      v[u] = in ? static_cast<double>(r1_v1(a, b, i, j)) : 0.0;
-      rz[u] = in ? static_cast<double>(a.rz[b * a.cols + j]) : 0.0;
+      v[u] = in ? x[j] : static_cast<T>(0);
+      r[u] = in ? ri[j] : static_cast<T>(0);
+      z[u] = in ? rz[j] : static_cast<T>(0);
+      c[u] = in ? static_cast<T>(t[j]) : static_cast<T>(0);
     }
 #pragma unroll
-    for (int u = 0; u < kRowUnroll; ++u)
-      if (j0 + 64 * u < a.cols) s += v[u] * rz[u];
-  }
-  const T u = static_cast<T>(wave_sum(s));
-  const T cu = a.rc[b] * u, li = a.li[b * a.rows + i];
-  T *out = a.out + (b * a.rows + i) * a.cols;
-  for (int64_t j0 = lane; j0 < a.cols; j0 += 64 * kRowUnroll) {
+    for (int u = 0; u < kRowUnroll; ++u) v[u] = (whiten ? (v[u] * li) * r[u] : v[u]) + cl * c[u];
+  };
+  double s = 0.0;
+  for (int64_t j0 = lane; j0 < a.cols; j0 += kRound) {
+    load(j0);
 #pragma unroll
-    for (int q = 0; q < kRowUnroll; ++q) {
-      const int64_t j = j0 + 64 * q;
+    for (int u = 0; u < kRowUnroll; ++u)
+      if (j0 + kLanes * u < a.cols) s += static_cast<double>(v[u]) * static_cast<double>(z[u]);
+  }
+  s = kW == 1 ? wave_sum(s) : block_sum(s, part);
+  const T cu = a.rc[a.rb * b] * static_cast<T>(s);
+  for (int64_t j0 = lane; j0 < a.cols; j0 += kRound) {
+    if (a.cols > kRound) load(j0);
+#pragma unroll
+    for (int u = 0; u < kRowUnroll; ++u) {
+      const int64_t j = j0 + kLanes * u;
       if (j >= a.cols) continue;
-      T v = r1_v1(a, b, i, j) + cu * a.rz[b * a.cols + j];
-      if (a.order == 1) v = (v * li) * a.ri[b * a.cols + j];
-      out[j] = v;
+      T w = v[u] + cu * z[u];
+      if (!whiten) w = (w * li) * r[u];
+      out[j] = w;
     }
   }
 }
@@ -132,7 +145,13 @@ static int launch_rank1(const Rank1Args<T> &a, int64_t batch, hipStream_t st) {
                      dim3(kColTile * kColRows), 0, st, a);
   int rc = check_launch("rank1_apply column sums");
   if (rc) return rc;
-  hipLaunchKernelGGL(rank1_row_kernel<T>, dim3(static_cast<unsigned>(ceil_div(a.rows, 4)), nb), dim3(256), 0, st, a);
+  // Four waves per row from 256 columns on (four columns per lane with one),
+  // as long as the rows alone don't fill the device many times over.
+  if (a.cols >= 256 && a.rows <= 65536)
+    hipLaunchKernelGGL((rank1_row_kernel<T, 4>), dim3(static_cast<unsigned>(a.rows), nb), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((rank1_row_kernel<T, 1>), dim3(static_cast<unsigned>(ceil_div(a.rows, 4)), nb), dim3(256), 0,
+                       st, a);
   return check_launch("rank1_apply rows");
 }
 
@@ -240,9 +259,11 @@ extern "C" int smx_inverse_sqrt(int kind, int dtype, const void *second, const v
   return check_launch("inverse_sqrt");
 }
 
-extern "C" int smx_rank1_apply(int dtype, const void *x, void *out, int64_t batch, int64_t rows, int64_t cols,
-                               const void *li, const void *lz, const void *lc, const void *ri, const void *rz,
-                               const void *rc, int order, double *work, void *stream) {
+extern "C" int smx_rank1_apply_shared(int dtype, const void *x, void *out, int64_t batch, int64_t rows, int64_t cols,
+                                      const void *li, const void *lz, const void *lc, const void *ri, const void *rz,
+                                      const void *rc, int shared, int order, double *work, void *stream) {
+  SMX_REQUIRE(shared >= 0 && shared <= 3, SMX_EINVAL, "rank1_apply: shared must be in [0, 3]");
+  const int64_t lb = shared & 1 ? 0 : 1, rb = shared & 2 ? 0 : 1;
   SMX_REQUIRE(dtype == SMX_F32 || dtype == SMX_F64, SMX_EDTYPE, "rank1_apply: dtype must be f32 or f64");
   SMX_REQUIRE(x && out && li && lz && lc && ri && rz && rc && work, SMX_EINVAL, "rank1_apply: null pointer");
   SMX_REQUIRE(order == 0 || order == 1, SMX_EINVAL, "rank1_apply: order must be 0 (whiten) or 1 (mapback)");
@@ -256,14 +277,20 @@ extern "C" int smx_rank1_apply(int dtype, const void *x, void *out, int64_t batc
     Rank1Args<float> a{static_cast<const float *>(x), static_cast<float *>(out), rows, cols,
                        static_cast<const float *>(li), static_cast<const float *>(lz), static_cast<const float *>(lc),
                        static_cast<const float *>(ri), static_cast<const float *>(rz), static_cast<const float *>(rc),
-                       t, order};
+                       t, order, lb, rb};
     return launch_rank1(a, batch, st);
   }
   Rank1Args<double> a{static_cast<const double *>(x), static_cast<double *>(out), rows, cols,
                       static_cast<const double *>(li), static_cast<const double *>(lz),
                       static_cast<const double *>(lc), static_cast<const double *>(ri),
-                      static_cast<const double *>(rz), static_cast<const double *>(rc), t, order};
+                      static_cast<const double *>(rz), static_cast<const double *>(rc), t, order, lb, rb};
   return launch_rank1(a, batch, st);
+}
+
+extern "C" int smx_rank1_apply(int dtype, const void *x, void *out, int64_t batch, int64_t rows, int64_t cols,
+                               const void *li, const void *lz, const void *lc, const void *ri, const void *rz,
+                               const void *rc, int order, double *work, void *stream) {
+  return smx_rank1_apply_shared(dtype, x, out, batch, rows, cols, li, lz, lc, ri, rz, rc, 0, order, work, stream);
 }
 
 extern "C" int smx_graft(const float *x, float *out, int64_t n, int64_t output_rows, double *work, int32_t work_len,

@@ -94,6 +94,9 @@ def rank1_inverse_sqrt(second: torch.Tensor, mean: torch.Tensor):
 
 
 def _batched_factor(f, batch_shape, n, dt):
+    vec, z, c = (torch.as_tensor(t) for t in f)
+    if vec.shape == (n,) and z.shape == (n,) and c.dim() == 0:  # one factor for the whole batch
+        return _to_gpu(vec, dt), _to_gpu(z, dt), _to_gpu(c, dt)
     vec = _to_gpu(f[0], dt).expand(*batch_shape, n).reshape(-1, n).contiguous()
     z = _to_gpu(f[1], dt).expand(*batch_shape, n).reshape(-1, n).contiguous()
     c = _to_gpu(f[2], dt).expand(torch.Size(batch_shape)).reshape(-1).contiguous()

@@ -30,3 +30,25 @@ def test_rank1_apply_edges(device, dtype, tol, shape):
         one = lambda f: tuple(t[k].double() for t in f)
         want = O.rank1_mapback(x[k].double(), one(left), one(right))
         assert (got[k] - want).norm() <= tol * want.norm()
+
+
+@pytest.mark.parametrize("shared", ["left", "right", "both"])
+@pytest.mark.parametrize("shape", [(3, 33, 65), (2, 5, 256), (4, 7, 2048), (2, 6, 2049), (2, 65537, 257)])
+def test_factors_shared_by_the_batch_equal_expanded_ones(device, shape, shared):
+    # A row on one wave and on four, on one round of columns and on two: the
+    # same values are read, so the bits are the same.
+    b, r, c = shape
+    g = torch.Generator().manual_seed(b + 10 * r + 100 * c)
+    x = torch.randn(shape, generator=g).to(device)
+    one = lambda n: tuple(t.to(device) for t in (torch.rand(n, generator=g) + .5, torch.randn(n, generator=g) * .3 / n ** .5,
+                                                 torch.tensor(-.25)))
+    many = lambda f: (f[0].expand(b, -1).contiguous(), f[1].expand(b, -1).contiguous(), f[2].expand(b).contiguous())
+    left, right = one(r), one(c)
+    lf = left if shared != "right" else many(left)
+    rf = right if shared != "left" else many(right)
+    for fn in (rank1_whiten, rank1_mapback):
+        got, want = fn(x, lf, rf), fn(x, many(left), many(right))
+        assert torch.equal(got, want)
+    k = b - 1
+    ref = O.rank1_whiten(x[k].double().cpu(), *[tuple(t.double().cpu() for t in f) for f in (left, right)])
+    assert (rank1_whiten(x, left, right)[k].double().cpu() - ref).norm() <= 1e-6 * ref.norm()
