@@ -93,10 +93,16 @@ def rank1_inverse_sqrt(second: torch.Tensor, mean: torch.Tensor):
     return out(inv), out(z), out(kappa)
 
 
-def _batched_factor(f, batch_shape, n, dt):
+def _factor(f, batch_shape, n, dt):
+    """A factor as rank1_apply takes it: unbatched where one serves the whole
+    batch (read in place), else expanded over the batch."""
     vec, z, c = (torch.as_tensor(t) for t in f)
-    if vec.shape == (n,) and z.shape == (n,) and c.dim() == 0:  # one factor for the whole batch
+    if vec.shape == (n,) and z.shape == (n,) and c.dim() == 0:
         return _to_gpu(vec, dt), _to_gpu(z, dt), _to_gpu(c, dt)
+    return _batched_factor(f, batch_shape, n, dt)
+
+
+def _batched_factor(f, batch_shape, n, dt):
     vec = _to_gpu(f[0], dt).expand(*batch_shape, n).reshape(-1, n).contiguous()
     z = _to_gpu(f[1], dt).expand(*batch_shape, n).reshape(-1, n).contiguous()
     c = _to_gpu(f[2], dt).expand(torch.Size(batch_shape)).reshape(-1).contiguous()
@@ -110,8 +116,8 @@ def _rank1(matrix: torch.Tensor, left, right, order: int) -> torch.Tensor:
     batch_shape = x.shape[:-2]
     xb = x.reshape(-1, r, c)
     out = torch.empty_like(xb)
-    lf = _batched_factor(left, batch_shape, r, dt)
-    rf = _batched_factor(right, batch_shape, c, dt)
+    lf = _factor(left, batch_shape, r, dt)
+    rf = _factor(right, batch_shape, c, dt)
     _native.rank1_apply(xb, out, lf, rf, order)
     res = out.reshape(x.shape)
     return res.to(matrix.device, torch.promote_types(matrix.dtype, dt))
@@ -684,6 +690,8 @@ class DiagonalWeightedPE(Optimizer):
                              self._descriptor_stage(device))
         for s in sources:
             self.state[s]["a_count"] = 0
+        for parameter, _, _ in items:
+            self.state[parameter]["b_count"] = 0
 
         # Converted or re-laid-out gradients are temporaries: they must stay
         # alive until the launch that reads them is enqueued (the allocator
@@ -692,7 +700,6 @@ class DiagonalWeightedPE(Optimizer):
         packed, shapes, keep = bytearray(size * len(items)), [], []
         for k, (parameter, source, group) in enumerate(items):
             state = self.state[parameter]
-            state["b_count"] = 0
             if not parameter.is_contiguous():
                 _check_layout(parameter, self.parameter_names[id(parameter)], True)
             momentum = state.get("momentum_buffer")
@@ -761,8 +768,8 @@ class DiagonalWeightedPE(Optimizer):
                     _native.dtype_code(parameter.dtype))
                 offset += n
             lr = group["lr"] * group["adamw_lr_ratio"]
-            _native.adamw(_native.table(_native.AdamwDesc, packed), offset, lr, b1, b2, group["adamw_eps"], group["weight_decay"], device,
-                          self._descriptor_stage(device))
+            _native.adamw(_native.table(_native.AdamwDesc, packed), offset, lr, b1, b2, group["adamw_eps"],
+                          group["weight_decay"], device, self._descriptor_stage(device))
             del keep
 
     def close(self):

@@ -111,6 +111,19 @@ def test_helper_factor_batching(monkeypatch):
     assert M._work_dtype(torch.zeros(2, dtype=torch.bfloat16)) == torch.float32
 
 
+def test_helper_factor_shared(monkeypatch):
+    # An unbatched factor is handed on as it is, a batched one and one whose
+    # parts differ in rank per matrix.
+    from sandmuon_amd import optimizer as M
+    monkeypatch.setattr(M, "_to_gpu", lambda t, dtype: torch.as_tensor(t).to(dtype).contiguous())
+    vec, z, c, batch = torch.rand(5), torch.rand(5), torch.tensor(-.4), torch.Size([2, 3])
+    assert [t.shape for t in M._factor((vec, z, c), batch, 5, torch.float32)] == [(5,), (5,), ()]
+    for factor in ((vec.expand(2, 3, 5), z, c), (vec, z, c.expand(2, 3)), (vec, z.expand(3, 5), c)):
+        v, w, k = M._factor(factor, batch, 5, torch.float64)
+        assert v.shape == w.shape == (6, 5) and k.shape == (6,)
+        assert torch.equal(v, vec.double().expand(6, 5)) and torch.equal(w, z.double().expand(6, 5))
+
+
 def _bare_optimizer(params):
     """A DiagonalWeightedPE shell over CPU parameters: torch's Optimizer
     state without the GPU constructor (no hooks, no library calls), enough
