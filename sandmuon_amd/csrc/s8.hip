@@ -1431,8 +1431,12 @@ s8_stage_kernel(StageArgs args) {
   // FP32: the mapback's and the stand-alone map's input).
   const bool tiled_t = !(PHASE == kApply && last && (ref.op == kOpApplyX || ref.op == kOpApplyFinal));
   const bool tiled_m = PHASE != kApply;
-  // add eye_a on the diagonal: a I of P, or -I of H (shift)
-  const bool eye = (PHASE == kSquare && stage != 1) || (PHASE == kGram && shift);
+  // add eye_a on the diagonal: a I of P, or -I of H (shift).  Only a diagonal
+  // tile holds any of it, and such a tile has no mirror: the other tiles
+  // branch over that code, and the staged rows (put_row) have none.  (A
+  // short launch is bound by the code it fetches: one 512 x 512 matrix 184 ->
+  // 173 us a call; 36 of 768 x 768 in fp32 mode 1207 -> 1189 us.)
+  const bool eye = diag && ((PHASE == kSquare && stage != 1) || (PHASE == kGram && shift));
   const float eye_a = !kPair ? args.a : PHASE == kGram ? -pow2f(kExpG) : (shift ? args.ah : args.a) * pow2f(kExpP);
   // the wave's staging block of a transposed output: [column][row]
   float *const U = reinterpret_cast<float *>(smem) + wave * 2 * kEpBlock;
@@ -1518,10 +1522,6 @@ s8_stage_kernel(StageArgs args) {
     if constexpr (FM == kFormF16) {
       const f32x4 v4 = *reinterpret_cast<const f32x4 *>(S + row * kEpStride + ec4);
       float w[4] = {v4.x, v4.y, v4.z, v4.w};
-      if (eye)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (gr == gc0 + ec4 + e && gr < K.r) w[e] += eye_a;
       uint32_t b[2];
 #pragma unroll
       for (int e = 0; e < 2; ++e)
@@ -1543,10 +1543,6 @@ s8_stage_kernel(StageArgs args) {
     if (pl) {
       float w[8];
       ep_read8(S, row, ec8, w);
-      if (eye)
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (gr == gc0 + ec8 + e && gr < K.r) w[e] += eye_a;
       uint32_t b[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -1558,10 +1554,6 @@ s8_stage_kernel(StageArgs args) {
     } else {
       const f32x4 v4 = *reinterpret_cast<const f32x4 *>(S + row * kEpStride + ec4);
       float w[4] = {v4.x, v4.y, v4.z, v4.w};
-      if (eye)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (gr == gc0 + ec4 + e && gr < K.r) w[e] += eye_a;
       *reinterpret_cast<float4 *>(out) = make_float4(w[0], w[1], w[2], w[3]);
       if (acc_r) accum4(w, gc0 + ec4, r);
     }
@@ -1678,10 +1670,13 @@ s8_stage_kernel(StageArgs args) {
       for (int e = 0; e < 16; ++e)
         if (do_m) U[col16(e) * kEpStride + lr] = w[e];
       if (do_t) {
-        if (eye)
+        if (eye) {
+          // the diagonal's column in the lane's col16 order, if it has one
+          const int d = gr < K.r ? static_cast<int>(gr - cb) - col16(0) : -1;
 #pragma unroll
           for (int e = 0; e < 16; ++e)
-            if (gr == cb + col16(e) && gr < K.r) w[e] += eye_a;
+            if (d == col16(e) - col16(0)) w[e] += eye_a;
+        }
         put_direct(fm_c, w, gr, cb, dst_t, ld_t, tiled_t);
         if (rs_on) {
           // a and z of the lane's columns, then the row's two lanes (lh)
