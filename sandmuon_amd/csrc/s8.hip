@@ -990,9 +990,13 @@ __device__ __forceinline__ void gemm_tile(const Opnd &A_in, const Opnd &B_in, in
 // ahead (their 16-byte chunks are what a lane's MFMA takes, and nothing is
 // shared between waves); a K-major B goes through a wave-private LDS
 // buffer for its transposed reads.  No barrier inside the K loop.  Then the
-// partials are added through LDS in wave order, and waves 0 and 1 hold the
-// tile's 32 x 32 blocks: blocks (w, 0) and (w, 1), or, by_col, (0, w) and
-// (1, w), in acc[0][0] and acc[0][1].  Bound by latency: a launch of a
+// partials are added through LDS in wave order.  Of a symmetric result each
+// wave then holds one of the tile's 32 x 32 blocks, block (w / 2, w % 2) in
+// acc[0][0].  Of an apply, whose row sums run over a whole tile row, waves 0
+// and 1 hold two: blocks (w, 0) and (w, 1), or, by_col, (0, w) and (1, w), in
+// acc[0][0] and acc[0][1].  (A wave per block instead of two blocks in
+// waves 0 and 1 halves what a symmetric launch's wave fetches and runs after
+// the K loop: one 512 x 512 matrix 173 -> 162 us a call.)  Bound by latency: a launch of a
 // single 768 x 768 matrix takes 48 K stages as one chain of 21 blocks in
 // 128 x 128 tiles, here 12 in 84 blocks.
 constexpr int kDeep = 4;
@@ -1097,10 +1101,10 @@ __device__ __forceinline__ void gemm_tile_split(const Opnd &A_in, const Opnd &B_
         part[((wave * 4 + 2 * i + j) * 4 + q) * 64 + lane] =
             f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
   __syncthreads();
-  if (wave < 2) {
+  if (!BKM || wave < 2) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int blk = by_col ? 2 * b + wave : 2 * wave + b;
+    for (int b = 0; b < (BKM ? 2 : 1); ++b) {
+      const int blk = !BKM ? wave : by_col ? 2 * b + wave : 2 * wave + b;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         f32x4 v = part[(blk * 4 + q) * 64 + lane];
@@ -1391,9 +1395,13 @@ s8_stage_kernel(StageArgs args) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wm = wave / Gm::kWavesN, wn = wave % Gm::kWavesN;
   const int lr = lane & 31, lh = lane >> 5;
-  // The wave's blocks: kSubM x kSubN from (R0, C0); kGeoT two (waves 0, 1).
-  const int64_t R0 = tm * Gm::kTileM + (Gm::kSplitK ? (by_col ? 0 : 32 * wave) : wm * (32 * kSubM));
-  const int64_t C0 = tn * kTileN + (Gm::kSplitK ? (by_col ? 32 * wave : 0) : wn * (32 * kSubN));
+  // The wave's blocks: kSubM x kSubN from (R0, C0); kGeoT one (kQuad), or two
+  // (waves 0, 1 of an apply).
+  constexpr bool kQuad = Gm::kSplitK && PHASE != kApply;
+  const int64_t R0 = tm * Gm::kTileM + (kQuad ? 32 * (wave >> 1)
+                                        : Gm::kSplitK ? (by_col ? 0 : 32 * wave) : wm * (32 * kSubM));
+  const int64_t C0 = tn * kTileN + (kQuad ? 32 * (wave & 1)
+                                    : Gm::kSplitK ? (by_col ? 32 * wave : 0) : wn * (32 * kSubN));
   const bool last = stage == 5;
   float *dst_t, *dst_m;
   int64_t ld_t, ld_m;
@@ -1653,7 +1661,7 @@ s8_stage_kernel(StageArgs args) {
     float rsd[3] = {0.f, 0.f, 0.f};
     // (expanded at compile time: a rolled block loop indexes acc at run
     // time, which moves every accumulator of the kernel to scratch memory)
-    static_for<Gm::kSplitK ? 2 : kSubM * kSubN>([&](auto blk_c) {
+    static_for<kQuad ? 1 : Gm::kSplitK ? 2 : kSubM * kSubN>([&](auto blk_c) {
       constexpr int blk = decltype(blk_c)::value, i = blk / kSubN, j = blk % kSubN;
       const int64_t rb = R0 + (Gm::kSplitK && by_col ? blk : i) * 32;
       const int64_t gr = rb + lr, cb = C0 + (Gm::kSplitK && by_col ? 0 : j) * 32;
@@ -1724,7 +1732,7 @@ s8_stage_kernel(StageArgs args) {
   };
   // Only the forms this launch kind can produce are compiled (the host
   // checks every launch's forms against the same table, form_compiled).
-  const bool owns = !Gm::kSplitK || wave < 2;  // the wave holds blocks of the tile
+  const bool owns = !Gm::kSplitK || kQuad || wave < 2;  // the wave holds blocks of the tile
   constexpr bool kPlanes = form_compiled(MODE, PHASE, kFormPlanes);
   constexpr bool kF16 = form_compiled(MODE, PHASE, kFormF16);
   constexpr bool kF32 = form_compiled(MODE, PHASE, kFormF32);
