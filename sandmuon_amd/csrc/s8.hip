@@ -237,14 +237,20 @@ constexpr int kBK = 16;             // K per pipeline stage
 // (its 256 A rows serve 256 B rows: cfg5 S8 7% faster).  A round of the
 // device's block slots does the same work in M and L; the host picks the
 // geometry per launch (pick_geo).
-//   kGeoT  64 x 64, 4 waves of 64 x 64 that each take a quarter of K
-//          (gemm_tile_split), two blocks per CU: for launches that leave
-//          CUs idle, where the length of a tile's chain of K stages is the
-//          launch's time.
+//   kGeoT  64 x 64, 4 waves of 32 x 32 (gemm_tile_quad), two blocks per CU:
+//          for launches that leave CUs idle, where the length of a tile's
+//          chain of K stages is the launch's time: a quarter of kGeoS's.
+// Every geometry adds the products of an output in the same order (K stage
+// by K stage, each stage's as mma_row issues them, the square's one_hot
+// products after those of their stage).  kGeoT and kGeoS also compute and
+// mirror the same elements of a symmetric result (those of kGeoM and kGeoL
+// differ below the diagonal of a 256 x 256 diagonal block, which they
+// compute: mma_row's two correction products swap there), so a matrix has
+// the same bits from either, whatever else is in its launch.
 enum TileGeo { kGeoM = 0, kGeoS = 1, kGeoL = 2, kGeoT = 3 };
 template <int TM, int TN>
 struct Geo {
-  static constexpr bool kSplitK = false;
+  static constexpr bool kQuad = false;
   static constexpr int kTileM = TM, kTileN = TN;
   static constexpr int kSubM = TM / 64;             // 32x32 MFMA row tiles per wave
   static constexpr int kWavesN = TN / (32 * kSubN);
@@ -267,16 +273,16 @@ struct Geo {
 };
 template <>
 struct Geo<64, 64> {
-  static constexpr bool kSplitK = true;
+  static constexpr bool kQuad = true;
   static constexpr int kTileM = 64, kTileN = 64;
-  static constexpr int kSubM = 2, kWavesN = 1;  // a wave covers the whole tile
+  static constexpr int kSubM = 1, kWavesN = 2;  // the waves of the K loop: 2 x 2 of 32 x 32
   static constexpr int kWaves = 4;
   static constexpr int kThreads = 64 * kWaves;
-  static constexpr int kOpA = 0;                   // only a K-major B goes through LDS
-  static constexpr int kLoadsB = 4;                // 1 KB pieces of a K-major stage
-  static constexpr int kBufBytes = 2 * 4096;       // per wave: two K-major stages
-  static constexpr int kAccBytes = 64 * 64 * 4;    // per wave: its partial sums of the tile
-  static constexpr int kRingBytes = kWaves * kAccBytes;
+  static constexpr int kOpA = 64 * kBK * 4, kOpB = 64 * kBK * 4;
+  static constexpr int kStageBytes = kOpA + kOpB;
+  static constexpr int kStages = 4;                 // ring slots, each of two K stages
+  static constexpr int kRingBytes = kStages * 2 * kStageBytes;
+  static constexpr int kLoadsA = 1, kLoadsB = 1;    // 1 KB loads per wave and K stage
   static constexpr int kKmRow = 64 * 4, kKmRowH = 64 * 2;
   static constexpr int kWavesPerEU = 2;
   static constexpr int kGeo = kGeoT;
@@ -519,24 +525,15 @@ template <>
 struct AFrag<kS8CompMix> : AFrag<SMX_S8_COMP_BF16> {};
 template <>
 struct AFrag<kS8Pair> : AFrag<SMX_S8_COMP_BF16> {};  // FP16 bits
-template <int MODE>
-struct BFrags;
-template <>
-struct BFrags<SMX_S8_COMP_BF16> {
-  bf16x8 h[kSubN], l[kSubN];
+// N: the wave's 32-column blocks (kSubN; one in kGeoT).
+template <int MODE, int N = kSubN>
+struct BFrags {
+  bf16x8 h[N], l[N];  // kS8F16, kS8Pair: FP16 bits
 };
-template <>
-struct BFrags<SMX_S8_FP32> {
-  float v[kSubN][8];
+template <int N>
+struct BFrags<SMX_S8_FP32, N> {
+  float v[N][8];
 };
-template <>
-struct BFrags<kS8HiOnly> : BFrags<SMX_S8_COMP_BF16> {};
-template <>
-struct BFrags<kS8F16> : BFrags<SMX_S8_COMP_BF16> {};
-template <>
-struct BFrags<kS8CompMix> : BFrags<SMX_S8_COMP_BF16> {};
-template <>
-struct BFrags<kS8Pair> : BFrags<SMX_S8_COMP_BF16> {};  // FP16 bits
 
 // Both 16-byte chunks of a row's K slice are read (the lo plane, or FP16's
 // second 16 K).
@@ -559,14 +556,14 @@ __device__ __forceinline__ void load_a(const char *st, int wm, int i, AFrag<MODE
   }
 }
 
-template <int MODE, class G>
-__device__ __forceinline__ void load_b(const char *st, int wn, BFrags<MODE> &f) {
+template <int MODE, class G, int N>
+__device__ __forceinline__ void load_b(const char *st, int wn, BFrags<MODE, N> &f) {
   const int lane = threadIdx.x & 63;
   const int lr = lane & 31, lh = lane >> 5;
   const char *bt = st + G::kOpA;
 #pragma unroll
-  for (int j = 0; j < kSubN; ++j) {
-    const int r = wn * (32 * kSubN) + j * 32 + frag_row<MODE>(lr);
+  for (int j = 0; j < N; ++j) {
+    const int r = wn * (32 * N) + j * 32 + frag_row<MODE>(lr);
     if constexpr (MODE != SMX_S8_FP32) {
       f.h[j] = read_b16(bt, r, lh);
       if constexpr (two_chunks<MODE>()) f.l[j] = read_b16(bt, r, 2 + lh);
@@ -583,22 +580,23 @@ __device__ __forceinline__ void load_b(const char *st, int wn, BFrags<MODE> &f) 
 // (s >> 2), columns 16 (g & 1) + 4 c .. + 3 of the 32-column block with
 // c = sw23(4 (s & 3)) / 4 (the two bits of s & 3 swapped), so lane
 // 16 (g & 1) + 4 a + b of the block receives column 16 (g & 1) + 4 c(a) + b
-// = sw23 of its index at the 4 rows.  Column block j of wave wn is pieces
-// 4 wn + 2 j and 4 wn + 2 j + 1 (g & 1 picks one), logical chunk 2 plane +
+// = sw23 of its index at the 4 rows.  Column block b of the tile (j of wave
+// wn: b = N wn + j) is pieces 2 b and 2 b + 1 (g & 1 picks one), logical chunk 2 plane +
 // (c >> 1) = 2 plane + (s & 1), byte 8 (c & 1) = 8 ((s >> 1) & 1) of it.
 // The swizzle of rows k and k + 4 is the same, and its piece term is g & 1,
 // so the per-lane offsets (wn included) are one per plane (o[plane][0]) and
 // every read adds a constant.  FP16: lane s of group g addresses row
 // 8 (g >> 1) + (s >> 2) (+4 for the second read, + the second row block's
 // pieces for the second 16 K), columns 16 (g & 1) + 4 c .. + 3 of piece
-// 2 wn + j (32 columns), i.e. chunk 2 (g & 1) + (s & 1), byte
+// b (32 columns), i.e. chunk 2 (g & 1) + (s & 1), byte
 // 8 ((s >> 1) & 1); o[j][0] holds the offset of block j.  FP32: eight
 // 4-byte reads.  (The 16 lanes of a read address the same bytes as with
 // unpermuted columns, in another lane order: the same banks.)
 struct BkmLane {
   uint32_t o[2][2];
 };
-__device__ __forceinline__ BkmLane bkm_lane(int wn) {
+// b0: the wave's first column block.
+__device__ __forceinline__ BkmLane bkm_lane(int b0) {
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4, s = lane & 15;
   const int k = 8 * (g >> 1) + (s >> 2);
@@ -606,14 +604,14 @@ __device__ __forceinline__ BkmLane bkm_lane(int wn) {
   BkmLane L;
 #pragma unroll
   for (int pl = 0; pl < 2; ++pl) {
-    L.o[pl][0] = static_cast<uint32_t>((4 * wn + (g & 1)) * 1024 + k * 64 + 8 * ((s >> 1) & 1) +
+    L.o[pl][0] = static_cast<uint32_t>((2 * b0 + (g & 1)) * 1024 + k * 64 + 8 * ((s >> 1) & 1) +
                                        (((2 * pl + (s & 1)) ^ sw) << 4));
     L.o[pl][1] = 0;
   }
   return L;
 }
 
-__device__ __forceinline__ BkmLane bkm_lane_f16(int wn) {
+__device__ __forceinline__ BkmLane bkm_lane_f16(int b0) {
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4, s = lane & 15;
   const int k = 8 * (g >> 1) + (s >> 2);
@@ -621,23 +619,23 @@ __device__ __forceinline__ BkmLane bkm_lane_f16(int wn) {
   BkmLane L;
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    L.o[j][0] = static_cast<uint32_t>((2 * wn + j) * 1024 + k * 64 + 8 * ((s >> 1) & 1) +
+    L.o[j][0] = static_cast<uint32_t>((b0 + j) * 1024 + k * 64 + 8 * ((s >> 1) & 1) +
                                       (((2 * (g & 1) + (s & 1)) ^ sw) << 4));
     L.o[j][1] = 0;
   }
   return L;
 }
 
-template <int MODE, class G>
-__device__ __forceinline__ void load_b_km(const char *st, int wn, BFrags<MODE> &f, const BkmLane &L) {
+template <int MODE, class G, int N>
+__device__ __forceinline__ void load_b_km(const char *st, int wn, BFrags<MODE, N> &f, const BkmLane &L) {
   constexpr int kOpA = G::kOpA;
   const int lane = threadIdx.x & 63;
   const char *bt = st + kOpA;
   if constexpr (MODE == kS8F16) {
-    static_assert(kSubN == 2, "one lane offset per 32-column block");
+    static_assert(N <= 2, "one lane offset per 32-column block");
     constexpr int kBlockBytes = G::kKmRowH / 64 * 1024;  // the pieces of one 16-row block
 #pragma unroll
-    for (int j = 0; j < kSubN; ++j) {
+    for (int j = 0; j < N; ++j) {
       lds_char *q = to_lds(st) + L.o[j][0];
       asm volatile("" : "+v"(q));
 #pragma unroll
@@ -660,7 +658,7 @@ __device__ __forceinline__ void load_b_km(const char *st, int wn, BFrags<MODE> &
       asm volatile("" : "+v"(q[pl]));
     }
 #pragma unroll
-    for (int j = 0; j < kSubN; ++j) {
+    for (int j = 0; j < N; ++j) {
 #pragma unroll
       for (int pl = 0; pl < (is_split(MODE) ? 2 : 1); ++pl) {
         lds_char *p = q[pl] + (kOpA + 2 * j * 1024);
@@ -672,18 +670,18 @@ __device__ __forceinline__ void load_b_km(const char *st, int wn, BFrags<MODE> &
     }
   } else {
     // (FP32 mode, natural column order: frag_row.)  Lane (n, h), n =
-    // 64 wn + 32 j + (lane & 31): piece 4 wn + 2 j + ((lane >> 4) & 1),
+    // 32 (N wn + j) + (lane & 31): piece 2 (N wn + j) + ((lane >> 4) & 1),
     // element 4 ((lane >> 2) & 3) + (lane & 3) of rows 8 h + q (no swizzle).
-    const char *base = bt + (4 * wn + ((lane >> 4) & 1)) * 1024 + 512 * (lane >> 5) + 4 * (lane & 15);
+    const char *base = bt + (2 * N * wn + ((lane >> 4) & 1)) * 1024 + 512 * (lane >> 5) + 4 * (lane & 15);
 #pragma unroll
-    for (int j = 0; j < kSubN; ++j)
+    for (int j = 0; j < N; ++j)
 #pragma unroll
       for (int q = 0; q < 8; ++q) f.v[j][q] = *reinterpret_cast<const float *>(base + 2048 * j + 64 * q);
   }
 }
 
-template <int MODE, class G, bool BKM>
-__device__ __forceinline__ void load_b_any(const char *st, int wn, BFrags<MODE> &f, const BkmLane &L) {
+template <int MODE, class G, bool BKM, int N>
+__device__ __forceinline__ void load_b_any(const char *st, int wn, BFrags<MODE, N> &f, const BkmLane &L) {
   if constexpr (BKM) load_b_km<MODE, G>(st, wn, f, L);
   else load_b<MODE, G>(st, wn, f);
 }
@@ -692,38 +690,38 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ f16x8 as_f16(bf16x8 v) { return __builtin_bit_cast(f16x8, v); }
 
 // MFMAs of row block i: acc[i][j] += A_i B_j^T over the stage's K.
-template <int MODE>
-__device__ __forceinline__ void mma_row(const AFrag<MODE> &a, const BFrags<MODE> &b, f32x16 (&acc)[kSubN]) {
+template <int MODE, int N>
+__device__ __forceinline__ void mma_row(const AFrag<MODE> &a, const BFrags<MODE, N> &b, f32x16 (&acc)[N]) {
   // (B first: the accumulator holds C^T = B A^T, lane r of it row r of C.)
   if constexpr (is_comp(MODE)) {
     // Corrections first, then hi*hi.
 #pragma unroll
-    for (int j = 0; j < kSubN; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.l[j], a.h, acc[j], 0, 0, 0);
+    for (int j = 0; j < N; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.l[j], a.h, acc[j], 0, 0, 0);
 #pragma unroll
-    for (int j = 0; j < kSubN; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], a.l, acc[j], 0, 0, 0);
+    for (int j = 0; j < N; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], a.l, acc[j], 0, 0, 0);
 #pragma unroll
-    for (int j = 0; j < kSubN; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], a.h, acc[j], 0, 0, 0);
+    for (int j = 0; j < N; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], a.h, acc[j], 0, 0, 0);
   } else if constexpr (MODE == kS8HiOnly) {
 #pragma unroll
-    for (int j = 0; j < kSubN; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], a.h, acc[j], 0, 0, 0);
+    for (int j = 0; j < N; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], a.h, acc[j], 0, 0, 0);
   } else if constexpr (MODE == kS8Pair) {
     // The same on FP16 pairs (lo*lo, 2^-24 of the product, is left out).
 #pragma unroll
-    for (int j = 0; j < kSubN; ++j)
+    for (int j = 0; j < N; ++j)
       acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.l[j]), as_f16(a.h), acc[j], 0, 0, 0);
 #pragma unroll
-    for (int j = 0; j < kSubN; ++j)
+    for (int j = 0; j < N; ++j)
       acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.h[j]), as_f16(a.l), acc[j], 0, 0, 0);
 #pragma unroll
-    for (int j = 0; j < kSubN; ++j)
+    for (int j = 0; j < N; ++j)
       acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.h[j]), as_f16(a.h), acc[j], 0, 0, 0);
   } else if constexpr (MODE == kS8F16) {
     // K 0-15, then K 16-31 of the stage.
 #pragma unroll
-    for (int j = 0; j < kSubN; ++j)
+    for (int j = 0; j < N; ++j)
       acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.h[j]), as_f16(a.h), acc[j], 0, 0, 0);
 #pragma unroll
-    for (int j = 0; j < kSubN; ++j)
+    for (int j = 0; j < N; ++j)
       acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.l[j]), as_f16(a.l), acc[j], 0, 0, 0);
   } else {
     // Lane half h supplies k = 8h + q to MFMA q (the same permutation for
@@ -731,7 +729,7 @@ __device__ __forceinline__ void mma_row(const AFrag<MODE> &a, const BFrags<MODE>
 #pragma unroll
     for (int q = 0; q < 8; ++q)
 #pragma unroll
-      for (int j = 0; j < kSubN; ++j)
+      for (int j = 0; j < N; ++j)
         acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b.v[j][q], a.v[q], acc[j], 0, 0, 0);
   }
 }
@@ -782,12 +780,12 @@ __device__ __forceinline__ AFrag<MODE> one_hot(float s, int r0) {
 // would misscale the linear term of P by up to 2^-9); FP16 the scalar's hi
 // and lo against the stage's first 16 K (rows r0 = 0 .. 15 of the block)
 // and its second 16 K (rows 16 .. 31); FP32 one product.
-template <int MODE>
-__device__ __forceinline__ void mma_one_hot(float s, int sel, const BFrags<MODE> &b, f32x16 (&acc)[kSubN]) {
+template <int MODE, int N>
+__device__ __forceinline__ void mma_one_hot(float s, int sel, const BFrags<MODE, N> &b, f32x16 (&acc)[N]) {
   if constexpr (MODE == kS8F16) {
     const AFrag<MODE> o0 = one_hot<MODE>(s, 0), o1 = one_hot<MODE>(s, 16);
 #pragma unroll
-    for (int j = 0; j < kSubN; ++j) {
+    for (int j = 0; j < N; ++j) {
       acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.h[j]), as_f16(o0.h), acc[j], 0, 0, 0);
       acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.h[j]), as_f16(o0.l), acc[j], 0, 0, 0);
       acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.l[j]), as_f16(o1.h), acc[j], 0, 0, 0);
@@ -796,7 +794,7 @@ __device__ __forceinline__ void mma_one_hot(float s, int sel, const BFrags<MODE>
   } else if constexpr (MODE == kS8HiOnly) {
     const AFrag<MODE> o = one_hot<MODE>(s, (sel & 1) * 16);
 #pragma unroll
-    for (int j = 0; j < kSubN; ++j) {
+    for (int j = 0; j < N; ++j) {
       acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], o.h, acc[j], 0, 0, 0);
       acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], o.l, acc[j], 0, 0, 0);
     }
@@ -885,7 +883,7 @@ __device__ __forceinline__ void pipe_iter(const Opnd &A, const Opnd &B, const Wa
     issue_stage<G, BKM, MODE == kS8F16 ? 2 : 1>(A, B, o, static_cast<int64_t>(kt + S) * kBK,
                                                 lds0 + (kt % S) * G::kStageBytes);
   const char *nxt = smem + ((kt + 1) % S) * G::kStageBytes;
-  if (more) load_b_any<MODE, G, BKM>(nxt, wn, bf[PAR ^ 1], bl);
+  if (more) load_b_any<MODE, G, BKM, kSubN>(nxt, wn, bf[PAR ^ 1], bl);
   // (Raising the wave's priority around its MFMAs, s_setprio 1, made the
   // Gram launches 5% faster with 256 x 128 tiles; with the current tiles it
   // made the S8 runs 0.5-1% slower, so the waves keep the default.)
@@ -929,7 +927,7 @@ __device__ __forceinline__ void gemm_tile(const Opnd &A_in, const Opnd &B_in, in
             : tile_offsets<G::kLoadsB>(B.ld, brow0, wave);
   o.b_lds = static_cast<uint32_t>(G::kOpA + wave * (G::kLoadsB - G::kLoadsA) * 1024);
   // used by the K-major B path only
-  const BkmLane bl = F16 ? bkm_lane_f16(wn) : bkm_lane(wn);
+  const BkmLane bl = F16 ? bkm_lane_f16(kSubN * wn) : bkm_lane(kSubN * wn);
   // LDS byte address of the ring plus this wave's first A chunk.
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)) + wave * G::kLoadsA * 1024;
 #pragma unroll
@@ -939,7 +937,7 @@ __device__ __forceinline__ void gemm_tile(const Opnd &A_in, const Opnd &B_in, in
   block_barrier();
   AFrag<MODE> af[kSubM];
   BFrags<MODE> bf[2];
-  load_b_any<MODE, G, BKM>(smem, wn, bf[0], bl);
+  load_b_any<MODE, G, BKM, kSubN>(smem, wn, bf[0], bl);
 #pragma unroll
   for (int i = 0; i < kSubM; ++i) load_a<MODE, G>(smem, wm, i, af[i]);
 #define SMX_PIPE(SEL, PAR, KT, STEADY) \
@@ -984,146 +982,118 @@ __device__ __forceinline__ void gemm_tile(const Opnd &A_in, const Opnd &B_in, in
   block_barrier();
 }
 
-// The same product for a 64 x 64 tile whose K is split over the block's four
-// waves (kGeoT).  Each wave keeps its whole 64 x 64 partial and loads its
-// fragments of row-major operands straight from memory, kDeep K stages
-// ahead (their 16-byte chunks are what a lane's MFMA takes, and nothing is
-// shared between waves); a K-major B goes through a wave-private LDS
-// buffer for its transposed reads.  No barrier inside the K loop.  Then the
-// partials are added through LDS in wave order.  Of a symmetric result each
-// wave then holds one of the tile's 32 x 32 blocks, block (w / 2, w % 2) in
-// acc[0][0].  Of an apply, whose row sums run over a whole tile row, waves 0
-// and 1 hold two: blocks (w, 0) and (w, 1), or, by_col, (0, w) and (1, w), in
-// acc[0][0] and acc[0][1].  (A wave per block instead of two blocks in
-// waves 0 and 1 halves what a symmetric launch's wave fetches and runs after
-// the K loop: one 512 x 512 matrix 173 -> 162 us a call.)  Bound by latency: a launch of a
-// single 768 x 768 matrix takes 48 K stages as one chain of 21 blocks in
-// 128 x 128 tiles, here 12 in 84 blocks.
-constexpr int kDeep = 4;
-template <int MODE, bool BKM>
-__device__ __forceinline__ void gemm_tile_split(const Opnd &A_in, const Opnd &B_in, int64_t K, int64_t arow0,
-                                                int64_t brow0, char *smem, bool by_col, f32x16 (&acc)[2][kSubN]) {
+// The same product for a 64 x 64 tile of four 32 x 32 waves (kGeoT), each
+// accumulator's products in gemm_tile's order.  The pipelines are
+// gemm_tile's too, with two K stages per ring slot and barrier: a wave has
+// only a block's three MFMAs per stage, too few to pass a barrier behind.
+// Wave w holds block (w / 2, w % 2) in acc[0][0].  Where the row sums of an
+// apply run over a whole tile row (`pairs`), waves 0 and 1 take two blocks
+// at the end: (w, 0) and (w, 1), or, by_col, (0, w) and (1, w), in acc[0][0]
+// and acc[0][1].  Bound by latency and, per CU, by the fragments' LDS reads
+// (16 KB per stage, 128 cycles at 128 bytes per cycle, for 96 of MFMAs).
+template <int MODE, bool ACCG, bool BKM>
+__device__ __forceinline__ void gemm_tile_quad(const Opnd &A_in, const Opnd &B_in, int64_t K, int64_t arow0,
+                                               int64_t brow0, float sel_s, char *smem, bool pairs, bool by_col,
+                                               f32x16 (&acc)[1][kSubN]) {
   using G = GeoT;
   constexpr bool F16 = MODE == kS8F16;
-  constexpr int kU = F16 ? 2 : 1;  // elements per 4-byte unit
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int lr = lane & 31, lh = lane >> 5;
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < kSubN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-  // K is a multiple of 256 (128 pairs of FP16): nk is a multiple of 4 (2).
-  const int nk = static_cast<int>(K / (kBK * kU)) / G::kWaves;
-  const int64_t k0 = static_cast<int64_t>(wave) * nk * kBK;  // 4-byte units
+  constexpr int kU = F16 ? 2 : 1, S = G::kStages;  // elements per 4-byte unit, ring slots
   const Opnd A{uniform_ptr(A_in.p), A_in.ld / kU}, B{uniform_ptr(B_in.p), B_in.ld / kU};
-  const SMX_GLOBAL char *ap = (const SMX_GLOBAL char *)A.p + 64 * k0;
-  const SMX_GLOBAL char *bp = (const SMX_GLOBAL char *)B.p + (BKM ? 4 * k0 * B.ld * kU : 64 * k0);
-  const int64_t bstep = BKM ? 4 * static_cast<int64_t>(kBK) * B.ld * kU : 64 * kBK;  // bytes of a K stage
-  // Row r of a 32-row block: its 16-row piece, its 64 bytes, chunk lh.
-  auto row_off = [&](int64_t row0, int r, int64_t ld) {
-    return static_cast<uint32_t>(((row0 >> 4) + (r >> 4)) * (ld >> 4) * 1024 + (r & 15) * 64 + 16 * lh);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wm = wave / G::kWavesN, wn = wave % G::kWavesN;
+  f32x16 c[1];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) c[0][e] = 0.f;
+  // K is a multiple of 256: np, the slots' worth of K, is at least 4.
+  const int np = static_cast<int>(K / (2 * kBK * kU));
+  WaveOffsets<G> o;
+  o.a = tile_offsets<1>(A.ld, arow0, wave);
+  o.b = BKM ? tile_offsets_km<1, F16 ? G::kKmRowH : G::kKmRow,
+                              F16 ? kKmSwzH : MODE == SMX_S8_FP32 ? kKmSwzNone : kKmSwzT>(B.ld, brow0 / kU, wave)
+            : tile_offsets<1>(B.ld, brow0, wave);
+  o.b_lds = G::kOpA;
+  const BkmLane bl = F16 ? bkm_lane_f16(wn) : bkm_lane(wn);
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)) + wave * 1024;
+  auto issue = [&](int p) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+      issue_stage<G, BKM, kU>(A, B, o, static_cast<int64_t>(2 * p + s) * kBK,
+                              lds0 + (2 * (p % S) + s) * G::kStageBytes);
   };
-  uint32_t ao[2], bo[4];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) ao[i] = row_off(arow0, 32 * i + lr, A.ld);
-  if constexpr (BKM) {
-    const auto t = tile_offsets_km<G::kLoadsB, F16 ? G::kKmRowH : G::kKmRow, F16 ? kKmSwzH : kKmSwzT>(B.ld, brow0 / kU, 0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) bo[i] = t.v[i];
-  } else {
-#pragma unroll
-    for (int j = 0; j < kSubN; ++j) bo[j] = row_off(brow0, 32 * j + sw23(lr), B.ld);
-  }
-  const BkmLane bl = F16 ? bkm_lane_f16(0) : bkm_lane(0);
-  char *const buf = smem + wave * G::kBufBytes;
-  struct Stage {
+  struct Slot {
     AFrag<MODE> a[2];
-    bf16x8 b[4];  // row-major: hi and lo of each column block; K-major: the lane's chunk of each piece
-  } st[kDeep];
-  auto chunk = [](const SMX_GLOBAL char *p) { return *reinterpret_cast<const SMX_GLOBAL bf16x8 *>(p); };
-  auto load = [&](int kt, Stage &s) {
-    const SMX_GLOBAL char *a = ap + static_cast<int64_t>(64 * kBK) * kt, *b = bp + bstep * kt;
+    BFrags<MODE, 1> b[2];
+  } fr[2];
+  auto read = [&](int p, Slot &f) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      s.a[i].h = chunk(a + ao[i]);
-      if constexpr (two_chunks<MODE>()) s.a[i].l = chunk(a + ao[i] + 32);
-    }
-    if constexpr (BKM) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) s.b[i] = chunk(b + bo[i]);
-    } else {
-#pragma unroll
-      for (int j = 0; j < kSubN; ++j) {
-        s.b[2 * j] = chunk(b + bo[j]);
-        if constexpr (two_chunks<MODE>()) s.b[2 * j + 1] = chunk(b + bo[j] + 32);
-      }
+    for (int s = 0; s < 2; ++s) {
+      const char *st = smem + (2 * (p % S) + s) * G::kStageBytes;
+      load_b_any<MODE, G, BKM, 1>(st, wn, f.b[s], bl);
+      load_a<MODE, G>(st, wm, 0, f.a[s]);
     }
   };
 #pragma unroll
-  for (int u = 0; u < kDeep; ++u)
-    if (u < nk) load(u, st[u]);
-  for (int kt = 0; kt < nk; kt += kDeep) {
-    static_for<kDeep>([&](auto u_c) {
-      constexpr int u = decltype(u_c)::value;
-      if (u >= 2 && kt + u >= nk) return;  // nk is even
-      Stage &s = st[u];
-      BFrags<MODE> bf;
-      if constexpr (BKM) {
-        char *slot = buf + (u & 1) * 4096;
+  for (int p = 0; p < S; ++p) issue(p);
+  wait_vm<4 * (S - 1)>();  // four loads per wave and slot
+  block_barrier();
+  read(0, fr[0]);
+  // The K stages of the wave's rows (one_hot): both of slot kt0 / 2, or stage
+  // kt0 of FP16.
+  const int kt0 = static_cast<int>((arow0 + 32 * wm) / (kBK * kU));
+  auto step = [&](int p, auto par_c) {
+    constexpr int par = decltype(par_c)::value;
+    const bool more = p + 1 < np;
+    // Slot p + 1 is here; up to S - 2 further ones may be in flight.
+    static_assert(S == 4, "at most two further slots");
+    if (p + 4 <= np) wait_vm<8>();
+    else if (p + 3 == np) wait_vm<4>();
+    else wait_vm<0>();
+    wait_lds();
+    block_barrier();
+    if (p + S < np) issue(p + S);
+    if (more) read(p + 1, fr[par ^ 1]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) *reinterpret_cast<bf16x8 *>(slot + i * 1024 + lane * 16) = s.b[i];
-        // (the wave's own writes: LDS keeps a wave's order)
-        asm volatile("" ::: "memory");
-        load_b_km<MODE, G>(slot, 0, bf, bl);
-      } else {
+    for (int s = 0; s < 2; ++s) {
+      mma_row<MODE, 1>(fr[par].a[s], fr[par].b[s], c);
+      if constexpr (ACCG)
+        if (F16 ? 2 * p + s == kt0 : 2 * p == kt0) mma_one_hot<MODE, 1>(sel_s, s, fr[par].b[s], c);
+    }
+  };
+  for (int p = 0; p < np; p += 2) {  // np is even
+    step(p, std::integral_constant<int, 0>{});
+    step(p + 1, std::integral_constant<int, 1>{});
+  }
+  block_barrier();
+  acc[0][0] = c[0];
+  if (BKM && pairs) {
+    // the blocks to LDS, [block][register quad][lane], and back to their wave
+    f32x4 *const part = reinterpret_cast<f32x4 *>(smem);
 #pragma unroll
-        for (int j = 0; j < kSubN; ++j) {
-          bf.h[j] = s.b[2 * j];
-          if constexpr (two_chunks<MODE>()) bf.l[j] = s.b[2 * j + 1];
+    for (int q = 0; q < 4; ++q)
+      part[(wave * 4 + q) * 64 + lane] = f32x4{c[0][4 * q], c[0][4 * q + 1], c[0][4 * q + 2], c[0][4 * q + 3]};
+    __syncthreads();
+    if (wave < 2) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int blk = by_col ? 2 * b + wave : 2 * wave + b;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4 v = part[(blk * 4 + q) * 64 + lane];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[0][b][4 * q + e] = v[e];
         }
       }
-#pragma unroll
-      for (int i = 0; i < 2; ++i) mma_row<MODE>(s.a[i], bf, acc[i]);
-      if (kt + u + kDeep < nk) load(kt + u + kDeep, s);
-    });
-  }
-  // Partials to LDS, [wave][block][register quad][lane], and the sums.
-  __syncthreads();
-  f32x4 *const part = reinterpret_cast<f32x4 *>(smem);
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < kSubN; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        part[((wave * 4 + 2 * i + j) * 4 + q) * 64 + lane] =
-            f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-  __syncthreads();
-  if (!BKM || wave < 2) {
-#pragma unroll
-    for (int b = 0; b < (BKM ? 2 : 1); ++b) {
-      const int blk = !BKM ? wave : by_col ? 2 * b + wave : 2 * wave + b;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        f32x4 v = part[(blk * 4 + q) * 64 + lane];
-#pragma unroll
-        for (int w = 1; w < G::kWaves; ++w) v += part[((w * 4 + blk) * 4 + q) * 64 + lane];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[0][b][4 * q + e] = v[e];
-      }
     }
+    __syncthreads();
   }
-  __syncthreads();
 }
 
-// One product of a tile in geometry G: gemm_tile or, for kGeoT,
-// gemm_tile_split (whose epilogue adds the square's G term from memory).
+// One product of a tile in geometry G.
 template <int MODE, class G, bool ACCG, bool BKM, bool UB = false>
 __device__ __forceinline__ void gemm_any(const Opnd &A, const Opnd &B, int64_t K, int64_t arow0, int64_t brow0,
-                                         float sel_s, char *smem, bool by_col, f32x16 (&acc)[G::kSubM][kSubN]) {
-  if constexpr (G::kSplitK) gemm_tile_split<MODE, BKM>(A, B, K, arow0, brow0, smem, by_col, acc);
+                                         float sel_s, char *smem, bool pairs, bool by_col,
+                                         f32x16 (&acc)[G::kSubM][kSubN]) {
+  if constexpr (G::kQuad) gemm_tile_quad<MODE, ACCG, BKM>(A, B, K, arow0, brow0, sel_s, smem, pairs, by_col, acc);
   else gemm_tile<MODE, G, ACCG, BKM, UB>(A, B, K, arow0, brow0, sel_s, smem, acc);
 }
 
@@ -1247,7 +1217,7 @@ s8_stage_kernel(StageArgs args) {
     // a column block of X and cycle through P's row blocks, so each X block
     // is fetched once (0.54 GB per cfg4 apply launch against 0.77 GB
     // row-major; the launch time is the same).
-    const int64_t nrow = Gm::kSplitK ? K.rp / 64 : Gm::kGeo == kGeoS ? K.tiles_s : K.tiles_m;  // row tiles
+    const int64_t nrow = Gm::kQuad ? K.rp / 64 : Gm::kGeo == kGeoS ? K.tiles_s : K.tiles_m;  // row tiles
     tn = tix / nrow;
     tm = tix % nrow;
   } else if constexpr (Gm::kGeo == kGeoM) {
@@ -1259,12 +1229,12 @@ s8_stage_kernel(StageArgs args) {
     diag = tb == tm;
   } else {
     const int64_t nt = Gm::kGeo == kGeoL ? K.tiles_m : K.tiles_s;  // tiles per row and column
-    int64_t rem = Gm::kSplitK ? tix >> 2 : tix;
+    int64_t rem = Gm::kQuad ? tix >> 2 : tix;
     tm = 0;
     while (rem >= nt - tm) { rem -= nt - tm; ++tm; }
     tn = tm + rem;
     diag = tn == tm;
-    if constexpr (Gm::kSplitK) {
+    if constexpr (Gm::kQuad) {
       tm = 2 * tm + ((tix >> 1) & 1);
       tn = 2 * tn + (tix & 1);
     }
@@ -1308,9 +1278,10 @@ s8_stage_kernel(StageArgs args) {
   // where G is not: neither the rounding of a diagonal near 1 nor the
   // cancellation of a + b G + c G^2 there reaches P.
   const bool shift = kPair && stage != 1 && !K.gs;
-  // kGeoT: the wave's two blocks below each other instead of side by side,
-  // where the row sums run down the tile's rows (a transposed parameter).
-  const bool by_col = Gm::kSplitK && PHASE == kApply && M.flip();
+  // kGeoT with row sums: waves 0 and 1 finish two blocks each, side by side
+  // or, where the sums run down the tile's rows (a transposed parameter),
+  // below each other.
+  const bool pairs = Gm::kQuad && rsum, by_col = pairs && M.flip();
   float scale = 1.f;
   float *sym_out = nullptr;  // SYM: the product's destination
   // Gram space (see the header): a segment's first Q sits in qa; Q' = P Q
@@ -1332,7 +1303,7 @@ s8_stage_kernel(StageArgs args) {
     }
     if constexpr (kPair) scale *= pow2f(-kExpP);  // P G -> T, T P -> G
     gemm_any<MODE, Gm, false, false, MODE == kS8CompMix>(Opnd{A, K.rp}, Opnd{B, K.rp}, K.rp, tm * Gm::kTileM,
-                                                         tn * kTileN, 0.f, smem, by_col, acc);
+                                                         tn * kTileN, 0.f, smem, pairs, by_col, acc);
   } else if constexpr (PHASE == kGram) {
     if (stage == 1) {
       const double f = M.cst()[kCstFro];
@@ -1342,7 +1313,7 @@ s8_stage_kernel(StageArgs args) {
     }
     // A Gram-space class takes its stage-3 Gram of X2 from x1.
     const Opnd X{K.gs && stage == 3 ? M.x1() : x_in, K.cp};
-    gemm_any<MODE, Gm, false, false>(X, X, K.cp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, by_col, acc);
+    gemm_any<MODE, Gm, false, false>(X, X, K.cp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, pairs, by_col, acc);
   } else if constexpr (PHASE == kSquare) {
     const Opnd G{M.g(), K.rp};
     // (the square kernels run at the VGPR budget, where the compiler keeps
@@ -1350,13 +1321,13 @@ s8_stage_kernel(StageArgs args) {
     constexpr bool kUB = true;
     if (stage == 1) {
       if constexpr (kPair) scale = pow2f(-2 * kExpG);
-      gemm_any<MODE, Gm, false, false, kUB>(G, G, K.rp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, by_col, acc);
+      gemm_any<MODE, Gm, false, false, kUB>(G, G, K.rp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, pairs, by_col, acc);
     } else {
       // acc = G G + (b/c) G; the epilogue forms P = c acc + a I.
       scale = kPair ? args.c * pow2f(kExpP - 2 * kExpG) : args.c;
       gemm_any<MODE, Gm, true, false, kUB>(G, G, K.rp, tm * Gm::kTileM, tn * kTileN,
                                             kPair ? (shift ? args.bh_over_c : args.b_over_c) * pow2f(kExpG)
-                                                  : args.b_over_c, smem, by_col, acc);
+                                                  : args.b_over_c, smem, pairs, by_col, acc);
     }
   } else {
     // X-space: X' = P X (stage 1: X' = P1 V / (||V|| s)).  Gram space:
@@ -1377,7 +1348,7 @@ s8_stage_kernel(StageArgs args) {
     const float *A = mid ? M.qb() : fin ? M.qa() : M.p();
     const Opnd B = gq ? Opnd{q_in, K.rp} : Opnd{mid ? M.x0() : fin ? M.x1() : x_in, K.cp};
     // B = X (or Q) rows k (K-major), columns of the tile.
-    gemm_any<MODE, Gm, false, true>(Opnd{A, K.rp}, B, K.rp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, by_col, acc);
+    gemm_any<MODE, Gm, false, true>(Opnd{A, K.rp}, B, K.rp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, pairs, by_col, acc);
   }
 
   // ------------------------------------------------------- epilogue ---
@@ -1395,13 +1366,10 @@ s8_stage_kernel(StageArgs args) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wm = wave / Gm::kWavesN, wn = wave % Gm::kWavesN;
   const int lr = lane & 31, lh = lane >> 5;
-  // The wave's blocks: kSubM x kSubN from (R0, C0); kGeoT one (kQuad), or two
-  // (waves 0, 1 of an apply).
-  constexpr bool kQuad = Gm::kSplitK && PHASE != kApply;
-  const int64_t R0 = tm * Gm::kTileM + (kQuad ? 32 * (wave >> 1)
-                                        : Gm::kSplitK ? (by_col ? 0 : 32 * wave) : wm * (32 * kSubM));
-  const int64_t C0 = tn * kTileN + (kQuad ? 32 * (wave & 1)
-                                    : Gm::kSplitK ? (by_col ? 32 * wave : 0) : wn * (32 * kSubN));
+  // The wave's blocks: kSubM x kSubN from (R0, C0); kGeoT one, or two
+  // (`pairs`: waves 0 and 1).
+  const int64_t R0 = tm * Gm::kTileM + (pairs ? (by_col ? 0 : 32 * wave) : wm * (32 * kSubM));
+  const int64_t C0 = tn * kTileN + (pairs ? (by_col ? 32 * wave : 0) : Gm::kQuad ? 32 * wn : wn * (32 * kSubN));
   const bool last = stage == 5;
   float *dst_t, *dst_m;
   int64_t ld_t, ld_m;
@@ -1448,7 +1416,7 @@ s8_stage_kernel(StageArgs args) {
   const float eye_a = !kPair ? args.a : PHASE == kGram ? -pow2f(kExpG) : (shift ? args.ah : args.a) * pow2f(kExpP);
   // the wave's staging block of a transposed output: [column][row]
   float *const U = reinterpret_cast<float *>(smem) + wave * 2 * kEpBlock;
-  float sq_local = 0.f;
+  double sq_local = 0.0;
   // The stage-5 result of the matrix step: per parameter row, partial sums
   // of Q z, (a Q)^2 and (a Q)(a z) over a strip of parameter columns (the
   // wave's 64 output columns; for a transposed parameter, 64 of its output
@@ -1456,7 +1424,7 @@ s8_stage_kernel(StageArgs args) {
   // directly stored row, the 8 of a staged transposed one) and stored for
   // the mapback (its row coefficients and graft norm), so no later pass
   // reads Q for them.
-  static_assert(PHASE != kApply || (kStripT == 32 * kSubN && (32 * kSubM) % kStripM == 0),
+  static_assert(PHASE != kApply || Gm::kQuad || (kStripT == 32 * kSubN && (32 * kSubM) % kStripM == 0),
                 "a row-sum strip is one wave's share of an apply tile");
   const int64_t prows = M.prow_pad();
   // a and z of the tile's parameter columns in LDS past the staging blocks
@@ -1620,36 +1588,6 @@ s8_stage_kernel(StageArgs args) {
       }
     }
   };
-  // kGeoT's square: b G of the lane's 16 values of row gr, columns cb +
-  // col16(e), in the scale of P (the K loop has just read them).  In place
-  // of the one-hot MFMAs, whose code is longer than a launch this short can
-  // fetch: 14.5 -> 11 us per launch of one 512 x 512 matrix.
-  auto add_bg = [&](float (&w)[16], int64_t gr, int64_t cb) {
-    const SMX_GLOBAL char *gp = (const SMX_GLOBAL char *)M.g();
-    constexpr bool F16 = MODE == kS8F16;
-    const int64_t base = (gr & ~int64_t{15}) * ((F16 ? 2 : 4) * K.rp) + ((gr & 15) << 6) + (F16 ? 32 : 64) * cb + 16 * lh;
-    const float b = kPair ? (shift ? args.bh : args.b) * pow2f(kExpP - kExpG) : args.b;
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const uint4 h = __builtin_bit_cast(uint4, *reinterpret_cast<const SMX_GLOBAL u32x4v *>(gp + base + (F16 ? 32 : 1024) * q));
-      const uint4 l = !is_split(MODE) ? make_uint4(0, 0, 0, 0)
-                          : __builtin_bit_cast(uint4, *reinterpret_cast<const SMX_GLOBAL u32x4v *>(gp + base + 1024 * q + 32));
-      const uint32_t hw[4] = {h.x, h.y, h.z, h.w}, lw[4] = {l.x, l.y, l.z, l.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float g0, g1;
-        if constexpr (kPair || F16) {
-          g0 = f16_bits_to_f32(hw[e] & 0xffff) + f16_bits_to_f32(lw[e] & 0xffff);
-          g1 = f16_bits_to_f32(hw[e] >> 16) + f16_bits_to_f32(lw[e] >> 16);
-        } else {
-          g0 = __uint_as_float(hw[e] << 16) + __uint_as_float(lw[e] << 16);
-          g1 = __uint_as_float(hw[e] & 0xffff0000u) + __uint_as_float(lw[e] & 0xffff0000u);
-        }
-        w[8 * q + 2 * e] = fmaf(b, g0, w[8 * q + 2 * e]);
-        w[8 * q + 2 * e + 1] = fmaf(b, g1, w[8 * q + 2 * e + 1]);
-      }
-    }
-  };
   // The block loop, specialised for the output form (one copy per form the
   // launch's mode can produce, so that each keeps only its own registers).
   auto epilogue = [&](auto fm_c) {
@@ -1661,22 +1599,22 @@ s8_stage_kernel(StageArgs args) {
     float rsd[3] = {0.f, 0.f, 0.f};
     // (expanded at compile time: a rolled block loop indexes acc at run
     // time, which moves every accumulator of the kernel to scratch memory)
-    static_for<kQuad ? 1 : Gm::kSplitK ? 2 : kSubM * kSubN>([&](auto blk_c) {
+    static_for<Gm::kQuad && PHASE != kApply ? 1 : kSubM * kSubN>([&](auto blk_c) {
       constexpr int blk = decltype(blk_c)::value, i = blk / kSubN, j = blk % kSubN;
-      const int64_t rb = R0 + (Gm::kSplitK && by_col ? blk : i) * 32;
-      const int64_t gr = rb + lr, cb = C0 + (Gm::kSplitK && by_col ? 0 : j) * 32;
-      float w[16];
+      if (Gm::kQuad && blk == 1 && !pairs) return;
+      const int64_t rb = R0 + (Gm::kQuad && by_col ? blk : i) * 32;
+      const int64_t gr = rb + lr, cb = C0 + (Gm::kQuad && by_col ? 0 : j) * 32;
+      float w[16], sq = 0.f;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         w[e] = acc[i][j][e] * scale;
         // stage 1's FP32 G2: its squared entries feed the Schatten scale
-        if constexpr (PHASE == kSquare && (FM == kFormF32 || FM == kFormAny)) sq_local = fmaf(w[e], w[e], sq_local);
-      }
-      if constexpr (PHASE == kSquare && Gm::kSplitK)
-        if (stage != 1) add_bg(w, gr, cb);
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
+        if constexpr (PHASE == kSquare && (FM == kFormF32 || FM == kFormAny)) sq = fmaf(w[e], w[e], sq);
         if (do_m) U[col16(e) * kEpStride + lr] = w[e];
+      }
+      // (FP32 within a block, FP64 over blocks: the sum, to FP64's rounding,
+      // of every geometry)
+      if constexpr (PHASE == kSquare && (FM == kFormF32 || FM == kFormAny)) sq_local += static_cast<double>(sq);
       if (do_t) {
         if (eye) {
           // the diagonal's column in the lane's col16 order, if it has one
@@ -1719,9 +1657,9 @@ s8_stage_kernel(StageArgs args) {
         for (int q = 0; q < 4; ++q) {
           const int row = er + 8 * q;
           const int64_t gm = cb + row;
-          float(&r)[3] = rs[Gm::kSplitK ? 0 : j][q];
+          float(&r)[3] = rs[Gm::kQuad ? 0 : j][q];
           put_row(fm_c, U, row, gm, rb, dst_m, ld_m, tiled_m, r, rs_on);
-          if (rs_on && (Gm::kSplitK ? blk == 1 : (i + 1) % (kStripM / 32) == 0))
+          if (rs_on && (Gm::kQuad ? blk == 1 : (i + 1) % (kStripM / 32) == 0))
             emit(gm, (rb + 32 - kStripM) / kStripM, r);
         }
       }
@@ -1732,7 +1670,7 @@ s8_stage_kernel(StageArgs args) {
   };
   // Only the forms this launch kind can produce are compiled (the host
   // checks every launch's forms against the same table, form_compiled).
-  const bool owns = !Gm::kSplitK || kQuad || wave < 2;  // the wave holds blocks of the tile
+  const bool owns = !pairs || wave < 2;  // the wave holds blocks of the tile
   constexpr bool kPlanes = form_compiled(MODE, PHASE, kFormPlanes);
   constexpr bool kF16 = form_compiled(MODE, PHASE, kFormF16);
   constexpr bool kF32 = form_compiled(MODE, PHASE, kFormF32);
@@ -1749,7 +1687,7 @@ s8_stage_kernel(StageArgs args) {
   }
   if constexpr (PHASE == kSquare) {
     if (stage == 1) {
-      const double s = block_sum(static_cast<double>(sq_local), dscratch);
+      const double s = block_sum(sq_local, dscratch);
       if (threadIdx.x == 0) M.sch()[tix] = (diag ? 1.0 : 2.0) * s;
     }
   }
@@ -2045,8 +1983,7 @@ static int pick_geo(const S8Layout &Lay, int phase, const std::vector<Seg> &segs
     const int64_t cnt = sg.hi - sg.lo;
     for (int g = 0; g < 4; ++g) tiles[g] += cnt * phase_tiles(k, phase, g, sg.op);
   }
-  if (g_tile_policy == 0 && !Lay.keep_bits && Lay.mode != SMX_S8_FP32 && tiles[kGeoT] <= 3 * cus)
-    return kGeoT;
+  if (g_tile_policy == 0 && tiles[kGeoT] <= 3 * cus) return kGeoT;
   if (g_tile_policy == 0 && 2 * tiles[kGeoL] >= 3 * cus) return kGeoL;
   const double r_m = static_cast<double>(ceil_div(tiles[kGeoM], 2 * cus));
   const double r_s = static_cast<double>(ceil_div(tiles[kGeoS], 3 * cus));
@@ -2057,8 +1994,7 @@ static int pick_geo(const S8Layout &Lay, int phase, const std::vector<Seg> &segs
 template <int MODE, int PHASE>
 static void launch_stage(int geo, int32_t blocks, const StageArgs &a, hipStream_t st) {
   if (geo == kGeoT) {
-    if constexpr (MODE != SMX_S8_FP32)
-      hipLaunchKernelGGL((s8_stage_kernel<MODE, PHASE, 64, 64>), dim3(blocks), dim3(GeoT::kThreads), 0, st, a);
+    hipLaunchKernelGGL((s8_stage_kernel<MODE, PHASE, 64, 64>), dim3(blocks), dim3(GeoT::kThreads), 0, st, a);
     return;
   }
   if (geo == kGeoS) {
