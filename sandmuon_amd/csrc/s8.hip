@@ -774,8 +774,12 @@ __device__ __forceinline__ AFrag<MODE> one_hot(float s, int r0) {
   return f;
 }
 
-// acc[i] += s G over the rows of the one-hot window stage: the split
-// operands' three products of the (hi, lo) scalar and B planes; a plain BF16
+// acc[i] += s G over the rows of the one-hot window stage.  Compensated: s in
+// three BF16 parts, both of the first with both B planes and the third with
+// hi, smallest first (the same s misscales a whole matrix: as hi + lo, with
+// lo * lo left out, the map of 768 x 768 matrices was 1.2e-4 off FP64, so
+// 3.5e-5; two more MFMAs in 2 of a 768-deep product's 48 K stages).  FP16
+// pairs: three products of the (hi, lo) scalar and B planes; a plain BF16
 // stage the scalar's hi and lo against B's hi plane (a BF16 scalar alone
 // would misscale the linear term of P by up to 2^-9); FP16 the scalar's hi
 // and lo against the stage's first 16 K (rows r0 = 0 .. 15 of the block)
@@ -798,6 +802,16 @@ __device__ __forceinline__ void mma_one_hot(float s, int sel, const BFrags<MODE,
       acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], o.h, acc[j], 0, 0, 0);
       acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], o.l, acc[j], 0, 0, 0);
     }
+  } else if constexpr (is_comp(MODE)) {
+    const AFrag<MODE> o = one_hot<MODE>(s, (sel & 1) * 16);
+    // (the third part: s less its hi and lo, exact in FP32)
+    const float sh = static_cast<float>(static_cast<__bf16>(s)), sl = static_cast<float>(static_cast<__bf16>(s - sh));
+    const AFrag<MODE> r = one_hot<MODE>((s - sh) - sl, (sel & 1) * 16);
+#pragma unroll
+    for (int j = 0; j < N; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.l[j], o.l, acc[j], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < N; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], r.h, acc[j], 0, 0, 0);
+    mma_row<MODE>(o, b, acc);
   } else {
     mma_row<MODE>(one_hot<MODE>(s, (sel & 1) * 16), b, acc);
   }
@@ -1919,7 +1933,7 @@ static std::vector<Seg> launch_segments(const S8Layout &Lay, const SlotSet &set,
 
 // MFMA FLOPs of one launch in MFMA mode `mode`: computed tiles x 2 * TM *
 // TN * K (x3 compensated), plus the square phase's one-hot MFMAs: per wave
-// and 32x32 column tile, 2 kSubM window stages of 3 (compensated), 2
+// and 32x32 column tile, 2 kSubM window stages of 5 (compensated), 2
 // (plain BF16: the scalar's hi and lo) or 1 (FP32) 16-deep products, or
 // kSubM stages of 4 (FP16: hi and lo over each 16 K of a 32-deep stage).
 static double launch_flops(int mode, int phase, int stage, int geo, const S8Layout &Lay,
@@ -1927,13 +1941,13 @@ static double launch_flops(int mode, int phase, int stage, int geo, const S8Layo
   if (phase == kPoly1) return 0.0;
   const double prod = is_comp(mode) ? 3.0 : 1.0;
   const int tm = geo == kGeoT ? 64 : geo == kGeoS ? 128 : 256, tn = geo == kGeoT ? 64 : geo == kGeoL ? 256 : 128;
-  // waves that issue the one-hot MFMAs of a tile, 32 sub_m rows each (kGeoT,
-  // which adds that term from memory, counts as many)
+  // waves that issue the one-hot MFMAs of a tile, 32 sub_m rows and kSubN
+  // column tiles each (kGeoT: of four waves with half of each)
   const int waves = geo == kGeoT ? 1 : geo == kGeoL ? 8 : 4;
   const int sub_m = geo == kGeoT ? 2 : tm / 64;
   // (kS8Pair counts one product per element pair, as the FP32 MFMAs whose
   // place it takes issue; it is carried out as three FP16 ones.)
-  const double onehot = is_comp(mode) ? 6.0 * sub_m : mode == kS8HiOnly ? 4.0 * sub_m
+  const double onehot = is_comp(mode) ? 10.0 * sub_m : mode == kS8HiOnly ? 4.0 * sub_m
                         : mode == kS8F16 ? 4.0 * sub_m : 2.0 * sub_m;
   double f = 0.0;
   for (const Seg &sg : segs) {

@@ -49,6 +49,20 @@ def test_s8_cfg2_inputs(device, mode, shape):
     assert max(errs) <= TOL[mode]
 
 
+# 64 x 64, 128 x 128, 256 x 128 and 256 x 256 tiles of the square
+@pytest.mark.parametrize("batch,size", [(2, 512), (24, 768), (74, 768), (8, 2048)])
+def test_s8_comp_error_against_fp64(device, batch, size):
+    # Gaussian matrices with row and column scales a decade each way: 3.5e-5
+    # off FP64 whatever the geometry (1.2e-4 where the square's scalar b / c
+    # has two BF16 parts).
+    g = torch.Generator(device=device).manual_seed(size + batch)
+    scale = lambda *s: torch.exp(torch.empty(*s, device=device).uniform_(-2.3, 2.3, generator=g))
+    x = torch.randn(batch, size, size, generator=g, device=device) * scale(batch, size, 1) * scale(batch, 1, size)
+    out = _s8_fp32(x, mode="comp_bf16")
+    for i in (0, batch - 1):
+        assert max(per_matrix_rel(out[i:i + 1], O.s8(x[i:i + 1].double().cpu()))) <= 6e-5
+
+
 def steep_batch(batch, rows, cols, p, seed):
     """Matrices whose singular values decay as i^-p (the shape of a low-rank
     training gradient) with random singular vectors."""
@@ -128,11 +142,12 @@ def prod(mode, stage, gs=False):
 def one_hot_flops(mode, stage, tiles, tm, waves, gs=False):
     """The square's one-hot (b/c) G MFMAs (32 x 32 x 16 each) per launch
     matrix: per tile and wave, over its 2 column tiles, 2 tm/64 K stages of
-    3 (compensated) or 1 (FP32) products, or tm/64 FP16 stages of 4 (the
-    scalar's hi and lo against both 16-deep halves)."""
-    per = {"comp_bf16": 2 * (tm // 64) * 3, "fp32": 2 * (tm // 64)}.get(mode, (tm // 64) * 4)
+    5 (compensated: the scalar's three BF16 parts) or 1 (FP32) products, or
+    tm/64 FP16 stages of 4 (the scalar's hi and lo against both 16-deep
+    halves)."""
+    per = {"comp_bf16": 2 * (tm // 64) * 5, "fp32": 2 * (tm // 64)}.get(mode, (tm // 64) * 4)
     if mode == "mixed" and (stage <= 2 or gs):
-        per = 2 * (tm // 64) * 3
+        per = 2 * (tm // 64) * 5
     return tiles * waves * per * 2 * 2 * 32 * 32 * 16
 
 
