@@ -396,6 +396,9 @@ int smx_s8(const float *x, float *out, int64_t batch, int64_t rows,
 int smx_s8_timing(int32_t enable);
 int32_t smx_s8_timing_read(float *ms, int32_t *phase, double *flops,
                            int32_t capacity);
+/* The output tile (rows x cols) of each recorded launch, in the same order;
+ * 0 x 0 for the records that are no tiled launch (phases 3, 4 and 6). */
+int32_t smx_s8_timing_tiles(int32_t *rows, int32_t *cols, int32_t capacity);
 
 /* ------------------------------------------------------------------ *
  * Module-level helpers (sandmuon/optimizer.py:19-66), in the dtype of their
@@ -479,11 +482,14 @@ int smx_mfma_peak(int32_t dtype, int32_t blocks, int64_t iters,
 
 /* ------------------------------------------------------------------ *
  * Tile geometry of the S8 GEMM launches (no counterpart in the reference;
- * a test and measurement aid).  0 (the default): each launch picks its
- * tiles from its size (256 x 256 blocks of 8 waves for launches that fill
- * the device with a long K loop, else 256 x 128 or 128 x 128 blocks of 4
- * waves); 1: 256 x 256 tiles for every launch; 2: never 256 x 256.  The
- * results agree to rounding across geometries.  Process-wide, read at each
+ * a test and measurement aid).  0 (the default): matrices that fit one
+ * block's LDS run whole in it, and each launch over the others picks its
+ * tiles from its size (64 x 64 tiles where they leave CUs idle, 256 x 256
+ * tiles of 8 waves for launches that fill the device with a long K loop, else
+ * 256 x 128 or 128 x 128 tiles of 4 waves); 1: 256 x 256 tiles for every
+ * launch; 2: 256 x 128 or 128 x 128 tiles for every launch (1 and 2: small
+ * matrices too).  64 x 64 and 128 x 128 tiles give the same bits, the others
+ * agree to rounding.  Process-wide, read at each
  * S8 launch; returns the previous value, or SMX_EINVAL for a value outside
  * [0, 2] (then nothing changes).
  * ------------------------------------------------------------------ */

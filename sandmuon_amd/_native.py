@@ -130,6 +130,7 @@ SIGNATURES = {
     "smx_s8_tile_geometry": (c_int, [c_int32]),
     "smx_mfma_peak": (c_int, [c_int32, c_int32, c_int64, c_void_p, c_void_p, c_void_p]),
     "smx_s8_timing": (c_int, [c_int32]),
+    "smx_s8_timing_tiles": (c_int32, [ctypes.POINTER(c_int32), ctypes.POINTER(c_int32), c_int32]),
     "smx_s8_timing_read": (c_int32, [ctypes.POINTER(ctypes.c_float), ctypes.POINTER(c_int32),
                                      ctypes.POINTER(c_double), c_int32]),
 }
@@ -466,6 +467,14 @@ def s8_timing_read(capacity: int = 4096):
     n = lib().smx_s8_timing_read(ms, ph, fl, capacity)
     _check(min(n, 0), "smx_s8_timing_read")
     return [(ms[i], S8_PHASES[ph[i]], fl[i]) for i in range(n)]
+
+
+def s8_timing_tiles(capacity: int = 4096):
+    """(phase name, tile rows, tile columns) of the recorded GEMM launches."""
+    rows, cols = (c_int32 * capacity)(), (c_int32 * capacity)()
+    n = lib().smx_s8_timing_tiles(rows, cols, capacity)
+    _check(min(n, 0), "smx_s8_timing_tiles")
+    return [(p, rows[i], cols[i]) for i, (_, p, _) in enumerate(s8_timing_read(n)) if rows[i]] if n else []
 
 
 def s8(x: torch.Tensor, out: torch.Tensor, mode: int) -> None:

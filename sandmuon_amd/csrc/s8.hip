@@ -1835,7 +1835,7 @@ __global__ void __launch_bounds__(256) s8_pair0_kernel(StageArgs args) {
 struct LaunchTiming {
   int level = 0;  // 0 off, 1 every launch and every run, 2 runs only
   std::vector<hipEvent_t> start, stop;
-  std::vector<int32_t> phase;
+  std::vector<int32_t> phase, geo;  // geo: TileGeo of a GEMM launch, else -1
   std::vector<double> flops;
   size_t used = 0;
 };
@@ -1854,6 +1854,7 @@ static int timing_begin(hipStream_t st, int &slot, bool whole_run) {
     g_timing.start.push_back(a);
     g_timing.stop.push_back(b);
     g_timing.phase.push_back(0);
+    g_timing.geo.push_back(-1);
     g_timing.flops.push_back(0.0);
   }
   slot = static_cast<int>(g_timing.used++);
@@ -1863,11 +1864,12 @@ static int timing_begin(hipStream_t st, int &slot, bool whole_run) {
   return SMX_OK;
 }
 
-static int timing_end(int slot, hipStream_t st, int phase, double flops) {
+static int timing_end(int slot, hipStream_t st, int phase, double flops, int geo = -1) {
   if (slot < 0) return SMX_OK;
   if (hipEventRecord(g_timing.stop[slot], st) != hipSuccess)
     return fail(SMX_ELAUNCH, "s8 timing: hipEventRecord failed");
   g_timing.phase[slot] = phase;
+  g_timing.geo[slot] = geo;
   g_timing.flops[slot] = flops;
   return SMX_OK;
 }
@@ -1970,14 +1972,19 @@ static int64_t device_cus() {
   return cus[dev];
 }
 
-// The tile geometry of one launch over `segs`.  64 x 64 tiles with K split
-// over the block's waves (kGeoT) up to three per CU: such a launch takes
-// the time of one tile's chain, a quarter as long there.  (One 512 x 512
-// matrix 261 -> 183 us, two of 768 x 3072 in an MLP step 1446 -> 1310 us,
-// four of 640 x 1280 in a direction 635 -> 520; with up to six tiles per
-// CU, half of 36 768 x 768 matrices 1235 -> 1620 us.)  It adds in another
-// order than the other geometries, so not where those bits are kept
-// (S8Layout::keep_bits), nor on FP32 MFMAs.  256 x 256 tiles when
+// The tile geometry of one launch over `segs`; `every` holds its segments in
+// all launch chains of the run, which run beside it.  64 x 64 tiles (kGeoT)
+// while the launch's are at most two per CU, the blocks that a CU holds, and
+// those of all chains at most 3.2 per CU: the launch then takes the time of
+// one tile's chain, a quarter as long as a 128 x 128 tile's.  Beyond that
+// the larger tile's fewer operand bytes per MFMA win.  A call in us, on 128 x
+// 128 tiles and on 64 x 64: one 512 x 512 matrix 255 -> 158, one 768 x 3072
+// 462 -> 278, three 1024 x 1024 (1.7 tiles per CU) 406 -> 343; in two chains,
+// eight 768 x 768 (2.6 per CU in all) 409 -> 372, nine 768 x 3072 (3.0) 807
+// -> 710, twenty 512 x 512 (3.1) 348 -> 334, but six 1024 x 1024 (3.4) 529 ->
+// 561 and twelve 768 x 768 (3.9) 484 -> 492; with up to three tiles per CU
+// and launch, one 2048 x 2048 (2.1) 726 -> 754 and eighteen 768 x 768 (3.0
+// per chain) 605 -> 688.  256 x 256 tiles when
 // the launch has at least 1.5 of them per CU: those blocks move a third
 // fewer operand bytes per MFMA (cfg5 S8 7% faster).  With fewer, each CU
 // holds one or two blocks of the launch and nothing of it to overlap a
@@ -1988,16 +1995,17 @@ static int64_t device_cus() {
 // (three per CU, a round counted 0.9 of one of two 256 x 128 blocks per
 // CU), else 256 x 128 (the cfg4 applies take 128 x 128 tiles: S8 runs 2%
 // shorter than with 256 x 128).
-static int pick_geo(const S8Layout &Lay, int phase, const std::vector<Seg> &segs) {
+static int pick_geo(const S8Layout &Lay, int phase, const std::vector<Seg> &segs, const std::vector<Seg> &every) {
   if (g_tile_policy == 1) return kGeoL;
   const int64_t cus = device_cus();
-  int64_t tiles[4] = {0, 0, 0, 0};
+  int64_t tiles[4] = {0, 0, 0, 0}, all_t = 0;
   for (const Seg &sg : segs) {
     const S8Class &k = Lay.cls[sg.cls];
     const int64_t cnt = sg.hi - sg.lo;
     for (int g = 0; g < 4; ++g) tiles[g] += cnt * phase_tiles(k, phase, g, sg.op);
   }
-  if (g_tile_policy == 0 && tiles[kGeoT] <= 3 * cus) return kGeoT;
+  for (const Seg &sg : every) all_t += (sg.hi - sg.lo) * phase_tiles(Lay.cls[sg.cls], phase, kGeoT, sg.op);
+  if (g_tile_policy == 0 && tiles[kGeoT] <= 2 * cus && 10 * all_t <= 32 * cus) return kGeoT;
   if (g_tile_policy == 0 && 2 * tiles[kGeoL] >= 3 * cus) return kGeoL;
   const double r_m = static_cast<double>(ceil_div(tiles[kGeoM], 2 * cus));
   const double r_s = static_cast<double>(ceil_div(tiles[kGeoS], 3 * cus));
@@ -2026,9 +2034,10 @@ static void launch_stage(int geo, int32_t blocks, const StageArgs &a, hipStream_
 // run in different MFMA modes (SMX_S8_MIXED at stages 3-5: an X-space
 // class in FP16, a Gram-space class compensated) go to one launch per
 // mode.
+// `run`: the matrices of all chains.
 template <int PHASE>
-static int launch_phase(const S8Layout &Lay, const SlotSet &set, int stage, int sq_geo, hipStream_t st, double &flops,
-                        const std::vector<int> &ops = {}) {
+static int launch_phase(const S8Layout &Lay, const SlotSet &set, const SlotSet &run, int stage, int sq_geo,
+                        hipStream_t st, double &flops, const std::vector<int> &ops = {}) {
   const std::vector<Seg> all = launch_segments(Lay, set, PHASE, stage, ops);
   std::vector<int> modes;
   for (const Seg &sg : all) {
@@ -2036,9 +2045,13 @@ static int launch_phase(const S8Layout &Lay, const SlotSet &set, int stage, int 
     if (std::find(modes.begin(), modes.end(), m) == modes.end()) modes.push_back(m);
   }
   for (const int mode : modes) {
-    std::vector<Seg> segs;
-    for (const Seg &sg : all)
-      if (seg_mode(Lay, PHASE, stage, sg) == mode) segs.push_back(sg);
+    auto of_mode = [&](const std::vector<Seg> &from) {
+      std::vector<Seg> to;
+      for (const Seg &sg : from)
+        if (seg_mode(Lay, PHASE, stage, sg) == mode) to.push_back(sg);
+      return to;
+    };
+    const std::vector<Seg> segs = of_mode(all);
     StageArgs a{};
     a.L = Lay;
     a.stage = stage;
@@ -2058,7 +2071,8 @@ static int launch_phase(const S8Layout &Lay, const SlotSet &set, int stage, int 
         if (!form_compiled(mode, PHASE, out_form(Lay.mode, g_comp_mask, PHASE, stage, sg.op, Lay.cls[sg.cls].gs != 0)))
           return fail(SMX_EINVAL, "s8: no epilogue for the output form of this product");
     const int geo =
-        PHASE == kSquare ? sq_geo : PHASE == kPoly1 ? kGeoM : pick_geo(Lay, PHASE, segs);
+        PHASE == kSquare ? sq_geo : PHASE == kPoly1 ? kGeoM
+                         : pick_geo(Lay, PHASE, segs, of_mode(launch_segments(Lay, run, PHASE, stage, ops)));
     int32_t off = 0;
     a.n_seg = 0;
     for (const Seg &sg : segs) {
@@ -2099,7 +2113,7 @@ static int launch_phase(const S8Layout &Lay, const SlotSet &set, int stage, int 
     if (rc) return rc;
     const double f = launch_flops(mode, PHASE, stage, geo, Lay, segs);
     flops += f;
-    rc = timing_end(slot, st, PHASE, f);
+    rc = timing_end(slot, st, PHASE, f, PHASE == kPoly1 ? -1 : geo);
     if (rc) return rc;
   }
   return SMX_OK;
@@ -2109,25 +2123,27 @@ static int launch_phase(const S8Layout &Lay, const SlotSet &set, int stage, int 
 // phase; Gram-space classes add their two SYM products before the apply
 // launch at stages 1, 3 and 4, and an apply of their own after it at stages
 // 2 (X2) and 5 (X5).
-static int run_s8_set_stage(const S8Layout &Lay, const SlotSet &set, int stage, hipStream_t st, double &flops) {
+static int run_s8_set_stage(const S8Layout &Lay, const SlotSet &set, const SlotSet &run, int stage, hipStream_t st,
+                            double &flops) {
   auto cnt = [&](int i) { return static_cast<int64_t>(set.hi[i] - set.lo[i]); };
   // The square covers every matrix of the set at every stage, so its
   // geometry (and the stage-1 Schatten partials) is the same for the run.
-  const int sq_geo = pick_geo(Lay, kSquare, launch_segments(Lay, set, kSquare, stage, {}));
+  const int sq_geo = pick_geo(Lay, kSquare, launch_segments(Lay, set, kSquare, stage, {}),
+                              launch_segments(Lay, run, kSquare, stage, {}));
   bool any_gs = false;
   for (int i = 0; i < Lay.n_classes; ++i) any_gs = any_gs || (Lay.cls[i].gs && cnt(i) > 0);
   int rc = SMX_OK;
   {
-    rc = launch_phase<kGram>(Lay, set, stage, sq_geo, st, flops);
-    if (!rc) rc = launch_phase<kSquare>(Lay, set, stage, sq_geo, st, flops);
-    if (!rc && stage == 1) rc = launch_phase<kPoly1>(Lay, set, stage, sq_geo, st, flops);
+    rc = launch_phase<kGram>(Lay, set, run, stage, sq_geo, st, flops);
+    if (!rc) rc = launch_phase<kSquare>(Lay, set, run, stage, sq_geo, st, flops);
+    if (!rc && stage == 1) rc = launch_phase<kPoly1>(Lay, set, run, stage, sq_geo, st, flops);
     if (!rc && any_gs && gs_sym(stage)) {
-      rc = launch_phase<kSym>(Lay, set, stage, sq_geo, st, flops, {kOpPG});
-      if (!rc) rc = launch_phase<kSym>(Lay, set, stage, sq_geo, st, flops, {kOpTP});
+      rc = launch_phase<kSym>(Lay, set, run, stage, sq_geo, st, flops, {kOpPG});
+      if (!rc) rc = launch_phase<kSym>(Lay, set, run, stage, sq_geo, st, flops, {kOpTP});
     }
-    if (!rc) rc = launch_phase<kApply>(Lay, set, stage, sq_geo, st, flops, {kOpApplyX, kOpApplyQ});
+    if (!rc) rc = launch_phase<kApply>(Lay, set, run, stage, sq_geo, st, flops, {kOpApplyX, kOpApplyQ});
     if (!rc && any_gs && (stage == 2 || stage == 5))
-      rc = launch_phase<kApply>(Lay, set, stage, sq_geo, st, flops, {stage == 2 ? kOpApplyMid : kOpApplyFinal});
+      rc = launch_phase<kApply>(Lay, set, run, stage, sq_geo, st, flops, {stage == 2 ? kOpApplyMid : kOpApplyFinal});
   }
   return rc;
 }
@@ -2220,10 +2236,11 @@ int run_s8_stages(const S8Layout &layout, hipStream_t st) {
   };
   std::stable_sort(order.begin(), order.end(),
                    [&](int x, int y) { return work(x, Lay.cls[x].count) > work(y, Lay.cls[y].count); });
-  SlotSet set[kChains];
+  SlotSet set[kChains], run;
   double load[kChains] = {};
   for (int i : order) {
     const int c = Lay.cls[i].count;
+    run.hi[i] = c;
     if (c >= kSplitCount) {
       int lo = 0;
       for (int t = 0; t < kChains; ++t) {
@@ -2258,7 +2275,7 @@ int run_s8_stages(const S8Layout &layout, hipStream_t st) {
     return e ? e : timing_end(rec, st, kSmall, f);
   };
   if (chains <= 1) {
-    for (int stage = 1; stage <= 5 && !rc && chains; ++stage) rc = run_s8_set_stage(Lay, set[0], stage, st, flops);
+    for (int stage = 1; stage <= 5 && !rc && chains; ++stage) rc = run_s8_set_stage(Lay, set[0], run, stage, st, flops);
     if (!rc) rc = run_small();
   } else {
     // Only enqueues happen under the lock.
@@ -2273,7 +2290,7 @@ int run_s8_stages(const S8Layout &layout, hipStream_t st) {
     // starts while the host is still enqueuing the others.
     for (int stage = 1; stage <= 5 && !rc; ++stage)
       for (int t = chains - 1; t >= 0 && !rc; --t)
-        if (!set[t].empty()) rc = run_s8_set_stage(Lay, set[t], stage, t ? f->aux[t - 1] : st, flops);
+        if (!set[t].empty()) rc = run_s8_set_stage(Lay, set[t], run, stage, t ? f->aux[t - 1] : st, flops);
     if (!rc) rc = run_small();  // beside the second chain
     // Join even after a failed launch, so the caller's stream never runs
     // ahead of work already on the other streams.
@@ -2401,6 +2418,17 @@ extern "C" int smx_s8_timing(int32_t enable) {
   g_timing.level = enable;
   if (enable) g_timing.used = 0;
   return SMX_OK;
+}
+
+extern "C" int32_t smx_s8_timing_tiles(int32_t *rows, int32_t *cols, int32_t capacity) {
+  SMX_REQUIRE(capacity >= 0, SMX_EINVAL, "s8 timing: negative capacity");
+  const int32_t n = static_cast<int32_t>(std::min<size_t>(g_timing.used, static_cast<size_t>(capacity)));
+  for (int32_t i = 0; i < n; ++i) {
+    const int g = g_timing.geo[i];
+    if (rows) rows[i] = g < 0 ? 0 : g == smx::kGeoT ? 64 : g == smx::kGeoS ? 128 : 256;
+    if (cols) cols[i] = g < 0 ? 0 : g == smx::kGeoT ? 64 : g == smx::kGeoL ? 256 : 128;
+  }
+  return n;
 }
 
 extern "C" int32_t smx_s8_timing_read(float *ms, int32_t *phase, double *flops, int32_t capacity) {

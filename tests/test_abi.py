@@ -238,3 +238,5 @@ def test_s8_timing_recorder_without_launches():
     assert lib.smx_s8_timing(0) == 0
     assert lib.smx_s8_timing(3) == -1
     assert lib.smx_s8_timing_read(None, None, None, -1) == -1
+    assert _native.s8_timing_tiles(16) == []
+    assert lib.smx_s8_timing_tiles(None, None, -1) == -1

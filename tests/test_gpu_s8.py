@@ -155,13 +155,14 @@ def one_hot_flops(mode, stage, tiles, tm, waves, gs=False):
 @pytest.mark.parametrize("mode", ["fp32", "comp_bf16", "mixed"])
 def test_s8_launch_timing_records_every_phase_x_space(device, mode):
     # oriented 300 x 500 padded to 512 x 512 (cp == rp): the stages run on
-    # the iterate.  The apply computes 2 x 4 tiles of 256 x 128, the Gram
-    # and the square the 10 upper-triangle 128 x 128 tiles of their 512 x 512
-    # results (three matrices take fewer rounds of the CUs' block slots in
-    # the smaller geometry); the square of stages 2-5 adds the one-hot MFMAs.
+    # the iterate, three matrices on 64 x 64 tiles.  The apply computes 8 x 8
+    # of them, the Gram and the square the quadrants of the 10 upper-triangle
+    # 128 x 128 tiles of their 512 x 512 results; the square of stages 2-5
+    # adds the one-hot MFMAs.
     x = torch.randn(3, 300, 500, device=device)
     _, phases, fl = _timed_s8(x, mode)
     assert phases == ["gram", "square", "poly1", "apply"] + ["gram", "square", "apply"] * 4
+    assert _native.s8_timing_tiles() == [(p, 64, 64) for p in phases if p != "poly1"]
     want = []
     for stage in range(1, 6):
         f = prod(mode, stage)
@@ -176,16 +177,16 @@ def test_s8_launch_timing_records_every_phase_x_space(device, mode):
 def test_s8_launch_timing_records_every_phase_gram_space(device, mode):
     # oriented 300 x 520 padded to 512 x 768 (cp > rp): Gram space, in two
     # segments.  Grams of X0 (stage 1) and X2 (stage 3), K = 768; applies of
-    # Q2 to X0 and of Q5 to X2 over 2 x 6 tiles; symmetric r x r products
-    # T = P G and G = T P (stages 1, 3, 4) and the Grams on the 10
-    # upper-triangle 128 x 128 tiles (three matrices take fewer rounds of
-    # the CUs' block slots in the smaller geometry) and full products
-    # Q' = P Q (stages 2, 4, 5) over 2 x 4 apply tiles, all with K = 512.
+    # Q2 to X0 and of Q5 to X2 over 8 x 12 tiles of 64 x 64; symmetric r x r
+    # products T = P G and G = T P (stages 1, 3, 4) and the Grams on the
+    # quadrants of the 10 upper-triangle 128 x 128 tiles and full products
+    # Q' = P Q (stages 2, 4, 5) over 8 x 8 tiles, all with K = 512.
     x = torch.randn(3, 300, 520, device=device)
     out, phases, fl = _timed_s8(x, mode)
     assert phases == (["gram", "square", "poly1", "sym", "sym"] + ["square", "apply", "apply"]
                       + ["gram", "square", "sym", "sym"] + ["square", "sym", "sym", "apply"]
                       + ["square", "apply", "apply"])
+    assert _native.s8_timing_tiles() == [(p, 64, 64) for p in phases if p != "poly1"]
     gram = lambda k: 3 * 10 * 2 * 128 * 128 * 768 * prod(mode, k, gs=True)
     sym = lambda k: 3 * 10 * 2 * 128 * 128 * 512 * prod(mode, k, gs=True)
     square = lambda k: sym(k) + (0 if k == 1 else 3 * one_hot_flops(mode, k, 10, 128, 4, gs=True))
@@ -261,17 +262,22 @@ def test_s8_launch_timing_256x256_tiles(device, mode):
     assert max(per_matrix_rel(out, O.s8(x.cpu()))) <= TOL[mode]
 
 
-# (tile rows, tile columns, waves) of each geometry
-GEOMETRY = {"128x128": (128, 128, 4), "256x128": (256, 128, 4), "256x256": (256, 256, 8)}
+# (tile rows, tile columns, waves of tile rows / 2 by 64 outputs) of each
+# geometry (64 x 64 tiles have four waves of half that)
+GEOMETRY = {"64x64": (64, 64, 2), "128x128": (128, 128, 4), "256x128": (256, 128, 4), "256x256": (256, 256, 8)}
 
 
-def expected_square_geometry(n, size, cus):
-    """The square's geometry for a launch over n matrices of size x size:
-    256 x 256 tiles when there are at least 1.5 of them per CU, else 128 x 128
+def expected_square_geometry(n, total, size, cus):
+    """The square's geometry for a launch over n matrices of size x size, of
+    `total` in all launch chains: 64 x 64 tiles when the launch has at most two
+    of them per CU and all chains at most 3.2, else 256 x 256 tiles when there
+    are at least 1.5 of them per CU, else 128 x 128
     tiles when they take fewer rounds of the CUs' block slots (three per CU,
     a round counted 0.9 of one of two 256 x 128 blocks), else 256 x 128."""
     t256, ts = size // 256, size // 128
     sym = lambda t: t * (t + 1) // 2
+    if 4 * n * sym(ts) <= 2 * cus and 40 * total * sym(ts) <= 32 * cus:
+        return "64x64", 4 * sym(ts)
     if 2 * n * sym(t256) >= 3 * cus:
         return "256x256", sym(t256)
     big_rounds = -(-n * 2 * sym(t256) // (2 * cus))
@@ -280,22 +286,25 @@ def expected_square_geometry(n, size, cus):
 
 
 @pytest.mark.parametrize("mode", ["fp32", "comp_bf16", "mixed"])
-@pytest.mark.parametrize("batch,size,geometry", [(8, 512, "128x128"), (74, 768, "256x128"), (800, 256, "256x256")])
+@pytest.mark.parametrize("batch,size,geometry", [(3, 1024, "64x64"), (3, 1280, "128x128"), (20, 512, "64x64"),
+                                                 (21, 512, "128x128"), (74, 768, "256x128"), (800, 256, "256x256")])
 def test_s8_square_tile_geometries(device, mode, batch, size, geometry):
-    """The square phase takes 256 x 256 tiles when the launch has at least
-    1.5 of them per CU, else 128 x 128 tiles when they need fewer rounds of
-    the CUs' block slots, else 256 x 128 tiles.  A class of 4 or more
-    matrices runs as two launch chains of halves, and each chain's launches
-    decide for themselves: 4 matrices of 512 x 512 on 256 CUs give 40 small
-    tiles against 24 of 256 x 128, one round each; 37 of 768 x 768 give 777
-    small tiles (two rounds of three per CU) against 444 of 256 x 128 (one
-    round of two) and 222 of 256 x 256; 400 of 256 x 256 give 400 tiles of
-    256 x 256.  Every geometry meets the gates; the recorded square FLOPs
-    show which one ran."""
+    """The square phase takes 64 x 64 tiles up to two per CU and launch and
+    3.2 per CU over the launch chains, else 256 x 256 tiles when the launch
+    has at least 1.5 of them per CU, else 128 x 128 tiles when they need fewer
+    rounds of the CUs' block slots, else 256 x 128 tiles.  A class of 4 or
+    more matrices runs as two launch chains of halves.  On 256 CUs: 3 matrices
+    of 1024 x 1024 give 432 tiles of 64 x 64, 3 of 1280 x 1280 660; 20 of
+    512 x 512 800 in two chains, 21 840; 37 of 768 x 768 give 777 tiles of
+    128 x 128 (two rounds of three per CU) against 444 of 256 x 128 (one round
+    of two) and 222 of 256 x 256; 400 of 256 x 256 give 400 tiles of
+    256 x 256.  Every geometry meets the gates; the recorded tiles show which
+    one ran."""
     cus = torch.cuda.get_device_properties(device).multi_processor_count
     chains = [batch - batch // 2, batch // 2] if batch >= 4 else [batch]
     for n in chains:
-        assert expected_square_geometry(n, size, cus)[0] == geometry, "the case no longer selects the geometry it names"
+        assert expected_square_geometry(n, batch, size, cus)[0] == geometry, \
+            "the case no longer selects the geometry it names"
     torch.manual_seed(batch)
     x = torch.randn(batch, size, size)
     from sandmuon_amd import _native
@@ -306,7 +315,8 @@ def test_s8_square_tile_geometries(device, mode, batch, size, geometry):
         _native.s8_timing(False)
     rec = _native.s8_timing_read()
     tm, tn, waves = GEOMETRY[geometry]
-    tiles = expected_square_geometry(chains[0], size, cus)[1]
+    assert {t for t in _native.s8_timing_tiles() if t[0] == "square"} == {("square", tm, tn)}
+    tiles = expected_square_geometry(chains[0], batch, size, cus)[1]
     # per matrix: stage 1 (G G) and stages 2-5 (G G plus the one-hot (b/c) G
     # MFMAs)
     fs = [tiles * 2 * tm * tn * size * prod(mode, k) + (0 if k == 1 else one_hot_flops(mode, k, tiles, tm, waves))

@@ -14,13 +14,17 @@ pytestmark = pytest.mark.gpu
 
 
 def _both(fn):
-    out = []
+    out, tiles = [], []
     for policy in (0, 2):
         prev = _native.s8_tile_geometry(policy)
+        _native.s8_timing(True)
         try:
             out.append(fn())
         finally:
+            _native.s8_timing(False)
             _native.s8_tile_geometry(prev)
+        tiles.append({t[1:] for t in _native.s8_timing_tiles()})
+    assert tiles == [{(64, 64)}, {(128, 128)}]
     return out
 
 

@@ -83,7 +83,7 @@ def test_tiled_index_is_a_bijection_keeping_row_blocks_in_place():
 
 
 @pytest.mark.parametrize("form", ["planes", "f32", "f16"])
-@pytest.mark.parametrize("tm,waves", [(128, 4), (256, 4), (256, 8)])
+@pytest.mark.parametrize("tm,waves", [(64, 4), (128, 4), (256, 4), (256, 8)])
 def test_row_major_tile_loads(form, tm, waves):
     """tile_offsets: the loads of one 16-deep stage (32-deep for FP16) of
     rows row0 .. row0 + tm - 1 leave logical chunk kc of tile row r at LDS
@@ -159,66 +159,66 @@ def km_stage(form, tn, waves, ld, k0, n0):
     return lds
 
 
-@pytest.mark.parametrize("tn,waves", [(128, 4), (256, 8)])
-def test_k_major_planes_reads(tn, waves):
+@pytest.mark.parametrize("tn,waves,blocks", [(64, 4, 1), (128, 4, 2), (256, 8, 2)])
+def test_k_major_planes_reads(tn, waves, blocks):
     """bkm_lane + load_b_km (BF16 planes): lane (n, h) of the wave's column
     block j gets B[k0 + 8h .. + 7][n] of each plane, conflict-free."""
     ld, k0, n0 = 512, 32, tn
     lds = km_stage("planes", tn, waves, ld, k0, n0)
-    for wn in range(tn // 64):
+    for wn in range(tn // (32 * blocks)):
         def lane_off(lane, pl):
             g, s = lane >> 4, lane & 15
             k = 8 * (g >> 1) + (s >> 2)
-            return (4 * wn + (g & 1)) * 1024 + k * 64 + 8 * ((s >> 1) & 1) + (((2 * pl + (s & 1)) ^ swzt(k, g & 1)) << 4)
-        for j in range(2):
+            return (2 * blocks * wn + (g & 1)) * 1024 + k * 64 + 8 * ((s >> 1) & 1) + (((2 * pl + (s & 1)) ^ swzt(k, g & 1)) << 4)
+        for j in range(blocks):
             for pl in range(2):
                 for second in range(2):
                     addr_of = lambda sl: lane_off(sl, pl) + 2048 * j + 256 * second
                     got = tr16(lds, addr_of)
                     for lane in range(64):
-                        n, h = 64 * wn + 32 * j + sw23(lane & 31), lane >> 5
+                        n, h = 32 * (blocks * wn + j) + sw23(lane & 31), lane >> 5
                         want = [("hi" if pl == 0 else "lo", k0 + 8 * h + 4 * second + t, n0 + n) for t in range(4)]
                         assert got[lane] == want
                     assert conflicts(addr_of, 16, 32) == 0 and conflicts(addr_of, 32, 64) == 0
 
 
-@pytest.mark.parametrize("tn,waves", [(128, 4), (256, 8)])
-def test_k_major_f16_reads(tn, waves):
+@pytest.mark.parametrize("tn,waves,blocks", [(64, 4, 1), (128, 4, 2), (256, 8, 2)])
+def test_k_major_f16_reads(tn, waves, blocks):
     """bkm_lane_f16 + load_b_km (FP16, 32-deep stages): lane (n, h) of
     block j gets B[k0 + 16 half + 8h .. + 7][n], conflict-free."""
     ld, k0, n0 = 512, 64, tn
     lds = km_stage("f16", tn, waves, ld, k0, n0)
     block_bytes = (2 * tn) // 64 * 1024
-    for wn in range(tn // 64):
+    for wn in range(tn // (32 * blocks)):
         def lane_off(lane, j):
             g, s = lane >> 4, lane & 15
             k = 8 * (g >> 1) + (s >> 2)
-            return (2 * wn + j) * 1024 + k * 64 + 8 * ((s >> 1) & 1) + (((2 * (g & 1) + (s & 1)) ^ swzt_h(k)) << 4)
-        for j in range(2):
+            return (blocks * wn + j) * 1024 + k * 64 + 8 * ((s >> 1) & 1) + (((2 * (g & 1) + (s & 1)) ^ swzt_h(k)) << 4)
+        for j in range(blocks):
             for half in range(2):
                 for second in range(2):
                     addr_of = lambda sl: lane_off(sl, j) + half * block_bytes + 256 * second
                     got = tr16(lds, addr_of)
                     for lane in range(64):
-                        n, h = 64 * wn + 32 * j + sw23(lane & 31), lane >> 5
+                        n, h = 32 * (blocks * wn + j) + sw23(lane & 31), lane >> 5
                         want = [("x", k0 + 16 * half + 8 * h + 4 * second + t, n0 + n) for t in range(4)]
                         assert got[lane] == want
                     assert conflicts(addr_of, 16, 32) == 0 and conflicts(addr_of, 32, 64) == 0
 
 
-@pytest.mark.parametrize("tn,waves", [(128, 4), (256, 8)])
-def test_k_major_f32_reads(tn, waves):
+@pytest.mark.parametrize("tn,waves,blocks", [(64, 4, 1), (128, 4, 2), (256, 8, 2)])
+def test_k_major_f32_reads(tn, waves, blocks):
     """load_b_km (FP32 mode, natural column order): lane (n, h) reads
-    B[k0 + 8h + q][n] at (4 wn + pp) KB + 512 h + 4 (lane & 15) + 2 KB j +
+    B[k0 + 8h + q][n] at (2 blocks wn + pp) KB + 512 h + 4 (lane & 15) + 2 KB j +
     64 q."""
     ld, k0, n0 = 512, 32, tn
     lds = km_stage("f32", tn, waves, ld, k0, n0)
-    for wn in range(tn // 64):
+    for wn in range(tn // (32 * blocks)):
         for lane in range(64):
-            base = (4 * wn + ((lane >> 4) & 1)) * 1024 + 512 * (lane >> 5) + 4 * (lane & 15)
-            for j in range(2):
+            base = (2 * blocks * wn + ((lane >> 4) & 1)) * 1024 + 512 * (lane >> 5) + 4 * (lane & 15)
+            for j in range(blocks):
                 for q in range(8):
-                    n, k = 64 * wn + 32 * j + (lane & 31), 8 * (lane >> 5) + q
+                    n, k = 32 * (blocks * wn + j) + (lane & 31), 8 * (lane >> 5) + q
                     assert lds[base + 2048 * j + 64 * q] == ("f", k0 + k, n0 + n)
 
 
