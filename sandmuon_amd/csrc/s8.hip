@@ -1624,11 +1624,13 @@ s8_stage_kernel(StageArgs args) {
         w[e] = acc[i][j][e] * scale;
         // stage 1's FP32 G2: its squared entries feed the Schatten scale
         if constexpr (PHASE == kSquare && (FM == kFormF32 || FM == kFormAny)) sq = fmaf(w[e], w[e], sq);
-        if (do_m) U[col16(e) * kEpStride + lr] = w[e];
       }
       // (FP32 within a block, FP64 over blocks: the sum, to FP64's rounding,
       // of every geometry)
       if constexpr (PHASE == kSquare && (FM == kFormF32 || FM == kFormAny)) sq_local += static_cast<double>(sq);
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (do_m) U[col16(e) * kEpStride + lr] = w[e];
       if (do_t) {
         if (eye) {
           // the diagonal's column in the lane's col16 order, if it has one
