@@ -42,6 +42,8 @@
 #include <cfloat>
 #include <cmath>
 #include <memory>
+#include <numeric>
+#include <tuple>
 #include <vector>
 
 namespace smx {
@@ -1197,13 +1199,14 @@ static bool oriented(const smx_matrix_desc &d, int64_t &r, int64_t &c, bool &fli
   return true;
 }
 
-// Groups of matrices with at most kMaxClasses distinct oriented shapes,
-// formed greedily in table order.
-static std::vector<std::vector<int32_t>> shape_groups(const int64_t *rows, const int64_t *cols, int32_t n) {
+// Groups of the matrices `of` with at most kMaxClasses distinct oriented
+// shapes, or shapes and `low` (S8Class::low), formed greedily in order.
+static std::vector<std::vector<int32_t>> class_groups(const int64_t *rows, const int64_t *cols, const bool *low,
+                                                      const std::vector<int32_t> &of) {
   std::vector<std::vector<int32_t>> groups;
-  std::vector<std::pair<int64_t, int64_t>> shapes;
-  for (int32_t i = 0; i < n; ++i) {
-    const std::pair<int64_t, int64_t> s(std::min(rows[i], cols[i]), std::max(rows[i], cols[i]));
+  std::vector<std::tuple<int64_t, int64_t, bool>> shapes;
+  for (const int32_t i : of) {
+    const std::tuple<int64_t, int64_t, bool> s(std::min(rows[i], cols[i]), std::max(rows[i], cols[i]), low && low[i]);
     if (groups.empty() || (std::find(shapes.begin(), shapes.end(), s) == shapes.end() &&
                            static_cast<int>(shapes.size()) == kMaxClasses)) {
       groups.emplace_back();
@@ -1213,6 +1216,12 @@ static std::vector<std::vector<int32_t>> shape_groups(const int64_t *rows, const
     groups.back().push_back(i);
   }
   return groups;
+}
+
+static std::vector<std::vector<int32_t>> shape_groups(const int64_t *rows, const int64_t *cols, int32_t n) {
+  std::vector<int32_t> all(n);
+  std::iota(all.begin(), all.end(), 0);
+  return class_groups(rows, cols, nullptr, all);
 }
 
 // The job table follows the S8 buffers of a group.
@@ -1229,8 +1238,8 @@ static size_t group_bytes(const int64_t *rows, const int64_t *cols, const std::v
   }
   S8Plan plan;
   std::vector<int32_t> cls(m), slot(m);
-  plan_s8(r.data(), c.data(), fl.get(), m, mode, nullptr, plan, cls.data(), slot.data());
-  return plan.bytes + table_bytes(m);
+  plan_s8(r.data(), c.data(), fl.get(), nullptr, m, mode, nullptr, plan, cls.data(), slot.data());
+  return plan.bytes + kPlanSlack + table_bytes(m);
 }
 
 // Waves per row and float4 per lane for rows of `cols` columns.
@@ -1291,6 +1300,7 @@ extern "C" int smx_matrix_step(const smx_matrix_desc *descs, int32_t n, int mode
   SMX_REQUIRE(mode == SMX_S8_FP32 || mode == SMX_S8_COMP_BF16 || mode == SMX_S8_MIXED, SMX_EINVAL,
               "matrix_step: unknown S8 mode");
   std::vector<int64_t> rows(n), cols(n);
+  std::unique_ptr<bool[]> low(new bool[n]);
   for (int32_t i = 0; i < n; ++i) {
     const smx_matrix_desc &d = descs[i];
     SMX_REQUIRE(d.param && d.grad && d.momentum && d.inv_row && d.inv_col, SMX_EINVAL,
@@ -1306,6 +1316,7 @@ extern "C" int smx_matrix_step(const smx_matrix_desc *descs, int32_t n, int mode
                 "matrix_step: param dtype must be f32, bf16 or f16");
     rows[i] = d.rows;
     cols[i] = d.cols;
+    low[i] = d.param_dtype != SMX_F32;
   }
   const size_t need = smx_matrix_step_workspace_bytes(rows.data(), cols.data(), n, mode);
   SMX_REQUIRE(workspace_bytes >= need, SMX_EWORKSPACE, "matrix_step: workspace too small");
@@ -1313,21 +1324,26 @@ extern "C" int smx_matrix_step(const smx_matrix_desc *descs, int32_t n, int mode
               "matrix_step: workspace must be 256-byte aligned");
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool r1 = descs[0].z != nullptr;
-  for (const auto &g : shape_groups(rows.data(), cols.data(), n)) {
+  // The groups the workspace is sized for, each in one part unless its shapes
+  // come with parameters of both widths in more than kMaxClasses classes.
+  std::vector<std::vector<int32_t>> groups;
+  for (const auto &g : shape_groups(rows.data(), cols.data(), n))
+    for (auto &part : class_groups(rows.data(), cols.data(), low.get(), g)) groups.push_back(std::move(part));
+  for (const auto &g : groups) {
     const int32_t m = static_cast<int32_t>(g.size());
     std::vector<int64_t> r(m), c(m);
-    std::unique_ptr<bool[]> fl(new bool[m]);
+    std::unique_ptr<bool[]> fl(new bool[m]), lo(new bool[m]);
     for (int32_t k = 0; k < m; ++k) {
       bool f;
       oriented(descs[g[k]], r[k], c[k], f);
       fl[k] = f;
+      lo[k] = low[g[k]];
     }
     S8Plan plan;
     std::vector<int32_t> cls(m), slot(m);
-    if (!plan_s8(r.data(), c.data(), fl.get(), m, mode, static_cast<char *>(workspace), plan, cls.data(),
+    if (!plan_s8(r.data(), c.data(), fl.get(), lo.get(), m, mode, static_cast<char *>(workspace), plan, cls.data(),
                  slot.data()))
       return fail(SMX_EINVAL, "matrix_step: internal shape grouping error");
-    plan.layout.keep_bits = std::any_of(g.begin(), g.end(), [&](int32_t i) { return descs[i].param_dtype != SMX_F32; });
     s8_choose_pairs(plan.layout);
     MatJob *table = reinterpret_cast<MatJob *>(static_cast<char *>(workspace) + plan.bytes);
     // Table order (one whiten launch each): parameters kept as they are,

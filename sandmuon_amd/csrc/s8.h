@@ -56,6 +56,13 @@ struct S8Class {
   int32_t tiles_s;     // rp / kSymTile
   int32_t gs;          // Gram-space iteration (cp > rp): the stages run on r x r
                        // products and X0 is applied once, at stage 5
+  int32_t low;         // matrices of 16-bit parameters: the arithmetic is not replaced
+                       // by one that is as close or closer to FP64 with other roundings
+                       // (small matrices in one block, FP16 pairs in the place of FP32
+                       // MFMAs, the third part of mma_one_hot's scalar).  An update that
+                       // is rounded to 8 or 11 bits, twice, turns a difference of 1e-4 of
+                       // the direction into up to two last places of single weights.  A
+                       // class of its own, so that it is no other matrix's rule
   // Iterate buffers (4 bytes per element), oriented layout only: tiled
   // operands (tiled_index), FP32 in SMX_S8_FP32 mode and interleaved BF16
   // hi/lo (put_operand) or FP16 in the others, except the stage-5 result,
@@ -87,12 +94,6 @@ struct S8Layout {
   int32_t n_classes;
   int32_t mode;
   int32_t rowsums;  // the stage-5 apply writes the mapback row-sum partials (matrix step)
-  // Matrices of 16-bit parameters: the arithmetic is not replaced by one that
-  // agrees to rounding only (FP16 pairs in the place of FP32 MFMAs).  Where an
-  // update is rounded to 8 or 11 bits, a last-place difference of the
-  // direction moves single weights by a whole last place, so such runs keep
-  // the bits they had.
-  int32_t keep_bits;
   int32_t pairs;  // SMX_S8_FP32 on FP16 pairs (s8_choose_pairs)
 };
 
@@ -250,8 +251,11 @@ struct S8Plan {
 // Compute the class layout for oriented shapes; `flips[i]` marks matrices
 // whose parameter layout is the transpose of the oriented shape.  Fills
 // class/slot of each matrix.  Returns false if more than kMaxClasses shapes.
-bool plan_s8(const int64_t *r, const int64_t *c, const bool *flips, int32_t n, int mode,
+// `low`: see S8Class::low (null: none).  A plan of more classes of the same
+// matrices takes at most kPlanSlack bytes more.
+bool plan_s8(const int64_t *r, const int64_t *c, const bool *flips, const bool *low, int32_t n, int mode,
              char *base, S8Plan &plan, int32_t *cls_of, int32_t *slot_of);
+constexpr size_t kPlanSlack = kMaxClasses * 16 * 256;  // 256-byte rounding of at most 16 buffers a class
 
 // Whether a class's matrices run whole in one block's LDS (s8_small.hip).
 bool s8_small(const S8Class &k);
@@ -259,9 +263,8 @@ bool s8_small(const S8Class &k);
 // adds its MFMA FLOPs.
 int run_s8_small(const S8Layout &layout, hipStream_t st, double &flops);
 
-// Sets `pairs`, and the classes' iteration form under it.  To be called once
-// a layout's keep_bits is set, before its results are located
-// (S8Mat::result).
+// Sets `pairs`, and the classes' iteration form under it.  To be called before
+// a layout's results are located (S8Mat::result).
 void s8_choose_pairs(S8Layout &layout);
 
 // Run the five S8 stages on a planned layout whose x0 and input norms

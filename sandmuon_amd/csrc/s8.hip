@@ -40,8 +40,7 @@
 // epilogue reads G.
 //
 // Arithmetic modes:
-//   SMX_S8_FP32       v_mfma_f32_32x32x2_f32 on FP32 operands (S8Layout::
-//                     keep_bits: the matrices of 16-bit parameters), or as
+//   SMX_S8_FP32       v_mfma_f32_32x32x2_f32 on FP32 operands, or as
 //                     kS8Pair: every operand, scaled by a power of two into
 //                     FP16's range (kExpX ...), an FP16 pair hi + lo of 22
 //                     significant bits in the place of FP32's 24; acc +=
@@ -740,6 +739,12 @@ __device__ __forceinline__ void mma_row(const AFrag<MODE> &a, const BFrags<MODE,
 // rows R..R+15 of the wave hold G[R + k][col] in accumulator layout; an A
 // fragment that is s on the diagonal k = row - R (a scaled one-hot row)
 // adds s G to those accumulator rows with the ordinary (compensated) MFMAs.
+// The scalar of that term; third: in three BF16 parts, not two (S8Class::low).
+struct SelScalar {
+  float s;
+  bool third;
+};
+
 template <int MODE>
 __device__ __forceinline__ AFrag<MODE> one_hot(float s, int r0) {
   const int lane = threadIdx.x & 63;
@@ -785,7 +790,9 @@ __device__ __forceinline__ AFrag<MODE> one_hot(float s, int r0) {
 // and lo against the stage's first 16 K (rows r0 = 0 .. 15 of the block)
 // and its second 16 K (rows 16 .. 31); FP32 one product.
 template <int MODE, int N>
-__device__ __forceinline__ void mma_one_hot(float s, int sel, const BFrags<MODE, N> &b, f32x16 (&acc)[N]) {
+__device__ __forceinline__ void mma_one_hot(const SelScalar &sel_s, int sel, const BFrags<MODE, N> &b,
+                                            f32x16 (&acc)[N]) {
+  const float s = sel_s.s;
   if constexpr (MODE == kS8F16) {
     const AFrag<MODE> o0 = one_hot<MODE>(s, 0), o1 = one_hot<MODE>(s, 16);
 #pragma unroll
@@ -806,9 +813,11 @@ __device__ __forceinline__ void mma_one_hot(float s, int sel, const BFrags<MODE,
     const AFrag<MODE> o = one_hot<MODE>(s, (sel & 1) * 16);
     // (the third part: s less its hi and lo, exact in FP32)
     const float sh = static_cast<float>(static_cast<__bf16>(s)), sl = static_cast<float>(static_cast<__bf16>(s - sh));
-    const AFrag<MODE> r = one_hot<MODE>((s - sh) - sl, (sel & 1) * 16);
+    // (two parts: products with 0, which leave the accumulator's bits)
+    AFrag<MODE> r = one_hot<MODE>(sel_s.third ? (s - sh) - sl : 0.f, (sel & 1) * 16);
+    r.l = one_hot<MODE>(sel_s.third ? sl : 0.f, (sel & 1) * 16).h;
 #pragma unroll
-    for (int j = 0; j < N; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.l[j], o.l, acc[j], 0, 0, 0);
+    for (int j = 0; j < N; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.l[j], r.l, acc[j], 0, 0, 0);
 #pragma unroll
     for (int j = 0; j < N; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], r.h, acc[j], 0, 0, 0);
     mma_row<MODE>(o, b, acc);
@@ -881,7 +890,7 @@ __device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xC07F);
 // kStages - 2 stages may stay in flight (no run-time conditions).
 template <int MODE, class G, int SEL, int PAR, bool STEADY, bool BKM>
 __device__ __forceinline__ void pipe_iter(const Opnd &A, const Opnd &B, const WaveOffsets<G> &o, const BkmLane &bl,
-                                          uint32_t lds0, float sel_s, char *smem, int kt, int nk, int wm, int wn,
+                                          uint32_t lds0, const SelScalar &sel_s, char *smem, int kt, int nk, int wm, int wn,
                                           AFrag<MODE> (&af)[G::kSubM], BFrags<MODE> (&bf)[2],
                                           f32x16 (&acc)[G::kSubM][kSubN]) {
   constexpr int S = G::kStages;
@@ -916,7 +925,7 @@ __device__ __forceinline__ void pipe_iter(const Opnd &A, const Opnd &B, const Wa
 // addressed in 4-byte units, half of each.
 template <int MODE, class G, bool ACCG, bool BKM, bool UB = false>
 __device__ __forceinline__ void gemm_tile(const Opnd &A_in, const Opnd &B_in, int64_t K, int64_t arow0, int64_t brow0,
-                                          float sel_s, char *smem, f32x16 (&acc)[G::kSubM][kSubN]) {
+                                          const SelScalar &sel_s, char *smem, f32x16 (&acc)[G::kSubM][kSubN]) {
   constexpr int kSubM = G::kSubM;
   constexpr bool F16 = MODE == kS8F16;
   constexpr int kU = F16 ? 2 : 1;  // elements per 4-byte unit
@@ -1007,7 +1016,7 @@ __device__ __forceinline__ void gemm_tile(const Opnd &A_in, const Opnd &B_in, in
 // (16 KB per stage, 128 cycles at 128 bytes per cycle, for 96 of MFMAs).
 template <int MODE, bool ACCG, bool BKM>
 __device__ __forceinline__ void gemm_tile_quad(const Opnd &A_in, const Opnd &B_in, int64_t K, int64_t arow0,
-                                               int64_t brow0, float sel_s, char *smem, bool pairs, bool by_col,
+                                               int64_t brow0, const SelScalar &sel_s, char *smem, bool pairs, bool by_col,
                                                f32x16 (&acc)[1][kSubN]) {
   using G = GeoT;
   constexpr bool F16 = MODE == kS8F16;
@@ -1105,7 +1114,7 @@ __device__ __forceinline__ void gemm_tile_quad(const Opnd &A_in, const Opnd &B_i
 // One product of a tile in geometry G.
 template <int MODE, class G, bool ACCG, bool BKM, bool UB = false>
 __device__ __forceinline__ void gemm_any(const Opnd &A, const Opnd &B, int64_t K, int64_t arow0, int64_t brow0,
-                                         float sel_s, char *smem, bool pairs, bool by_col,
+                                         const SelScalar &sel_s, char *smem, bool pairs, bool by_col,
                                          f32x16 (&acc)[G::kSubM][kSubN]) {
   if constexpr (G::kQuad) gemm_tile_quad<MODE, ACCG, BKM>(A, B, K, arow0, brow0, sel_s, smem, pairs, by_col, acc);
   else gemm_tile<MODE, G, ACCG, BKM, UB>(A, B, K, arow0, brow0, sel_s, smem, acc);
@@ -1317,7 +1326,7 @@ s8_stage_kernel(StageArgs args) {
     }
     if constexpr (kPair) scale *= pow2f(-kExpP);  // P G -> T, T P -> G
     gemm_any<MODE, Gm, false, false, MODE == kS8CompMix>(Opnd{A, K.rp}, Opnd{B, K.rp}, K.rp, tm * Gm::kTileM,
-                                                         tn * kTileN, 0.f, smem, pairs, by_col, acc);
+                                                         tn * kTileN, SelScalar{}, smem, pairs, by_col, acc);
   } else if constexpr (PHASE == kGram) {
     if (stage == 1) {
       const double f = M.cst()[kCstFro];
@@ -1327,7 +1336,7 @@ s8_stage_kernel(StageArgs args) {
     }
     // A Gram-space class takes its stage-3 Gram of X2 from x1.
     const Opnd X{K.gs && stage == 3 ? M.x1() : x_in, K.cp};
-    gemm_any<MODE, Gm, false, false>(X, X, K.cp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, pairs, by_col, acc);
+    gemm_any<MODE, Gm, false, false>(X, X, K.cp, tm * Gm::kTileM, tn * kTileN, SelScalar{}, smem, pairs, by_col, acc);
   } else if constexpr (PHASE == kSquare) {
     const Opnd G{M.g(), K.rp};
     // (the square kernels run at the VGPR budget, where the compiler keeps
@@ -1335,13 +1344,13 @@ s8_stage_kernel(StageArgs args) {
     constexpr bool kUB = true;
     if (stage == 1) {
       if constexpr (kPair) scale = pow2f(-2 * kExpG);
-      gemm_any<MODE, Gm, false, false, kUB>(G, G, K.rp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, pairs, by_col, acc);
+      gemm_any<MODE, Gm, false, false, kUB>(G, G, K.rp, tm * Gm::kTileM, tn * kTileN, SelScalar{}, smem, pairs, by_col, acc);
     } else {
       // acc = G G + (b/c) G; the epilogue forms P = c acc + a I.
       scale = kPair ? args.c * pow2f(kExpP - 2 * kExpG) : args.c;
       gemm_any<MODE, Gm, true, false, kUB>(G, G, K.rp, tm * Gm::kTileM, tn * kTileN,
-                                            kPair ? (shift ? args.bh_over_c : args.b_over_c) * pow2f(kExpG)
-                                                  : args.b_over_c, smem, pairs, by_col, acc);
+                                           SelScalar{kPair ? (shift ? args.bh_over_c : args.b_over_c) * pow2f(kExpG)
+                                                           : args.b_over_c, K.low == 0}, smem, pairs, by_col, acc);
     }
   } else {
     // X-space: X' = P X (stage 1: X' = P1 V / (||V|| s)).  Gram space:
@@ -1362,7 +1371,7 @@ s8_stage_kernel(StageArgs args) {
     const float *A = mid ? M.qb() : fin ? M.qa() : M.p();
     const Opnd B = gq ? Opnd{q_in, K.rp} : Opnd{mid ? M.x0() : fin ? M.x1() : x_in, K.cp};
     // B = X (or Q) rows k (K-major), columns of the tile.
-    gemm_any<MODE, Gm, false, true>(Opnd{A, K.rp}, B, K.rp, tm * Gm::kTileM, tn * kTileN, 0.f, smem, pairs, by_col, acc);
+    gemm_any<MODE, Gm, false, true>(Opnd{A, K.rp}, B, K.rp, tm * Gm::kTileM, tn * kTileN, SelScalar{}, smem, pairs, by_col, acc);
   }
 
   // ------------------------------------------------------- epilogue ---
@@ -2221,9 +2230,9 @@ int run_s8_stages(const S8Layout &layout, hipStream_t st) {
   int slot = -1;
   int rc = timing_begin(st, slot, true);
   S8Layout Lay = layout;
-  // Small classes run whole in one block each, except where bits are kept, or
-  // a tile geometry or a compensation mask is forced (test aids).
-  const bool small = g_tile_policy == 0 && g_comp_mask == 0x1f && !Lay.keep_bits;
+  // Small classes run whole in one block each, except where a tile geometry
+  // or a compensation mask is forced (test aids).
+  const bool small = g_tile_policy == 0 && g_comp_mask == 0x1f;
   if (Lay.pairs) {
     Lay.mode = kS8Pair;
     if (!rc) rc = run_s8_pair0(Lay, small, st);
@@ -2305,8 +2314,8 @@ int run_s8_stages(const S8Layout &layout, hipStream_t st) {
   return timing_end(slot, st, kSpan, flops);
 }
 
-// SMX_S8_FP32 runs on FP16 pairs (kS8Pair) unless the bits of FP32 MFMAs are
-// kept, or a matrix of up to 32 rows is wider than 256: the pairs' 22 bits
+// SMX_S8_FP32 runs on FP16 pairs (kS8Pair) unless there is a class of 16-bit
+// parameters, or a matrix of up to 32 rows is wider than 256: the pairs' 22 bits
 // cost more there than the longer accumulation of FP32 MFMAs (16 x 700: error
 // 7.2e-6 against 4.2e-6).  Small Gram-space classes then iterate in X-space,
 // where P comes from H = G - I: the r x r products of Gram space carry G
@@ -2314,30 +2323,32 @@ int run_s8_stages(const S8Layout &layout, hipStream_t st) {
 // short run takes fewer launches so (15 of 23).  From about 160 rows on
 // both are at or below FP32's error.
 void s8_choose_pairs(S8Layout &L) {
-  L.pairs = L.mode == SMX_S8_FP32 && !L.keep_bits;
+  L.pairs = L.mode == SMX_S8_FP32;
   for (int i = 0; i < L.n_classes; ++i)
-    if (L.cls[i].r <= 32 && L.cls[i].gs && !s8_small(L.cls[i])) L.pairs = 0;
+    if (L.cls[i].low || (L.cls[i].r <= 32 && L.cls[i].gs && !s8_small(L.cls[i]))) L.pairs = 0;
   for (int i = 0; i < L.n_classes && L.pairs; ++i)
     if (L.cls[i].r <= 160) L.cls[i].gs = 0;
 }
 
-bool plan_s8(const int64_t *r, const int64_t *c, const bool *flips, int32_t n, int mode, char *base,
+bool plan_s8(const int64_t *r, const int64_t *c, const bool *flips, const bool *low, int32_t n, int mode, char *base,
              S8Plan &plan, int32_t *cls_of, int32_t *slot_of) {
   S8Layout &Lay = plan.layout;
   Lay = S8Layout{};
   Lay.mode = mode;
-  // Classes by oriented shape in order of first appearance; transposed
+  // Classes by oriented shape and `low` in order of first appearance; transposed
   // parameters take the low slots of their class.
   std::vector<int> ncount, nflip;
   for (int32_t i = 0; i < n; ++i) {
+    const int32_t lo = low && low[i] ? 1 : 0;
     int ci = -1;
     for (int k = 0; k < Lay.n_classes; ++k)
-      if (Lay.cls[k].r == r[i] && Lay.cls[k].c == c[i]) { ci = k; break; }
+      if (Lay.cls[k].r == r[i] && Lay.cls[k].c == c[i] && Lay.cls[k].low == lo) { ci = k; break; }
     if (ci < 0) {
       if (Lay.n_classes == kMaxClasses) return false;
       ci = Lay.n_classes++;
       Lay.cls[ci].r = r[i];
       Lay.cls[ci].c = c[i];
+      Lay.cls[ci].low = lo;
       ncount.push_back(0);
       nflip.push_back(0);
     }

@@ -122,7 +122,7 @@ static bool plan_single(int64_t batch, int64_t rows, int64_t cols, int mode, cha
   std::unique_ptr<bool[]> f(new bool[batch]);
   for (int64_t i = 0; i < batch; ++i) f[i] = flip;
   std::vector<int32_t> cls(batch), slot(batch);
-  return plan_s8(r.data(), c.data(), f.get(), static_cast<int32_t>(batch), mode, base, plan, cls.data(),
+  return plan_s8(r.data(), c.data(), f.get(), nullptr, static_cast<int32_t>(batch), mode, base, plan, cls.data(),
                  slot.data());
 }
 

@@ -294,7 +294,7 @@ static void launch_small(int64_t bytes, int32_t blocks, const SmallArgs &a, hipS
 }
 
 bool s8_small(const S8Class &k) {
-  return k.r <= 16 * kSmallTiles && small_bytes(k) <= kSmallLdsBig;
+  return !k.low && k.r <= 16 * kSmallTiles && small_bytes(k) <= kSmallLdsBig;
 }
 
 int run_s8_small(const S8Layout &Lay, hipStream_t st, double &flops) {

@@ -76,3 +76,48 @@ def test_small_and_large_classes_in_one_matrix_step(device, mode):
     # 16-bit parameters keep their bits
     for a, b in zip(step(0, torch.bfloat16), step(2, torch.bfloat16)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_mixed_parameter_types_in_one_matrix_step(device, mode, dtype):
+    """An FP32 parameter's update has the same bits beside 16-bit parameters of
+    its shape and others, and a 16-bit one beside FP32 ones (7 shapes in both
+    types: 14 classes, more than one group); the 16-bit update is the FP32
+    one's, to the mode's rounding and its own."""
+    shapes = [(24, 40), (96, 48), (300, 180), (180, 400), (260, 260), (64, 500)] * 2 + [(256, 256)] * 50
+
+    def step(dtypes):
+        g = torch.Generator().manual_seed(5)
+        descs, keep, out = [], [], []
+        for (r, c), dt in zip(shapes, dtypes):
+            t = lambda *s: torch.randn(*s, generator=g).to(device)
+            w = (t(r, c) * .02).to(dtype).to(dt)  # the same values in either type
+            gr, m, ir, ic = t(r, c), t(r, c) * .1, t(r).abs() + .5, t(c).abs() + .5
+            keep += [gr, m, ir, ic]
+            out.append((w, w.double()))
+            descs.append(_native.MatrixDesc(
+                param=w.data_ptr(), grad=gr.data_ptr(), momentum=m.data_ptr(), inv_row=ir.data_ptr(),
+                inv_col=ic.data_ptr(), rows=r, cols=c, lr=1e-2, momentum_beta=.8, param_dtype=_native.dtype_code(dt)))
+        ws = torch.empty(_native.matrix_step_workspace_bytes(shapes, mode), dtype=torch.uint8, device=device)
+        _native.matrix_step(descs, mode, ws)
+        torch.cuda.synchronize()
+        return out
+
+    def close(a, b, w0):
+        # the update and the new weight each by half a last place of the type
+        # (2^-8 or 2^-11 of the value at most; f16: 2^-25 below its normal
+        # range), some FP32 roundings of both, which may cancel, and the map's
+        # error in the mode
+        half, least = (2 ** -8, 0.0) if dtype == torch.bfloat16 else (2 ** -11, 2 ** -25)
+        u = (w0 - b).abs()
+        bound = (b.abs() + u) * half + 2 * least + 2 ** -22 * b.abs().max()
+        return ((a - b).abs() <= bound * (1 + half) + {0: 4e-5, 1: 2e-3, 2: 8e-3}[mode] * u.max()).all()
+
+    n = len(shapes)
+    low = [k % 2 == (k // 6) % 2 for k in range(n)]
+    full, narrow = step([torch.float32] * n), step([dtype] * n)
+    for (a, w0), (b, _) in zip(narrow, full):
+        assert close(a.double(), b.double(), w0)
+    for lo, (a, _), (b, _), (c, _) in zip(low, step([dtype if lo else torch.float32 for lo in low]), full, narrow):
+        assert torch.equal(a, c if lo else b)
