@@ -732,9 +732,7 @@ def main():
     log(f"timed {args.steps} steps: {ms:.3f} ms/step (hooks {hooks_ms:.3f}, step {step_ms:.3f}, "
         f"S8 GEMM launches {s8_ms:.3f})")
 
-    peak_mfma = BF16_PEAK  # FP16 and BF16 MFMA share the peak
-    if args.s8_mode == "fp32":
-        s8_issued *= 3  # recorded as one product per element pair, issued as three FP16 ones
+    peak_mfma = BF16_PEAK  # every mode issues BF16 or FP16 MFMAs, which share the peak
     stats_gbs = stat_bytes / (hooks_ms * 1e-3) / 1e9
     s8_tfs = s8_issued / (s8_ms * 1e-3) / 1e12
     # The committed counter summary covers the cfg4 step in comp_bf16 mode;

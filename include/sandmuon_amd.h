@@ -61,10 +61,14 @@ enum smx_dtype { SMX_F32 = 0, SMX_BF16 = 1, SMX_F16 = 2, SMX_F64 = 3 };
  *   product as three FP16 MFMAs on hi/lo splits (hi*lo + lo*hi + hi*hi,
  *   v_mfma_f32_32x32x16_f16, FP32 accumulation); every operand is scaled by
  *   a power of two into FP16's range and held as the FP16 hi/lo pair (22
- *   significant bits).  Against FP64 it is as close as FP32 MFMAs on FP32
- *   operands, which round the accumulator eight times as often; those
- *   (v_mfma_f32_32x32x2_f32) still run in a matrix step that has 16-bit
- *   parameters, whose bits it keeps.
+ *   significant bits).  In the norm of a matrix's result it is as close to
+ *   FP64 as FP32 MFMAs on FP32 operands, which round the accumulator eight
+ *   times as often, and small rows, columns and blocks keep their own
+ *   accuracy: a matrix in which 16 neighbours of a row or column are all
+ *   below 2^-12 of its root mean square (zeros apart) runs on FP32 operands
+ *   and v_mfma_f32_32x32x2_f32, as its own data decide on the device.  So do
+ *   matrices of few rows and many columns (plan_s8), and those of 16-bit
+ *   parameters, whose bits a matrix step keeps.
  * SMX_S8_COMP_BF16: every product as three BF16 MFMAs on hi/lo splits
  *   (hi*lo + lo*hi + hi*hi, FP32 accumulation); intermediates are stored as
  *   the BF16 hi/lo pair.  The compensated-product scheme of
@@ -388,9 +392,10 @@ int smx_s8(const float *x, float *out, int64_t batch, int64_t rows,
  * padded columns exceed their padded rows, 6 matrices small enough to run
  * whole in one block each)
  * and the MFMA FLOPs the launch (or run) issues (tiles computed x
- * 2*256*256*K, x3 in SMX_S8_COMP_BF16 mode, plus the square phase's
- * one-hot MFMAs; SMX_S8_FP32 counts one product per element pair, a third
- * of what it issues).  It returns the number of records or a negative status.
+ * 2*256*256*K, x3 in SMX_S8_COMP_BF16 and SMX_S8_FP32 mode, plus the square
+ * phase's one-hot MFMAs; a matrix that runs on FP32 MFMAs counts as one on
+ * pairs; phase 6: the FP32 MFMAs of the small matrices).  It returns the
+ * number of records or a negative status.
  * The recorder is process-wide, not thread-safe.
  * ------------------------------------------------------------------ */
 int smx_s8_timing(int32_t enable);

@@ -295,6 +295,7 @@ __global__ void __launch_bounds__(kTotalThreads) matrix_total_kernel(const MatJo
   J.cst[kCstZZ] = s[2];
   J.cst[kCstAZ] = s[3];
   J.cst[kCstFro] = s[0] + (2.0 * kappa + kappa * kappa * s[2]) * s[1];
+  J.cst[kCstWide] = 0.0;
 }
 
 // ------------------------------------------------------------- whiten ---
@@ -1344,7 +1345,6 @@ extern "C" int smx_matrix_step(const smx_matrix_desc *descs, int32_t n, int mode
     if (!plan_s8(r.data(), c.data(), fl.get(), lo.get(), m, mode, static_cast<char *>(workspace), plan, cls.data(),
                  slot.data()))
       return fail(SMX_EINVAL, "matrix_step: internal shape grouping error");
-    s8_choose_pairs(plan.layout);
     MatJob *table = reinterpret_cast<MatJob *>(static_cast<char *>(workspace) + plan.bytes);
     // Table order (one whiten launch each): parameters kept as they are,
     // except those of the next bucket; parameters kept as they are whose

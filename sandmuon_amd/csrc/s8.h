@@ -41,8 +41,10 @@ constexpr double kS8Coefficients[5][3] = {
 // Per-matrix scalars (S8Class::cst): ||V||^2 of the whitened input (the
 // S8 normalisation; the total of the whiten partials, or of the input for
 // the stand-alone map), sum z^2 and sum (a z)^2 of the rank-one term, and
-// ||U||^2 of the mapped-back direction (the graft).
-constexpr int kCstFro = 0, kCstZZ = 1, kCstAZ = 2, kCstU = 3, kCst = 4;
+// ||U||^2 of the mapped-back direction (the graft).  kCstWide: not 0 where the
+// FP32 mode's scan found the input too wide in range for FP16 pairs
+// (s8_scan_kernel; the kernels that write kCstFro clear it).
+constexpr int kCstFro = 0, kCstZZ = 1, kCstAZ = 2, kCstU = 3, kCstWide = 4, kCst = 5;
 
 struct S8Class {
   int64_t r, c;        // oriented logical dims, r <= c
@@ -63,6 +65,7 @@ struct S8Class {
                        // is rounded to 8 or 11 bits, twice, turns a difference of 1e-4 of
                        // the direction into up to two last places of single weights.  A
                        // class of its own, so that it is no other matrix's rule
+  int32_t wide;        // SMX_S8_FP32: every matrix runs on FP32 MFMAs (plan_s8)
   // Iterate buffers (4 bytes per element), oriented layout only: tiled
   // operands (tiled_index), FP32 in SMX_S8_FP32 mode and interleaved BF16
   // hi/lo (put_operand) or FP16 in the others, except the stage-5 result,
@@ -94,7 +97,6 @@ struct S8Layout {
   int32_t n_classes;
   int32_t mode;
   int32_t rowsums;  // the stage-5 apply writes the mapback row-sum partials (matrix step)
-  int32_t pairs;  // SMX_S8_FP32 on FP16 pairs (s8_choose_pairs)
 };
 
 __host__ __device__ inline int64_t sym_tiles(int64_t t) { return t * (t + 1) / 2; }
@@ -124,6 +126,8 @@ struct S8Mat {
   // total has consumed.
   __host__ __device__ double *sch() const { return fro(); }
   __host__ __device__ double *cst() const { return kp()->cst + kCst * static_cast<int64_t>(slot); }
+  // SMX_S8_FP32: the matrix runs on FP32 MFMAs, not on FP16 pairs.
+  __device__ bool wide() const { return kp()->wide != 0 || cst()[kCstWide] != 0.0; }
   __host__ __device__ const float *acol() const { return kp()->colv[2 * slot]; }
   __host__ __device__ const float *zcol() const { return kp()->colv[2 * slot + 1]; }
   __host__ __device__ const float **colv() const { return kp()->colv + 2 * slot; }
@@ -262,10 +266,6 @@ bool s8_small(const S8Class &k);
 // Runs every small class of the layout, a launch per number of row tiles;
 // adds its MFMA FLOPs.
 int run_s8_small(const S8Layout &layout, hipStream_t st, double &flops);
-
-// Sets `pairs`, and the classes' iteration form under it.  To be called before
-// a layout's results are located (S8Mat::result).
-void s8_choose_pairs(S8Layout &layout);
 
 // Run the five S8 stages on a planned layout whose x0 and input norms
 // (cst()[kCstFro]) are filled.  The result of each matrix is in S8Mat::result().

@@ -40,16 +40,21 @@
 // epilogue reads G.
 //
 // Arithmetic modes:
-//   SMX_S8_FP32       v_mfma_f32_32x32x2_f32 on FP32 operands, or as
-//                     kS8Pair: every operand, scaled by a power of two into
-//                     FP16's range (kExpX ...), an FP16 pair hi + lo of 22
-//                     significant bits in the place of FP32's 24; acc +=
-//                     lo*hi + hi*lo + hi*hi with v_mfma_f32_32x32x16_f16 and
-//                     FP32 accumulation.  One rounding of the accumulator
+//   SMX_S8_FP32       (run as kS8Pair) every operand, scaled by a power of
+//                     two into FP16's range (kExpX ...), an FP16 pair hi + lo
+//                     of 22 significant bits in the place of FP32's 24; acc
+//                     += lo*hi + hi*lo + hi*hi with v_mfma_f32_32x32x16_f16
+//                     and FP32 accumulation.  One rounding of the accumulator
 //                     per 16 products instead of one per two makes the map
 //                     no further from FP64 than the FP32 MFMAs, at a fifth
 //                     of their matrix cycles (36 matrices of 768 x 768:
 //                     2755 -> 1175 us a call; error 4.4e-6 -> 2.4e-6).
+//                     One exponent serves a whole matrix, so a matrix whose
+//                     rows, columns or blocks lie far apart in scale runs on
+//                     FP32 operands and v_mfma_f32_32x32x2_f32 instead, as
+//                     its own data decide (s8_scan_kernel; every kernel of
+//                     the mode holds both bodies), and so do the classes
+//                     whose pairs are no closer to FP64 (plan_s8).
 //   SMX_S8_COMP_BF16  every operand is stored by its producer as BF16 hi +
 //                     lo (put_operand); acc += hi*lo + lo*hi + hi*hi with
 //                     v_mfma_f32_32x32x16_bf16 (the compensated product of
@@ -138,7 +143,8 @@ constexpr int kMaxSeg = 2 * kMaxClasses;
 //              code would otherwise outgrow the instruction cache).
 constexpr int kS8HiOnly = 3;
 constexpr int kS8F16 = 4;
-//   kS8Pair    SMX_S8_FP32 on FP16 pairs (above).
+//   kS8Pair    the run mode of SMX_S8_FP32: FP16 pairs, and FP32 MFMAs (the
+//              body of mode SMX_S8_FP32) for the matrices that are wide.
 constexpr int kS8CompMix = 5;
 constexpr int kS8Pair = 6;
 __host__ __device__ constexpr bool is_comp(int m) { return m == SMX_S8_COMP_BF16 || m == kS8CompMix; }
@@ -179,7 +185,7 @@ __device__ __forceinline__ int s8_exp0(double fro2) {
 // The MFMA mode of one product of the map (phase, stage and, for SYM and
 // APPLY, its SegOp) under the run's public `mode` and compensation mask.
 __host__ __device__ constexpr int gemm_mode(int mode, int mask, int phase, int stage, int op, bool gs) {
-  return mode == SMX_S8_FP32 || mode == kS8Pair ? mode
+  return mode == kS8Pair ? mode
          : mode == SMX_S8_COMP_BF16 ? (((mask >> (stage - 1)) & 1) ? SMX_S8_COMP_BF16 : kS8HiOnly)
          : (stage <= 2 || gs) ? kS8CompMix
                               : kS8F16;
@@ -1217,15 +1223,11 @@ __host__ __device__ inline int64_t phase_tiles(const S8Class &k, int phase, int 
   return square_tiles(k, geo);
 }
 
+// One tile of a launch in MFMA mode MODE.
 template <int MODE, int PHASE, int TM, int TN>
-__global__ void __launch_bounds__((Geo<TM, TN>::kThreads))
-__attribute__((amdgpu_waves_per_eu(Geo<TM, TN>::kWavesPerEU, Geo<TM, TN>::kWavesPerEU)))
-s8_stage_kernel(StageArgs args) {
+__device__ __forceinline__ void stage_tile(const StageArgs &args, char *smem, double *dscratch, double *bcast) {
   using Gm = Geo<TM, TN>;
   constexpr int kSubM = Gm::kSubM, kTileN = Gm::kTileN, kThreads = Gm::kThreads, kWaves = Gm::kWaves;
-  __shared__ __attribute__((aligned(16))) char smem[Gm::kRingBytes];
-  __shared__ double dscratch[16];
-  __shared__ double bcast;
 
   const TileRef ref = tile_of(args);
   const S8Class &K = *ref.k;
@@ -1295,7 +1297,7 @@ s8_stage_kernel(StageArgs args) {
   f32x16 acc[kSubM][kSubN];
   // What the epilogue multiplies by; kPair: with the exponents of the FP16
   // pairs (kExpX ...) folded in.
-  constexpr bool kPair = MODE == kS8Pair;
+  constexpr bool kPair = MODE == kS8Pair, kScaled = kPair || MODE == SMX_S8_FP32;  // X0 holds V 2^k (s8_exp0)
   // X-space pairs: from stage 2 on the Gram is stored as H = G - I and P is
   // formed from it.  The iterate's singular values approach 1, so H is small
   // where G is not: neither the rounding of a diagonal near 1 nor the
@@ -1320,7 +1322,7 @@ s8_stage_kernel(StageArgs args) {
       A = M.t(); B = pk; sym_out = M.g();
       if (stage == 1) {
         // G1 = P1 G0 P1 / s^2
-        const Stage1Scalars sc = stage1_scalars(M, args.sq_geo, &bcast);
+        const Stage1Scalars sc = stage1_scalars(M, args.sq_geo, bcast);
         scale = sc.ok ? 1.0f / (sc.s * sc.s) : 0.f;
       }
     }
@@ -1330,7 +1332,7 @@ s8_stage_kernel(StageArgs args) {
   } else if constexpr (PHASE == kGram) {
     if (stage == 1) {
       const double f = M.cst()[kCstFro];
-      scale = f > 0.0 ? static_cast<float>(kPair ? ldexp(1.0 / f, kExpG - 2 * s8_exp0(f)) : 1.0 / f) : 0.f;
+      scale = f > 0.0 ? static_cast<float>(kScaled ? ldexp(1.0 / f, (kPair ? kExpG : 0) - 2 * s8_exp0(f)) : 1.0 / f) : 0.f;
     } else if constexpr (kPair) {
       scale = pow2f(kExpG - 2 * kExpX);
     }
@@ -1358,9 +1360,10 @@ s8_stage_kernel(StageArgs args) {
     const int op = ref.op;
     const bool gq = op == kOpApplyQ, mid = op == kOpApplyMid, fin = op == kOpApplyFinal;
     if (stage == 1 || mid) {
-      const Stage1Scalars sc = stage1_scalars(M, args.sq_geo, &bcast);
+      const Stage1Scalars sc = stage1_scalars(M, args.sq_geo, bcast);
       const double inv = sc.ok ? 1.0 / (sqrt(sc.fro2) * static_cast<double>(sc.s)) : 0.0;
-      scale = static_cast<float>(kPair ? ldexp(inv, kExpX - (mid ? kExpQ : kExpP) - s8_exp0(sc.fro2)) : inv);
+      scale = static_cast<float>(kScaled ? ldexp(inv, (kPair ? kExpX - (mid ? kExpQ : kExpP) : 0) - s8_exp0(sc.fro2))
+                                         : inv);
     } else if constexpr (kPair) {
       // Q2 and Q4 are products of two P (a segment's first Q is its P);
       // the stage-5 results are FP32 without an exponent.
@@ -1399,7 +1402,8 @@ s8_stage_kernel(StageArgs args) {
   bool do_t, do_m;
   // The output's form is that of the product that reads it (out_form); a
   // transposed stage-5 result (dst_m) is FP32 as the stage-5 form is.
-  const int form = out_form(args.L.mode, args.mask, PHASE, stage, ref.op, K.gs != 0);
+  const int form = MODE == SMX_S8_FP32 ? kFormF32
+                                       : out_form(args.L.mode, args.mask, PHASE, stage, ref.op, K.gs != 0);
   if constexpr (PHASE == kApply) {
     if (ref.op == kOpApplyQ) {
       dst_t = q_out; ld_t = K.rp;
@@ -1718,6 +1722,25 @@ s8_stage_kernel(StageArgs args) {
   }
 }
 
+template <int MODE, int PHASE, int TM, int TN>
+__global__ void __launch_bounds__((Geo<TM, TN>::kThreads))
+__attribute__((amdgpu_waves_per_eu(Geo<TM, TN>::kWavesPerEU, Geo<TM, TN>::kWavesPerEU)))
+s8_stage_kernel(StageArgs args) {
+  __shared__ __attribute__((aligned(16))) char smem[Geo<TM, TN>::kRingBytes];
+  __shared__ double dscratch[16];
+  __shared__ double bcast;
+  if constexpr (MODE == kS8Pair) {
+    const TileRef ref = tile_of(args);
+    const int64_t tpm = phase_tiles(*ref.k, PHASE, Geo<TM, TN>::kGeo, ref.op);
+    if (ref.L >= tpm * ref.cnt) return;
+    if (S8Mat{*ref.k, ref.slot0 + static_cast<int>(ref.L / tpm)}.wide()) {  // uniform per block
+      stage_tile<SMX_S8_FP32, PHASE, TM, TN>(args, smem, dscratch, &bcast);
+      return;
+    }
+  }
+  stage_tile<MODE, PHASE, TM, TN>(args, smem, dscratch, &bcast);
+}
+
 // Stage-1 polynomial operand (sandmuon/optimizer.py:84-86) over the r x r
 // matrices of a class: P1 = a I + (b G)/s^2 + (c G2)/s^4 from the
 // normalised G and the FP32 G2 of the square phase, written over G2 in the
@@ -1739,8 +1762,7 @@ __host__ __device__ inline int64_t poly_blocks_per_matrix(const S8Class &k) {
 }
 
 template <int MODE>
-__global__ void __launch_bounds__(256) s8_poly1_kernel(StageArgs args) {
-  __shared__ double bcast;
+__device__ __forceinline__ void poly1_chunk(const StageArgs &args, double *bcast) {
   constexpr bool kPair = MODE == kS8Pair, PL = MODE == SMX_S8_COMP_BF16 || kPair;
   const TileRef ref = tile_of(args);
   const S8Class &K = *ref.k;
@@ -1771,7 +1793,7 @@ __global__ void __launch_bounds__(256) s8_poly1_kernel(StageArgs args) {
       gl[k] = make_uint2(g.z, g.w);
     }
   }
-  const Stage1Scalars sc = stage1_scalars(M, args.sq_geo, &bcast);
+  const Stage1Scalars sc = stage1_scalars(M, args.sq_geo, bcast);
   const float s2 = sc.s * sc.s;
   const float is2 = sc.ok ? 1.0f / s2 : 0.f, is4 = sc.ok ? 1.0f / (s2 * s2) : 0.f;
   // FP16 pairs: G holds 2^kExpG G, P1 goes out as 2^kExpP P1
@@ -1809,14 +1831,84 @@ __global__ void __launch_bounds__(256) s8_poly1_kernel(StageArgs args) {
   }
 }
 
-// kS8Pair: the FP32 iterate X0 that the whiten or the load left becomes
-// FP16 pairs of V 2^k, in place (a group is 64 bytes in both forms).  Only
-// here is ||V|| known, and with it the exponent; 8 bytes per element at the
-// copy rate.  Blocks and lanes as s8_poly1_kernel, over the iterate's groups.
+template <int MODE>
+__global__ void __launch_bounds__(256) s8_poly1_kernel(StageArgs args) {
+  __shared__ double bcast;
+  if constexpr (MODE == kS8Pair) {
+    const TileRef ref = tile_of(args);
+    const int64_t tpm = poly_blocks_per_matrix(*ref.k);
+    if (ref.L >= tpm * ref.cnt) return;
+    if (S8Mat{*ref.k, ref.slot0 + static_cast<int>(ref.L / tpm)}.wide()) {
+      poly1_chunk<SMX_S8_FP32>(args, &bcast);
+      return;
+    }
+  }
+  poly1_chunk<MODE>(args, &bcast);
+}
+
+// SMX_S8_FP32: whether a matrix is too wide in range for pairs.  A pair holds an
+// element below 2^-13 of the operand's scale to an absolute 2^-39 of it, so a
+// row (column, block) at a scale d below the others' has a relative error of
+// about 2e-10 / d where FP32 MFMAs keep 3e-6: 8e-7 at d = 2^-12, the limit
+// here, 2e-4 at 1e-6.  The runs compared are 16 elements of a row and of a
+// column (one 16 x 16 piece of the tiled iterate a wave), by their largest
+// magnitude against the root mean square of the whole matrix: a row or a
+// column that is small consists of small runs, and so does a small block.  Runs
+// of zeros are exact in either form, and runs that the padding cuts short are
+// no evidence (a row or column there has whole runs across).  Gaussian matrices
+// under row and column scales a decade each way stay on pairs: their smallest
+// run is about 2^-8.
+// A pass over X0 at the copy rate (36 matrices of 768 x 768: 20 of 1170 us).
+constexpr float kWideRun = 1.f / 4096.f;
 __host__ __device__ inline int64_t pair_blocks_per_matrix(const S8Class &k) {
   return k.rp * k.cp / 16 / kPolyChunk;
 }
 
+__global__ void __launch_bounds__(256) s8_scan_kernel(StageArgs args) {
+  const TileRef ref = tile_of(args);
+  const S8Class &K = *ref.k;
+  const int64_t tpm = pair_blocks_per_matrix(K);
+  if (ref.L >= tpm * ref.cnt || K.wide) return;
+  const S8Mat M{K, ref.slot0 + static_cast<int>(ref.L / tpm)};
+  const int64_t g0 = (ref.L % tpm) * kPolyChunk, gpr = K.cp / 16;  // first group of the block, groups per row
+  const SMX_GLOBAL f32x4v *X = (const SMX_GLOBAL f32x4v *)M.x0() + g0 * 4 + threadIdx.x;
+  f32x4v x[kPolyUnits];
+#pragma unroll
+  for (int k = 0; k < kPolyUnits; ++k) x[k] = X[256 * k];  // lane l: row l >> 2 of a piece, columns 4 (l & 3) ..
+  const double f = M.cst()[kCstFro];
+  // (no element reaches an infinite limit: a matrix with infinities is wide)
+  const float limit = static_cast<float>(sqrt(f / (static_cast<double>(K.r) * static_cast<double>(K.c)))) * kWideRun;
+  auto small = [&](float m) { return m > 0.f && m < limit; };
+  bool any = false;
+#pragma unroll
+  for (int k = 0; k < kPolyUnits; ++k) {
+    const int64_t piece = (g0 + (threadIdx.x + 256 * k) / 4) / 16;  // 16 groups: 16 rows of one K group
+    const bool rows_whole = (piece / gpr + 1) * 16 <= K.r, cols_whole = (piece % gpr + 1) * 16 <= K.c;
+    float c[4], row = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      c[e] = fabsf(x[k][e]);
+      row = fmaxf(row, c[e]);
+    }
+    row = fmaxf(row, dpp_mov<0xB1>(row));
+    row = fmaxf(row, dpp_mov<0x4E>(row));  // the row's four lanes
+    any = any || (cols_whole && small(row));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+#pragma unroll
+      for (int d = 4; d < 64; d *= 2) c[e] = fmaxf(c[e], __shfl_xor(c[e], d));
+      any = any || (rows_whole && small(c[e]));
+    }
+  }
+  if (any) M.cst()[kCstWide] = 1.0;  // (every writer writes the same)
+}
+
+// SMX_S8_FP32: the FP32 iterate X0 that the whiten or the load left becomes
+// FP16 pairs of V 2^k, in place (a group is 64 bytes in both forms), or FP32
+// V 2^k of a wide matrix (exact: an input of any norm keeps its accuracy).
+// Only here is ||V|| known, and with it the exponent; 8 bytes per element at
+// the copy rate.  Blocks and lanes as s8_poly1_kernel, over the iterate's
+// groups.
 __global__ void __launch_bounds__(256) s8_pair0_kernel(StageArgs args) {
   const TileRef ref = tile_of(args);
   const S8Class &K = *ref.k;
@@ -1834,10 +1926,11 @@ __global__ void __launch_bounds__(256) s8_pair0_kernel(StageArgs args) {
     x[k] = *reinterpret_cast<const SMX_GLOBAL f32x4v *>(X + idx[k]);
   }
   const int e0 = s8_exp0(M.cst()[kCstFro]);
+  const bool pairs = !M.wide();
 #pragma unroll
   for (int k = 0; k < kPolyUnits; ++k) {
     const float v[4] = {ldexpf(x[k].x, e0), ldexpf(x[k].y, e0), ldexpf(x[k].z, e0), ldexpf(x[k].w, e0)};
-    put_operand4_paired<true>(X, idx[k], v, true, true);
+    put_operand4_paired<true>(X, idx[k], v, pairs, true);
   }
 }
 
@@ -1945,23 +2038,21 @@ static std::vector<Seg> launch_segments(const S8Layout &Lay, const SlotSet &set,
 }
 
 // MFMA FLOPs of one launch in MFMA mode `mode`: computed tiles x 2 * TM *
-// TN * K (x3 compensated), plus the square phase's one-hot MFMAs: per wave
-// and 32x32 column tile, 2 kSubM window stages of 5 (compensated), 2
-// (plain BF16: the scalar's hi and lo) or 1 (FP32) 16-deep products, or
+// TN * K (x3 on compensated operands and FP16 pairs; what a wide matrix of
+// SMX_S8_FP32 issues in its place only the device knows), plus the square phase's one-hot MFMAs: per wave
+// and 32x32 column tile, 2 kSubM window stages of 5 (compensated), 3 (pairs)
+// or 2 (plain BF16: the scalar's hi and lo) 16-deep products, or
 // kSubM stages of 4 (FP16: hi and lo over each 16 K of a 32-deep stage).
 static double launch_flops(int mode, int phase, int stage, int geo, const S8Layout &Lay,
                            const std::vector<Seg> &segs) {
   if (phase == kPoly1) return 0.0;
-  const double prod = is_comp(mode) ? 3.0 : 1.0;
+  const double prod = is_split(mode) ? 3.0 : 1.0;
   const int tm = geo == kGeoT ? 64 : geo == kGeoS ? 128 : 256, tn = geo == kGeoT ? 64 : geo == kGeoL ? 256 : 128;
   // waves that issue the one-hot MFMAs of a tile, 32 sub_m rows and kSubN
   // column tiles each (kGeoT: of four waves with half of each)
   const int waves = geo == kGeoT ? 1 : geo == kGeoL ? 8 : 4;
   const int sub_m = geo == kGeoT ? 2 : tm / 64;
-  // (kS8Pair counts one product per element pair, as the FP32 MFMAs whose
-  // place it takes issue; it is carried out as three FP16 ones.)
-  const double onehot = is_comp(mode) ? 10.0 * sub_m : mode == kS8HiOnly ? 4.0 * sub_m
-                        : mode == kS8F16 ? 4.0 * sub_m : 2.0 * sub_m;
+  const double onehot = mode == kS8Pair ? 6.0 * sub_m : is_comp(mode) ? 10.0 * sub_m : 4.0 * sub_m;
   double f = 0.0;
   for (const Seg &sg : segs) {
     const S8Class &k = Lay.cls[sg.cls];
@@ -2106,18 +2197,15 @@ static int launch_phase(const S8Layout &Lay, const SlotSet &set, const SlotSet &
     if constexpr (PHASE == kPoly1) {
       if (mode == kS8Pair)
         hipLaunchKernelGGL(s8_poly1_kernel<kS8Pair>, dim3(off), dim3(256), 0, st, a);
-      else if (mode != SMX_S8_FP32)
-        hipLaunchKernelGGL(s8_poly1_kernel<SMX_S8_COMP_BF16>, dim3(off), dim3(256), 0, st, a);
       else
-        hipLaunchKernelGGL(s8_poly1_kernel<SMX_S8_FP32>, dim3(off), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(s8_poly1_kernel<SMX_S8_COMP_BF16>, dim3(off), dim3(256), 0, st, a);
       rc = check_launch("s8 stage-1 polynomial");
     } else {
       if (mode == SMX_S8_COMP_BF16) launch_stage<SMX_S8_COMP_BF16, PHASE>(geo, off, a, st);
       else if (mode == kS8CompMix) launch_stage<kS8CompMix, PHASE>(geo, off, a, st);
       else if (mode == kS8HiOnly) launch_stage<kS8HiOnly, PHASE>(geo, off, a, st);
       else if (mode == kS8F16) launch_stage<kS8F16, PHASE>(geo, off, a, st);
-      else if (mode == kS8Pair) launch_stage<kS8Pair, PHASE>(geo, off, a, st);
-      else launch_stage<SMX_S8_FP32, PHASE>(geo, off, a, st);
+      else launch_stage<kS8Pair, PHASE>(geo, off, a, st);
       rc = check_launch(PHASE == kGram ? "s8 gram" : PHASE == kSquare ? "s8 square" : PHASE == kSym ? "s8 sym"
                                                                                                   : "s8 apply");
     }
@@ -2207,7 +2295,8 @@ static int fork_stream(ForkStream *&out) {
 // one record for the run, on the caller's stream.
 constexpr int kSplitCount = 2 * kChains;
 
-// The FP16 pairs of the X0 of a kS8Pair run's chains, before they fork.
+// The FP16 pairs (or scaled FP32) of the X0 of a kS8Pair run's chains, before
+// they fork.
 static int run_s8_pair0(const S8Layout &Lay, bool small, hipStream_t st) {
   StageArgs a{};
   a.L = Lay;
@@ -2222,6 +2311,9 @@ static int run_s8_pair0(const S8Layout &Lay, bool small, hipStream_t st) {
   }
   a.seg_off[a.n_seg] = off;
   if (off == 0) return SMX_OK;
+  hipLaunchKernelGGL(s8_scan_kernel, dim3(off), dim3(256), 0, st, a);
+  const int rc = check_launch("s8 input scan");
+  if (rc) return rc;
   hipLaunchKernelGGL(s8_pair0_kernel, dim3(off), dim3(256), 0, st, a);
   return check_launch("s8 input pairs");
 }
@@ -2233,7 +2325,7 @@ int run_s8_stages(const S8Layout &layout, hipStream_t st) {
   // Small classes run whole in one block each, except where a tile geometry
   // or a compensation mask is forced (test aids).
   const bool small = g_tile_policy == 0 && g_comp_mask == 0x1f;
-  if (Lay.pairs) {
+  if (Lay.mode == SMX_S8_FP32) {
     Lay.mode = kS8Pair;
     if (!rc) rc = run_s8_pair0(Lay, small, st);
   }
@@ -2314,22 +2406,6 @@ int run_s8_stages(const S8Layout &layout, hipStream_t st) {
   return timing_end(slot, st, kSpan, flops);
 }
 
-// SMX_S8_FP32 runs on FP16 pairs (kS8Pair) unless there is a class of 16-bit
-// parameters, or a matrix of up to 32 rows is wider than 256: the pairs' 22 bits
-// cost more there than the longer accumulation of FP32 MFMAs (16 x 700: error
-// 7.2e-6 against 4.2e-6).  Small Gram-space classes then iterate in X-space,
-// where P comes from H = G - I: the r x r products of Gram space carry G
-// itself (100 x 1100: 5.9e-6 against FP32's 5.5e-6, X-space 3.4e-6), and a
-// short run takes fewer launches so (15 of 23).  From about 160 rows on
-// both are at or below FP32's error.
-void s8_choose_pairs(S8Layout &L) {
-  L.pairs = L.mode == SMX_S8_FP32;
-  for (int i = 0; i < L.n_classes; ++i)
-    if (L.cls[i].low || (L.cls[i].r <= 32 && L.cls[i].gs && !s8_small(L.cls[i]))) L.pairs = 0;
-  for (int i = 0; i < L.n_classes && L.pairs; ++i)
-    if (L.cls[i].r <= 160) L.cls[i].gs = 0;
-}
-
 bool plan_s8(const int64_t *r, const int64_t *c, const bool *flips, const bool *low, int32_t n, int mode, char *base,
              S8Plan &plan, int32_t *cls_of, int32_t *slot_of) {
   S8Layout &Lay = plan.layout;
@@ -2395,6 +2471,21 @@ bool plan_s8(const int64_t *r, const int64_t *c, const bool *flips, const bool *
     C.cst = reinterpret_cast<double *>(take(static_cast<size_t>(C.count) * kCst * sizeof(double)));
     C.colv = reinterpret_cast<const float **>(take(static_cast<size_t>(C.count) * 2 * sizeof(float *)));
     C.mrp = reinterpret_cast<float *>(take(static_cast<size_t>(C.count) * 3 * (C.rp * C.cp / kStripT) * sizeof(float)));
+    // SMX_S8_FP32: pairs where their map is no further from FP64 than FP32
+    // MFMAs'.  From 160 rows on that is so in either form (192 x 600: error
+    // 5.5e-6 against 6.2e-6, 768 x 3000 7.6e-6 against 1.0e-5).  Smaller
+    // Gram-space classes iterate in X-space, where P comes from H = G - I (the
+    // r x r products of Gram space carry G itself: 100 x 1100 5.9e-6 against
+    // 5.5e-6, X-space 4.5e-6), while their five Grams' longer sums cost less
+    // than that gains: from 65 rows and up to 12 times as many columns, 20 from
+    // 129 rows (96 x 600 3.6e-6 against 5.3e-6, 128 x 1200 4.4e-6 against
+    // 5.5e-6, 160 x 3000 5.7e-6 against 6.4e-6; but 64 x 1200 5.7e-6 against
+    // 4.7e-6, 96 x 3000 7.6e-6 against 6.2e-6, 128 x 2000 6.2e-6 against
+    // 5.6e-6).  The others run on FP32 MFMAs.
+    if (mode == SMX_S8_FP32) {
+      C.wide = C.low || (C.gs && C.r <= 160 && (C.r <= 64 || C.c > (C.r <= 128 ? 12 : 20) * C.r)) ? 1 : 0;
+      if (!C.wide && C.r <= 160) C.gs = 0;
+    }
   }
   plan.bytes = off;
   return true;

@@ -85,7 +85,10 @@ __global__ void __launch_bounds__(256) s8_load_total_kernel(S8IoArgs a, int32_t 
   double s = 0.0;
   for (int32_t i = threadIdx.x; i < n; i += 256) s += M.fro()[i];
   s = block_sum(s, scratch);
-  if (threadIdx.x == 0) M.cst()[kCstFro] = s;
+  if (threadIdx.x == 0) {
+    M.cst()[kCstFro] = s;
+    M.cst()[kCstWide] = 0.0;
+  }
 }
 
 // Store: final iterate (parameter layout) -> out (strided), four columns
@@ -147,7 +150,6 @@ extern "C" int smx_s8(const float *x, float *out, int64_t batch, int64_t rows, i
   S8Plan plan;
   plan_single(batch, rows, cols, mode, static_cast<char *>(workspace), plan);
   SMX_REQUIRE(workspace_bytes >= plan.bytes, SMX_EWORKSPACE, "s8: workspace too small");
-  s8_choose_pairs(plan.layout);
   hipStream_t st = static_cast<hipStream_t>(stream);
   S8IoArgs a{};
   a.k = plan.layout.cls[0];

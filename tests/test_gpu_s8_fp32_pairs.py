@@ -1,4 +1,5 @@
-"""The fp32 mode's FP16 pairs: accuracy against the FP64 map and range.
+"""The fp32 mode: FP16 pairs, and FP32 MFMAs for matrices whose rows, columns
+or blocks lie far apart in scale; accuracy against the FP64 map and range.
 
 A pair carries 22 significant bits and every product FP32 accumulation, so
 the map's error is that of FP32 GEMMs: a few 1e-6 on scaled Gaussian
@@ -11,6 +12,7 @@ import pytest
 import torch
 
 from oracle import sandmuon_oracle as O
+from sandmuon_amd import _native
 from sandmuon_amd.optimizer import _s8_fp32
 
 pytestmark = pytest.mark.gpu
@@ -47,6 +49,70 @@ def test_fp32_mode_ignores_powers_of_two(device, shape, k):
     # The input's exponent is folded into the scales exactly.
     x = _input(shape, "scaled", 5).to(device)
     assert torch.equal(_s8_fp32(x * math.ldexp(1.0, k)), _s8_fp32(x))
+
+
+# One block, X-space, Gram space and transposed, the classes of few rows.  FP32
+# MFMAs measured 3e-6 at every scale: each product carries 2^-24 of itself,
+# and every term of a scaled row, column or block has its scale.  (2^-11:
+# still pairs, 2^-39 of the operand's scale in every element.)
+@pytest.mark.parametrize("shape", [(40, 60), (256, 256), (300, 280), (200, 700), (700, 200), (90, 600), (20, 2400)])
+@pytest.mark.parametrize("scale", [2 ** -11, 2 ** -13, 1e-6, 1e-9, 1e-12, 1e-18])
+def test_fp32_mode_keeps_small_rows_columns_and_blocks(device, shape, scale):
+    x = torch.randn(3, *shape, generator=torch.Generator().manual_seed(sum(shape)))
+    h, w = shape[0] // 2, shape[1] // 2
+    x[0, 5] *= scale
+    x[1, :, 9] *= scale
+    x[2, :h, w:] *= scale
+    x[2, h:, :w] *= scale
+    want = O.s8(x.double())
+    got = _s8_fp32(x.to(device)).cpu().double()
+    # (a block's coupling passes through three products with it)
+    for a, b, tol in ((got[0, 5], want[0, 5], 2e-5), (got[1, :, 9], want[1, :, 9], 2e-5),
+                      (got[2, :h, w:], want[2, :h, w:], 2e-4), (got[2, h:, :w], want[2, h:, :w], 2e-4)):
+        assert ((a - b).norm() / b.norm()).item() <= tol
+
+
+@pytest.mark.parametrize("shape", [(300, 280), (200, 700), (700, 300)])
+def test_fp32_mode_wide_matrices_in_a_batch(device, shape):
+    """Each matrix has the bits it has alone, in every geometry."""
+    x = torch.randn(12, *shape, generator=torch.Generator().manual_seed(sum(shape)))
+    x[1::2, 7] *= 1e-7
+    x = x.to(device)
+    out = _s8_fp32(x)
+    for policy in (0, 2):
+        prev = _native.s8_tile_geometry(policy)
+        try:
+            for i in range(4):
+                assert torch.equal(out[i], _s8_fp32(x[i]))
+        finally:
+            _native.s8_tile_geometry(prev)
+
+
+def test_fp32_arithmetic_does_not_depend_on_a_narrow_neighbour(device):
+    """A 16 x 2304 matrix, too wide for one block, beside a 768 x 768 one."""
+    def step(shapes):
+        g = torch.Generator().manual_seed(7)
+        descs, keep = [], []
+        for r, c in shapes:
+            t = lambda *s: torch.randn(*s, generator=g).to(device)
+            w, gr, m = t(r, c) * .02, t(r, c), torch.zeros(r, c, device=device)
+            ir, ic = t(r).abs() + .5, t(c).abs() + .5
+            keep.append((w.clone(), w, gr, m, ir, ic))
+            descs.append(_native.MatrixDesc(
+                param=w.data_ptr(), grad=gr.data_ptr(), momentum=m.data_ptr(), inv_row=ir.data_ptr(),
+                inv_col=ic.data_ptr(), rows=r, cols=c, lr=1e-2, momentum_beta=.8))
+        ws = torch.empty(_native.matrix_step_workspace_bytes(shapes, 0), dtype=torch.uint8, device=device)
+        _native.matrix_step(descs, 0, ws)
+        torch.cuda.synchronize()
+        return keep
+
+    alone, both = step([(768, 768)]), step([(768, 768), (16, 2304)])
+    assert torch.equal(alone[0][1], both[0][1])
+    for w0, w, gr, _, ir, ic in both:
+        v = O.s8((gr.double() * ir.double()[:, None] * ic.double()).cpu()[None])[0].to(device)
+        u = v * ir.double()[:, None] * ic.double()
+        u *= 1e-2 * math.sqrt(w.shape[0]) / u.norm()
+        assert ((w0.double() - w.double() - u).norm() / u.norm()).item() <= 1e-4
 
 
 def test_fp32_mode_keeps_non_finite_inputs_visible(device):

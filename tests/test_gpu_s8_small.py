@@ -78,7 +78,7 @@ def test_small_and_large_classes_in_one_matrix_step(device, mode):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("mode", [0, 1, 2])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_mixed_parameter_types_in_one_matrix_step(device, mode, dtype):
     """An FP32 parameter's update has the same bits beside 16-bit parameters of
