@@ -422,7 +422,7 @@ int32_t smx_s8_timing_tiles(int32_t *rows, int32_t *cols, int32_t capacity);
  *   (:48-60, order 1) on a contiguous batch [batch, rows, cols] of `dtype`;
  *   both sides may carry a rank-one term.  li/lz are [batch, rows], ri/rz
  *   [batch, cols], lc/rc [batch] (device, `dtype`).  `work` holds
- *   batch*(rows+cols) doubles.  out must not alias x.
+ *   batch*cols doubles.  out must not alias x.
  * smx_graft: _graft_direction (:63-66) on n contiguous fp32 values (the
  *   reference grafts in float32 whatever the input dtype):
  *   out = x*sqrt(output_rows)/max(||x||_F, FLT_MIN); a zero input gives a

@@ -516,7 +516,7 @@ def rank1_apply(x: torch.Tensor, out: torch.Tensor, left, right, order: int) -> 
     b, r, c = x.shape
     li, lz, lc = left
     ri, rz, rc_ = right
-    work = torch.empty(max(b * (r + c), 1), dtype=torch.float64, device=x.device)
+    work = torch.empty(max(b * c, 1), dtype=torch.float64, device=x.device)
     shared = (1 if li.dim() == 1 else 0) | (2 if ri.dim() == 1 else 0)
     rc = lib().smx_rank1_apply_shared(helper_dtype_code(x.dtype), x.data_ptr(), out.data_ptr(), b, r, c,
                                       li.data_ptr(), lz.data_ptr(), lc.data_ptr(), ri.data_ptr(), rz.data_ptr(),

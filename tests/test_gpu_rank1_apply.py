@@ -1,6 +1,6 @@
 """smx_rank1_apply at the edges of its column tiles (32), row groups (32, four
-rows in flight) and row loops (64 columns, four in flight), against the same
-formula in float64.  The bound: FP64 sums, so an element carries the few
+rows in flight) and row loops (rounds of eight columns for each of a row's 64
+or 256 lanes: 512 or 2048 columns), against the same formula in float64.  The bound: FP64 sums, so an element carries the few
 FP32 roundings of its own expression (eps32 = 6e-8 each)."""
 import pytest
 import torch
@@ -30,6 +30,28 @@ def test_rank1_apply_edges(device, dtype, tol, shape):
         one = lambda f: tuple(t[k].double() for t in f)
         want = O.rank1_mapback(x[k].double(), one(left), one(right))
         assert (got[k] - want).norm() <= tol * want.norm()
+
+
+# Rows of several rounds, which are read again for the output: four waves per
+# row from 2049 columns on, one wave (more than 65536 rows) from 513
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-6), (torch.float64, 1e-13)])
+@pytest.mark.parametrize("shape", [(2, 6, 2047), (2, 6, 2048), (2, 6, 2049), (2, 5, 4100), (1, 65537, 512),
+                                   (1, 65537, 513)])
+def test_rank1_apply_long_rows(device, dtype, tol, shape):
+    b, r, c = shape
+    g = torch.Generator().manual_seed(r + c)
+    x = torch.randn(shape, generator=g, dtype=dtype)
+    fac = lambda n: (torch.rand(b, n, generator=g, dtype=dtype) + .5,
+                     torch.randn(b, n, generator=g, dtype=dtype) / n ** .5, -torch.rand(b, generator=g, dtype=dtype) * .5)
+    left, right = fac(r), fac(c)
+    for fn, oracle in ((rank1_whiten, O.rank1_whiten), (rank1_mapback, O.rank1_mapback)):
+        got = fn(x.to(device), left, right).cpu().double()
+        for k in range(b):
+            one = lambda f: tuple(t[k].double() for t in f)
+            want = oracle(x[k].double(), one(left), one(right))
+            assert (got[k] - want).norm() <= tol * want.norm()
+            # the last round's columns by themselves
+            assert (got[k, :, -1] - want[:, -1]).norm() <= 10 * tol * want[:, -1].norm()
 
 
 @pytest.mark.parametrize("shared", ["left", "right", "both"])
