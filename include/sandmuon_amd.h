@@ -67,7 +67,7 @@ enum smx_dtype { SMX_F32 = 0, SMX_BF16 = 1, SMX_F16 = 2, SMX_F64 = 3 };
  *   accuracy: a matrix in which 16 neighbours of a row or column are all
  *   below 2^-12 of its root mean square (zeros apart) runs on FP32 operands
  *   and v_mfma_f32_32x32x2_f32, as its own data decide on the device.  So do
- *   matrices of few rows and many columns (plan_s8), and those of 16-bit
+ *   matrices of up to 32 rows that are wider than 256, and those of 16-bit
  *   parameters, whose bits a matrix step keeps.
  * SMX_S8_COMP_BF16: every product as three BF16 MFMAs on hi/lo splits
  *   (hi*lo + lo*hi + hi*hi, FP32 accumulation); intermediates are stored as

@@ -44,11 +44,12 @@
 //                     two into FP16's range (kExpX ...), an FP16 pair hi + lo
 //                     of 22 significant bits in the place of FP32's 24; acc
 //                     += lo*hi + hi*lo + hi*hi with v_mfma_f32_32x32x16_f16
-//                     and FP32 accumulation.  One rounding of the accumulator
-//                     per 16 products instead of one per two makes the map
-//                     no further from FP64 than the FP32 MFMAs, at a fifth
-//                     of their matrix cycles (36 matrices of 768 x 768:
-//                     2755 -> 1175 us a call; error 4.4e-6 -> 2.4e-6).
+//                     and FP32 accumulation, the corrections in accumulators
+//                     of their own (lo_apart).  One rounding of the main
+//                     accumulator per 16 products instead of one per two
+//                     makes the map no further from FP64 than the FP32 MFMAs,
+//                     at a fifth of their matrix cycles (36 matrices of 768 x
+//                     768: 2755 -> 1190 us a call; error 4.4e-6 -> 1.6e-6).
 //                     One exponent serves a whole matrix, so a matrix whose
 //                     rows, columns or blocks lie far apart in scale runs on
 //                     FP32 operands and v_mfma_f32_32x32x2_f32 instead, as
@@ -696,7 +697,8 @@ __device__ __forceinline__ f16x8 as_f16(bf16x8 v) { return __builtin_bit_cast(f1
 
 // MFMAs of row block i: acc[i][j] += A_i B_j^T over the stage's K.
 template <int MODE, int N>
-__device__ __forceinline__ void mma_row(const AFrag<MODE> &a, const BFrags<MODE, N> &b, f32x16 (&acc)[N]) {
+__device__ __forceinline__ void mma_row(const AFrag<MODE> &a, const BFrags<MODE, N> &b, f32x16 (&acc)[N],
+                                        f32x16 (&lo)[N]) {
   // (B first: the accumulator holds C^T = B A^T, lane r of it row r of C.)
   if constexpr (is_comp(MODE)) {
     // Corrections first, then hi*hi.
@@ -710,13 +712,14 @@ __device__ __forceinline__ void mma_row(const AFrag<MODE> &a, const BFrags<MODE,
 #pragma unroll
     for (int j = 0; j < N; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], a.h, acc[j], 0, 0, 0);
   } else if constexpr (MODE == kS8Pair) {
-    // The same on FP16 pairs (lo*lo, 2^-24 of the product, is left out).
+    // The same on FP16 pairs (lo*lo, 2^-24 of the product, is left out), the
+    // corrections to `lo`.
 #pragma unroll
     for (int j = 0; j < N; ++j)
-      acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.l[j]), as_f16(a.h), acc[j], 0, 0, 0);
+      lo[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.l[j]), as_f16(a.h), lo[j], 0, 0, 0);
 #pragma unroll
     for (int j = 0; j < N; ++j)
-      acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.h[j]), as_f16(a.l), acc[j], 0, 0, 0);
+      lo[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.h[j]), as_f16(a.l), lo[j], 0, 0, 0);
 #pragma unroll
     for (int j = 0; j < N; ++j)
       acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(b.h[j]), as_f16(a.h), acc[j], 0, 0, 0);
@@ -797,7 +800,7 @@ __device__ __forceinline__ AFrag<MODE> one_hot(float s, int r0) {
 // and its second 16 K (rows 16 .. 31); FP32 one product.
 template <int MODE, int N>
 __device__ __forceinline__ void mma_one_hot(const SelScalar &sel_s, int sel, const BFrags<MODE, N> &b,
-                                            f32x16 (&acc)[N]) {
+                                            f32x16 (&acc)[N], f32x16 (&lo)[N]) {
   const float s = sel_s.s;
   if constexpr (MODE == kS8F16) {
     const AFrag<MODE> o0 = one_hot<MODE>(s, 0), o1 = one_hot<MODE>(s, 16);
@@ -826,9 +829,9 @@ __device__ __forceinline__ void mma_one_hot(const SelScalar &sel_s, int sel, con
     for (int j = 0; j < N; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.l[j], r.l, acc[j], 0, 0, 0);
 #pragma unroll
     for (int j = 0; j < N; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.h[j], r.h, acc[j], 0, 0, 0);
-    mma_row<MODE>(o, b, acc);
+    mma_row<MODE>(o, b, acc, lo);
   } else {
-    mma_row<MODE>(one_hot<MODE>(s, (sel & 1) * 16), b, acc);
+    mma_row<MODE>(one_hot<MODE>(s, (sel & 1) * 16), b, acc, lo);
   }
 }
 
@@ -898,7 +901,7 @@ template <int MODE, class G, int SEL, int PAR, bool STEADY, bool BKM>
 __device__ __forceinline__ void pipe_iter(const Opnd &A, const Opnd &B, const WaveOffsets<G> &o, const BkmLane &bl,
                                           uint32_t lds0, const SelScalar &sel_s, char *smem, int kt, int nk, int wm, int wn,
                                           AFrag<MODE> (&af)[G::kSubM], BFrags<MODE> (&bf)[2],
-                                          f32x16 (&acc)[G::kSubM][kSubN]) {
+                                          f32x16 (&acc)[G::kSubM][kSubN], f32x16 (&lo)[G::kSubM][kSubN]) {
   constexpr int S = G::kStages;
   const bool more = STEADY || kt + 1 < nk;
   if constexpr (STEADY) {
@@ -918,11 +921,21 @@ __device__ __forceinline__ void pipe_iter(const Opnd &A, const Opnd &B, const Wa
   // made the S8 runs 0.5-1% slower, so the waves keep the default.)
 #pragma unroll
   for (int i = 0; i < G::kSubM; ++i) {
-    mma_row<MODE>(af[i], bf[PAR], acc[i]);
+    mma_row<MODE>(af[i], bf[PAR], acc[i], lo[i]);
     if (more) load_a<MODE, G>(nxt, wm, i, af[i]);
   }
-  if constexpr (SEL >= 0) mma_one_hot<MODE>(sel_s, SEL, bf[PAR], acc[MODE == kS8F16 ? SEL : SEL >> 1]);
+  constexpr int sub = MODE == kS8F16 ? SEL : SEL >> 1;
+  if constexpr (SEL >= 0) mma_one_hot<MODE>(sel_s, SEL, bf[PAR], acc[sub], lo[sub]);
 }
+
+// Whether the corrections of FP16 pairs have accumulators of their own, added
+// at the end: the main ones are then rounded once and not three times per K
+// stage (error of 768 x 768 matrices 2.5e-6 -> 1.6e-6, of 640 x 1280 7.6e-6 ->
+// 5.2e-6).  In 64 x 64 and 128 x 128 tiles, whose kernels of that mode then
+// take two waves per SIMD, as fast as three without (0-2% over 40 shapes); the
+// 256-row tiles have no registers for them.
+template <int MODE, class G>
+constexpr bool lo_apart() { return MODE == kS8Pair && (G::kQuad || G::kSubM == 2); }
 
 // ACCG: also accumulate sel_s * G over the wave's rows (square phase; A and
 // B are the same symmetric G, K = rows of G).  BKM: B is a K-major
@@ -948,6 +961,16 @@ __device__ __forceinline__ void gemm_tile(const Opnd &A_in, const Opnd &B_in, in
     for (int j = 0; j < kSubN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  constexpr bool kLo = lo_apart<MODE, G>();
+  f32x16 lo_regs[kSubM][kSubN];
+  f32x16(&lo)[kSubM][kSubN] = kLo ? lo_regs : acc;
+  if constexpr (kLo)
+#pragma unroll
+    for (int i = 0; i < kSubM; ++i)
+#pragma unroll
+      for (int j = 0; j < kSubN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) lo[i][j][e] = 0.f;
   const int nk = static_cast<int>(K / (kBK * kU));
   WaveOffsets<G> o;
   o.a = tile_offsets<G::kLoadsA>(A.ld, arow0, wave);
@@ -970,7 +993,7 @@ __device__ __forceinline__ void gemm_tile(const Opnd &A_in, const Opnd &B_in, in
 #pragma unroll
   for (int i = 0; i < kSubM; ++i) load_a<MODE, G>(smem, wm, i, af[i]);
 #define SMX_PIPE(SEL, PAR, KT, STEADY) \
-  pipe_iter<MODE, G, SEL, PAR, STEADY, BKM>(A, B, o, bl, lds0, sel_s, smem, KT, nk, wm, wn, af, bf, acc)
+  pipe_iter<MODE, G, SEL, PAR, STEADY, BKM>(A, B, o, bl, lds0, sel_s, smem, KT, nk, wm, wn, af, bf, acc, lo)
   // Stages [kt, to) in pairs (kt and `to` even): branch-free while a refill
   // is due, then the general form.
   const int steady_end = nk - G::kStages;
@@ -1009,6 +1032,11 @@ __device__ __forceinline__ void gemm_tile(const Opnd &A_in, const Opnd &B_in, in
   run(kt, nk);
 #undef SMX_PIPE
   block_barrier();
+  if constexpr (kLo)
+#pragma unroll
+    for (int i = 0; i < kSubM; ++i)
+#pragma unroll
+      for (int j = 0; j < kSubN; ++j) acc[i][j] += lo[i][j];
 }
 
 // The same product for a 64 x 64 tile of four 32 x 32 waves (kGeoT), each
@@ -1030,9 +1058,11 @@ __device__ __forceinline__ void gemm_tile_quad(const Opnd &A_in, const Opnd &B_i
   const Opnd A{uniform_ptr(A_in.p), A_in.ld / kU}, B{uniform_ptr(B_in.p), B_in.ld / kU};
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wm = wave / G::kWavesN, wn = wave % G::kWavesN;
-  f32x16 c[1];
+  f32x16 c[1], lo_regs[1];
+  constexpr bool kLo = lo_apart<MODE, G>();
+  f32x16(&lo)[1] = kLo ? lo_regs : c;
 #pragma unroll
-  for (int e = 0; e < 16; ++e) c[0][e] = 0.f;
+  for (int e = 0; e < 16; ++e) c[0][e] = lo[0][e] = 0.f;
   // K is a multiple of 256: np, the slots' worth of K, is at least 4.
   const int np = static_cast<int>(K / (2 * kBK * kU));
   WaveOffsets<G> o;
@@ -1083,9 +1113,9 @@ __device__ __forceinline__ void gemm_tile_quad(const Opnd &A_in, const Opnd &B_i
     if (more) read(p + 1, fr[par ^ 1]);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      mma_row<MODE, 1>(fr[par].a[s], fr[par].b[s], c);
+      mma_row<MODE, 1>(fr[par].a[s], fr[par].b[s], c, lo);
       if constexpr (ACCG)
-        if (F16 ? 2 * p + s == kt0 : 2 * p == kt0) mma_one_hot<MODE, 1>(sel_s, s, fr[par].b[s], c);
+        if (F16 ? 2 * p + s == kt0 : 2 * p == kt0) mma_one_hot<MODE, 1>(sel_s, s, fr[par].b[s], c, lo);
     }
   };
   for (int p = 0; p < np; p += 2) {  // np is even
@@ -1093,6 +1123,7 @@ __device__ __forceinline__ void gemm_tile_quad(const Opnd &A_in, const Opnd &B_i
     step(p + 1, std::integral_constant<int, 1>{});
   }
   block_barrier();
+  if constexpr (kLo) c[0] += lo[0];
   acc[0][0] = c[0];
   if (BKM && pairs) {
     // the blocks to LDS, [block][register quad][lane], and back to their wave
@@ -1724,7 +1755,8 @@ __device__ __forceinline__ void stage_tile(const StageArgs &args, char *smem, do
 
 template <int MODE, int PHASE, int TM, int TN>
 __global__ void __launch_bounds__((Geo<TM, TN>::kThreads))
-__attribute__((amdgpu_waves_per_eu(Geo<TM, TN>::kWavesPerEU, Geo<TM, TN>::kWavesPerEU)))
+__attribute__((amdgpu_waves_per_eu(MODE == kS8Pair ? 2 : Geo<TM, TN>::kWavesPerEU,
+                                   MODE == kS8Pair ? 2 : Geo<TM, TN>::kWavesPerEU)))
 s8_stage_kernel(StageArgs args) {
   __shared__ __attribute__((aligned(16))) char smem[Geo<TM, TN>::kRingBytes];
   __shared__ double dscratch[16];
@@ -2472,18 +2504,16 @@ bool plan_s8(const int64_t *r, const int64_t *c, const bool *flips, const bool *
     C.colv = reinterpret_cast<const float **>(take(static_cast<size_t>(C.count) * 2 * sizeof(float *)));
     C.mrp = reinterpret_cast<float *>(take(static_cast<size_t>(C.count) * 3 * (C.rp * C.cp / kStripT) * sizeof(float)));
     // SMX_S8_FP32: pairs where their map is no further from FP64 than FP32
-    // MFMAs'.  From 160 rows on that is so in either form (192 x 600: error
-    // 5.5e-6 against 6.2e-6, 768 x 3000 7.6e-6 against 1.0e-5).  Smaller
-    // Gram-space classes iterate in X-space, where P comes from H = G - I (the
-    // r x r products of Gram space carry G itself: 100 x 1100 5.9e-6 against
-    // 5.5e-6, X-space 4.5e-6), while their five Grams' longer sums cost less
-    // than that gains: from 65 rows and up to 12 times as many columns, 20 from
-    // 129 rows (96 x 600 3.6e-6 against 5.3e-6, 128 x 1200 4.4e-6 against
-    // 5.5e-6, 160 x 3000 5.7e-6 against 6.4e-6; but 64 x 1200 5.7e-6 against
-    // 4.7e-6, 96 x 3000 7.6e-6 against 6.2e-6, 128 x 2000 6.2e-6 against
-    // 5.6e-6).  The others run on FP32 MFMAs.
+    // MFMAs': from 160 rows on in either form (192 x 600: error 4.5e-6 against
+    // 6.2e-6, 768 x 3000 5.3e-6 against 1.0e-5).  Smaller Gram-space classes
+    // iterate in X-space, where P comes from H = G - I (the r x r products of
+    // Gram space carry G itself), and a short run takes fewer launches so (15
+    // of 23): 48 x 1200 5.0e-6 against 5.8e-6, 64 x 3000 6.2e-6 against 6.9e-6,
+    // 128 x 1200 3.2e-6 against 5.5e-6.  Up to 32 rows that are wider than 256
+    // run on FP32 MFMAs, the pairs' 22 bits costing more there than the longer
+    // accumulation (16 x 700: 7.2e-6 against 4.2e-6).
     if (mode == SMX_S8_FP32) {
-      C.wide = C.low || (C.gs && C.r <= 160 && (C.r <= 64 || C.c > (C.r <= 128 ? 12 : 20) * C.r)) ? 1 : 0;
+      C.wide = C.low || (C.gs && C.r <= 32) ? 1 : 0;
       if (!C.wide && C.r <= 160) C.gs = 0;
     }
   }

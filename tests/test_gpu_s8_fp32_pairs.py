@@ -43,6 +43,22 @@ def test_fp32_mode_against_fp64(device, shape, kind, tol):
     assert err <= tol
 
 
+# Gaussian matrices with row and column scales a decade each way, against the
+# error of FP32 MFMAs on FP32 operands on such matrices (their mean over
+# seeds): alone and in a batch of 128 x 128 tiles, Gram space, few rows
+@pytest.mark.parametrize("shape,fp32", [((1, 768, 768), 4.5e-6), ((30, 768, 768), 4.5e-6), ((3, 640, 1280), 1.0e-5),
+                                        ((3, 64, 3000), 6.9e-6), ((3, 128, 600), 5.7e-6), ((2, 192, 1200), 5.6e-6)])
+def test_fp32_mode_is_no_further_from_fp64_than_fp32_mfmas(device, shape, fp32):
+    err = 0.0
+    for seed in range(4):
+        g = torch.Generator(device=device).manual_seed(seed)
+        f = lambda *s: torch.exp(torch.empty(*s, device=device).uniform_(-2.3, 2.3, generator=g))
+        x = torch.randn(shape, generator=g, device=device) * f(*shape[:2], 1) * f(shape[0], 1, shape[2])
+        want = O.s8(x[:3].double().cpu())
+        err += ((_s8_fp32(x)[:3].double().cpu() - want).norm() / want.norm()).item() / 4
+    assert err <= fp32
+
+
 @pytest.mark.parametrize("shape", [(2, 130, 150), (2, 90, 700)])
 @pytest.mark.parametrize("k", [-60, -20, 30, 55])
 def test_fp32_mode_ignores_powers_of_two(device, shape, k):

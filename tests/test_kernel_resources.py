@@ -39,11 +39,12 @@ def test_no_kernel_spills_or_uses_scratch():
 
 
 def test_s8_gemm_kernels_keep_their_occupancy():
-    # 128 x 128 tiles (4 waves): at most 168 VGPRs, three waves per SIMD;
+    # 128 x 128 tiles (4 waves): at most 168 VGPRs, three waves per SIMD (the
+    # FP16 pairs of mode 6, with accumulators for their corrections: two);
     # 256-row tiles: 256 VGPRs, two waves per SIMD.
     r = {k: v for k, v in report().items() if "s8_stage_kernel" in k}
     assert len(r) >= 30, sorted(r)
     for k, v in r.items():
-        small = k.endswith("Li128ELi128EEEvNS_9StageArgsE")
+        small = k.endswith("Li128ELi128EEEvNS_9StageArgsE") and "s8_stage_kernelILi6E" not in k
         assert v["occupancy"] >= (3 if small else 2), (k, v)
         assert v["vgprs"] + v["agprs"] <= (168 if small else 256), (k, v)
