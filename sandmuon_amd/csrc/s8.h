@@ -67,7 +67,8 @@ struct S8Class {
                        // class of its own, so that it is no other matrix's rule
   int32_t wide;        // SMX_S8_FP32: every matrix runs on FP32 MFMAs (plan_s8)
   // Iterate buffers (4 bytes per element), oriented layout only: tiled
-  // operands (tiled_index), FP32 in SMX_S8_FP32 mode and interleaved BF16
+  // operands (tiled_index), in SMX_S8_FP32 mode FP16 pairs (FP32 where
+  // S8Mat::wide, FP32 as the whiten or load leaves X0) and interleaved BF16
   // hi/lo (put_operand) or FP16 in the others, except the stage-5 result,
   // which is a row-major FP32 matrix.
   float *x0, *x1;      // [count][rp][cp] ping, pong (Gram space: X0, then X2)

@@ -93,7 +93,7 @@ __global__ void __launch_bounds__(256) s8_load_total_kernel(S8IoArgs a, int32_t 
 
 // Store: final iterate (parameter layout) -> out (strided), four columns
 // per thread; VEC: 16-byte stores.  (A result whose padded shape is `out`'s
-// own is written there by the last stage: direct_out.)
+// own is written there by the last stage: `direct` of smx_s8.)
 // grid = (ceil(rows * ceil(cols / 4) / 256), batch).
 template <bool VEC>
 __global__ void __launch_bounds__(256) s8_store_kernel(S8IoArgs a) {

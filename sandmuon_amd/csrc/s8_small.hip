@@ -5,7 +5,8 @@
 // A class is small when its iterate and Gram, padded to 16, fit one block's
 // LDS in FP32 (small_bytes) with at most kSmallTiles row tiles.  Every
 // product runs on FP32 MFMAs (v_mfma_f32_16x16x4_f32) whatever the mode: no
-// operand is rounded below FP32.  From stage 2 on the Gram is held as H = G
+// operand is rounded below FP32 but the input, which the other modes hand over
+// as BF16 hi + lo (16-17 bits).  From stage 2 on the Gram is held as H = G
 // - I and P formed from it (as kS8Pair does in s8.hip).  Bound by latency
 // (chains of dependent MFMAs and LDS reads between barriers), not by the
 // matrix cores' rate, up to about 64 rows.  The S8 of the 12 matrices of a

@@ -15,7 +15,8 @@ results):
 * ``s8_mode`` selects the arithmetic of the S8 products: "comp_bf16"
   (compensated BF16 MFMA in all five stages), "mixed" (compensated BF16
   stages 1-2, FP16 MFMA stages 3-5: about 1e-3 from the FP32 map at a
-  quarter less S8 time) or "fp32" (FP32 accuracy: FP16 pairs of 22 bits);
+  quarter less S8 time) or "fp32" (FP32 accuracy: FP16 pairs of 22
+  bits, FP32 MFMAs for matrices wide in range);
 * ``hook_batch_bytes``: the hooks queue their inputs and take the
   statistics of the queue in one launch once it holds this many bytes (and
   at step(), state_dict() and close()); 0 launches in every hook call.  The

@@ -1,8 +1,8 @@
 """Small matrices, whose S8 map runs whole in one block: at the edges of its
 16-row tiles, its Gram split over waves (1 to 8 row tiles), its two LDS sizes
 and the largest iterate that fits, against FP64.  Every product is FP32
-whatever the mode, so the bound is FP32's: some 1e-5 on these inputs, three
-times what they measure."""
+whatever the mode (comp_bf16 and mixed round the input to BF16 hi + lo, 2^-17
+of an element, first): some 1e-5 on these inputs, a third of the bound."""
 import math
 
 import pytest
