@@ -1889,8 +1889,8 @@ __global__ void __launch_bounds__(256) s8_poly1_kernel(StageArgs args) {
 // of zeros are exact in either form, and runs that the padding cuts short are
 // no evidence (a row or column there has whole runs across).  Gaussian matrices
 // under row and column scales a decade each way stay on pairs: their smallest
-// run is about 2^-8.
-// A pass over X0 at the copy rate (36 matrices of 768 x 768: 20 of 1170 us).
+// run is about 2^-8.  A pass over X0 at 5 TB/s (36 matrices of 768 x 768: 17 of
+// 1170 us; 32 with a piece per wave, whose column maxima cross 16-lane rows).
 constexpr float kWideRun = 1.f / 4096.f;
 __host__ __device__ inline int64_t pair_blocks_per_matrix(const S8Class &k) {
   return k.rp * k.cp / 16 / kPolyChunk;
@@ -1902,35 +1902,38 @@ __global__ void __launch_bounds__(256) s8_scan_kernel(StageArgs args) {
   const int64_t tpm = pair_blocks_per_matrix(K);
   if (ref.L >= tpm * ref.cnt || K.wide) return;
   const S8Mat M{K, ref.slot0 + static_cast<int>(ref.L / tpm)};
-  const int64_t g0 = (ref.L % tpm) * kPolyChunk, gpr = K.cp / 16;  // first group of the block, groups per row
-  const SMX_GLOBAL f32x4v *X = (const SMX_GLOBAL f32x4v *)M.x0() + g0 * 4 + threadIdx.x;
-  f32x4v x[kPolyUnits];
+  // 16 lanes a piece: load k, lane l the quarter l & 3 of row 4 k + (l >> 2), so
+  // that a column's 16 rows are in 4 lanes of one 16-lane row.
+  const int64_t piece = (ref.L % tpm) * (kPolyChunk / 16) + (threadIdx.x >> 4), gpr = K.cp / 16;
+  const SMX_GLOBAL f32x4v *X = (const SMX_GLOBAL f32x4v *)M.x0() + piece * 64 + (threadIdx.x & 15);
+  f32x4v x[4];
 #pragma unroll
-  for (int k = 0; k < kPolyUnits; ++k) x[k] = X[256 * k];  // lane l: row l >> 2 of a piece, columns 4 (l & 3) ..
+  for (int k = 0; k < 4; ++k) x[k] = X[16 * k];
   const double f = M.cst()[kCstFro];
   // (no element reaches an infinite limit: a matrix with infinities is wide)
   const float limit = static_cast<float>(sqrt(f / (static_cast<double>(K.r) * static_cast<double>(K.c)))) * kWideRun;
   auto small = [&](float m) { return m > 0.f && m < limit; };
+  const bool rows_whole = (piece / gpr + 1) * 16 <= K.r, cols_whole = (piece % gpr + 1) * 16 <= K.c;
   bool any = false;
+  float c[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int k = 0; k < kPolyUnits; ++k) {
-    const int64_t piece = (g0 + (threadIdx.x + 256 * k) / 4) / 16;  // 16 groups: 16 rows of one K group
-    const bool rows_whole = (piece / gpr + 1) * 16 <= K.r, cols_whole = (piece % gpr + 1) * 16 <= K.c;
-    float c[4], row = 0.f;
+  for (int k = 0; k < 4; ++k) {
+    float row = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      c[e] = fabsf(x[k][e]);
-      row = fmaxf(row, c[e]);
+      const float v = fabsf(x[k][e]);
+      row = fmaxf(row, v);
+      c[e] = fmaxf(c[e], v);
     }
-    row = fmaxf(row, dpp_mov<0xB1>(row));
-    row = fmaxf(row, dpp_mov<0x4E>(row));  // the row's four lanes
+    row = fmaxf(row, dpp_mov<0xB1>(row));  // the row's four lanes
+    row = fmaxf(row, dpp_mov<0x4E>(row));
     any = any || (cols_whole && small(row));
+  }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-#pragma unroll
-      for (int d = 4; d < 64; d *= 2) c[e] = fmaxf(c[e], __shfl_xor(c[e], d));
-      any = any || (rows_whole && small(c[e]));
-    }
+  for (int e = 0; e < 4; ++e) {
+    c[e] = fmaxf(c[e], dpp_mov<0x124>(c[e]));  // row_ror:4 and 8: the column's four lanes
+    c[e] = fmaxf(c[e], dpp_mov<0x128>(c[e]));
+    any = any || (rows_whole && small(c[e]));
   }
   if (any) M.cst()[kCstWide] = 1.0;  // (every writer writes the same)
 }

@@ -82,6 +82,30 @@ def test_tiled_index_is_a_bijection_keeping_row_blocks_in_place():
     assert seen == set(range(rows * ld))
 
 
+def test_scan_reads_rows_and_columns_of_a_piece():
+    """s8_scan_kernel: 16 lanes take a 16 x 16 piece of the FP32 iterate, load k
+    of lane l the 16 bytes at 1024 piece + 256 k + 16 l: row 4 k + (l >> 2),
+    columns 4 (l & 3) .. + 3.  The quads of lanes hold whole rows, and lanes
+    l, l - 4, l - 8, l - 12 of the 16 (rotations by 4, then 8) whole columns."""
+    ld = 48
+    mem = memory("f32", 32, ld)
+    for piece in range(2 * ld // 16):
+        r0, c0 = 16 * (piece // (ld // 16)), 16 * (piece % (ld // 16))
+        held = {l: {mem[1024 * piece + 256 * k + 16 * l + 4 * e]: (k, e) for k in range(4) for e in range(4)}
+                for l in range(16)}
+        for k in range(4):
+            for quad in range(4):
+                row = {el[1:] for l in range(4 * quad, 4 * quad + 4) for el, (kk, _) in held[l].items() if kk == k}
+                assert row == {(r0 + 4 * k + quad, c0 + c) for c in range(16)}
+        for l in range(16):
+            reach = {l}
+            for ror in (4, 8):
+                reach |= {(m - ror) % 16 for m in reach}
+            for e in range(4):
+                col = {el[1:] for m in reach for el, (_, ee) in held[m].items() if ee == e}
+                assert col == {(r0 + r, c0 + 4 * (l & 3) + e) for r in range(16)}
+
+
 @pytest.mark.parametrize("form", ["planes", "f32", "f16"])
 @pytest.mark.parametrize("tm,waves", [(64, 4), (128, 4), (256, 4), (256, 8)])
 def test_row_major_tile_loads(form, tm, waves):
