@@ -2112,14 +2112,17 @@ static int64_t device_cus() {
 // The tile geometry of one launch over `segs`; `every` holds its segments in
 // all launch chains of the run, which run beside it.  64 x 64 tiles (kGeoT)
 // while the launch's are at most two per CU, the blocks that a CU holds, and
-// those of all chains at most 3.2 per CU: the launch then takes the time of
-// one tile's chain, a quarter as long as a 128 x 128 tile's.  Beyond that
+// those of all chains at most 3.2 per CU, or 4 where no class has more than
+// 512 rows (the shorter a tile's K loop, the more its start and end weigh, and
+// the more these overlap in the smaller tile): the launch then takes the time
+// of one tile's chain, a quarter as long as a 128 x 128 tile's.  Beyond that
 // the larger tile's fewer operand bytes per MFMA win.  A call in us, on 128 x
 // 128 tiles and on 64 x 64: one 512 x 512 matrix 255 -> 158, one 768 x 3072
 // 462 -> 278, three 1024 x 1024 (1.7 tiles per CU) 406 -> 343; in two chains,
 // eight 768 x 768 (2.6 per CU in all) 409 -> 372, nine 768 x 3072 (3.0) 807
 // -> 710, twenty 512 x 512 (3.1) 348 -> 334, but six 1024 x 1024 (3.4) 529 ->
-// 561 and twelve 768 x 768 (3.9) 484 -> 492; with up to three tiles per CU
+// 561 and twelve 768 x 768 (3.9) 484 -> 492; the step of four 512-wide blocks
+// (24 matrices of 512 rows, 3.75) 633 -> 574; with up to three tiles per CU
 // and launch, one 2048 x 2048 (2.1) 726 -> 754 and eighteen 768 x 768 (3.0
 // per chain) 605 -> 688.  256 x 256 tiles when
 // the launch has at least 1.5 of them per CU: those blocks move a third
@@ -2135,14 +2138,17 @@ static int64_t device_cus() {
 static int pick_geo(const S8Layout &Lay, int phase, const std::vector<Seg> &segs, const std::vector<Seg> &every) {
   if (g_tile_policy == 1) return kGeoL;
   const int64_t cus = device_cus();
-  int64_t tiles[4] = {0, 0, 0, 0}, all_t = 0;
+  int64_t tiles[4] = {0, 0, 0, 0}, all_t = 0, rows = 0;
   for (const Seg &sg : segs) {
     const S8Class &k = Lay.cls[sg.cls];
     const int64_t cnt = sg.hi - sg.lo;
     for (int g = 0; g < 4; ++g) tiles[g] += cnt * phase_tiles(k, phase, g, sg.op);
   }
-  for (const Seg &sg : every) all_t += (sg.hi - sg.lo) * phase_tiles(Lay.cls[sg.cls], phase, kGeoT, sg.op);
-  if (g_tile_policy == 0 && tiles[kGeoT] <= 2 * cus && 10 * all_t <= 32 * cus) return kGeoT;
+  for (const Seg &sg : every) {
+    all_t += (sg.hi - sg.lo) * phase_tiles(Lay.cls[sg.cls], phase, kGeoT, sg.op);
+    rows = std::max(rows, Lay.cls[sg.cls].rp);
+  }
+  if (g_tile_policy == 0 && tiles[kGeoT] <= 2 * cus && 10 * all_t <= (rows <= 512 ? 40 : 32) * cus) return kGeoT;
   if (g_tile_policy == 0 && 2 * tiles[kGeoL] >= 3 * cus) return kGeoL;
   const double r_m = static_cast<double>(ceil_div(tiles[kGeoM], 2 * cus));
   const double r_s = static_cast<double>(ceil_div(tiles[kGeoS], 3 * cus));

@@ -271,13 +271,13 @@ GEOMETRY = {"64x64": (64, 64, 2), "128x128": (128, 128, 4), "256x128": (256, 128
 def expected_square_geometry(n, total, size, cus):
     """The square's geometry for a launch over n matrices of size x size, of
     `total` in all launch chains: 64 x 64 tiles when the launch has at most two
-    of them per CU and all chains at most 3.2, else 256 x 256 tiles when there
+    of them per CU and all chains at most 3.2 (4 up to 512 rows), else 256 x 256 tiles when there
     are at least 1.5 of them per CU, else 128 x 128
     tiles when they take fewer rounds of the CUs' block slots (three per CU,
     a round counted 0.9 of one of two 256 x 128 blocks), else 256 x 128."""
     t256, ts = size // 256, size // 128
     sym = lambda t: t * (t + 1) // 2
-    if 4 * n * sym(ts) <= 2 * cus and 40 * total * sym(ts) <= 32 * cus:
+    if 4 * n * sym(ts) <= 2 * cus and 40 * total * sym(ts) <= (40 if size <= 512 else 32) * cus:
         return "64x64", 4 * sym(ts)
     if 2 * n * sym(t256) >= 3 * cus:
         return "256x256", sym(t256)
@@ -287,16 +287,17 @@ def expected_square_geometry(n, total, size, cus):
 
 
 @pytest.mark.parametrize("mode", ["fp32", "comp_bf16", "mixed"])
-@pytest.mark.parametrize("batch,size,geometry", [(3, 1024, "64x64"), (3, 1280, "128x128"), (20, 512, "64x64"),
-                                                 (21, 512, "128x128"), (74, 768, "256x128"), (800, 256, "256x256")])
+@pytest.mark.parametrize("batch,size,geometry", [(3, 1024, "64x64"), (3, 1280, "128x128"), (24, 512, "64x64"),
+                                                 (26, 512, "128x128"), (9, 768, "64x64"), (10, 768, "128x128"), (74, 768, "256x128"), (800, 256, "256x256")])
 def test_s8_square_tile_geometries(device, mode, batch, size, geometry):
     """The square phase takes 64 x 64 tiles up to two per CU and launch and
-    3.2 per CU over the launch chains, else 256 x 256 tiles when the launch
+    3.2 per CU over the launch chains (4 up to 512 rows), else 256 x 256 tiles when the launch
     has at least 1.5 of them per CU, else 128 x 128 tiles when they need fewer
     rounds of the CUs' block slots, else 256 x 128 tiles.  A class of 4 or
     more matrices runs as two launch chains of halves.  On 256 CUs: 3 matrices
-    of 1024 x 1024 give 432 tiles of 64 x 64, 3 of 1280 x 1280 660; 20 of
-    512 x 512 800 in two chains, 21 840; 37 of 768 x 768 give 777 tiles of
+    of 1024 x 1024 give 432 tiles of 64 x 64, 3 of 1280 x 1280 660; 24 of
+    512 x 512 960 in two chains, 26 520 in each; 9 of 768 x 768 756 in two
+    chains, 10 840; 37 of 768 x 768 give 777 tiles of
     128 x 128 (two rounds of three per CU) against 444 of 256 x 128 (one round
     of two) and 222 of 256 x 256; 400 of 256 x 256 give 400 tiles of
     256 x 256.  Every geometry meets the gates; the recorded tiles show which
