@@ -393,8 +393,8 @@ int smx_s8(const float *x, float *out, int64_t batch, int64_t rows,
  * whole in one block each)
  * and the MFMA FLOPs the launch (or run) issues (tiles computed x
  * 2*256*256*K, x3 in SMX_S8_COMP_BF16 and SMX_S8_FP32 mode, plus the square
- * phase's one-hot MFMAs; a matrix that runs on FP32 MFMAs counts as one on
- * pairs; phase 6: the FP32 MFMAs of the small matrices).  It returns the
+ * phase's one-hot MFMAs; in SMX_S8_FP32 mode a matrix that runs on FP32 MFMAs
+ * for its range counts as one on pairs, a class that does as a whole x1; phase 6: the FP32 MFMAs of the small matrices).  It returns the
  * number of records or a negative status.
  * The recorder is process-wide, not thread-safe.
  * ------------------------------------------------------------------ */

@@ -54,8 +54,9 @@
 //                     rows, columns or blocks lie far apart in scale runs on
 //                     FP32 operands and v_mfma_f32_32x32x2_f32 instead, as
 //                     its own data decide (s8_scan_kernel; every kernel of
-//                     the mode holds both bodies), and so do the classes
-//                     whose pairs are no closer to FP64 (plan_s8).
+//                     pairs holds both bodies).  So do, in launches of
+//                     mode SMX_S8_FP32, the classes whose pairs are no
+//                     closer to FP64 (plan_s8).
 //   SMX_S8_COMP_BF16  every operand is stored by its producer as BF16 hi +
 //                     lo (put_operand); acc += hi*lo + lo*hi + hi*hi with
 //                     v_mfma_f32_32x32x16_bf16 (the compensated product of
@@ -145,7 +146,9 @@ constexpr int kMaxSeg = 2 * kMaxClasses;
 constexpr int kS8HiOnly = 3;
 constexpr int kS8F16 = 4;
 //   kS8Pair    the run mode of SMX_S8_FP32: FP16 pairs, and FP32 MFMAs (the
-//              body of mode SMX_S8_FP32) for the matrices that are wide.
+//              body of mode SMX_S8_FP32) for the matrices that are wide; a
+//              class that is wide as a whole runs in launches of mode
+//              SMX_S8_FP32, whose kernels hold that body alone.
 constexpr int kS8CompMix = 5;
 constexpr int kS8Pair = 6;
 __host__ __device__ constexpr bool is_comp(int m) { return m == SMX_S8_COMP_BF16 || m == kS8CompMix; }
@@ -186,7 +189,7 @@ __device__ __forceinline__ int s8_exp0(double fro2) {
 // The MFMA mode of one product of the map (phase, stage and, for SYM and
 // APPLY, its SegOp) under the run's public `mode` and compensation mask.
 __host__ __device__ constexpr int gemm_mode(int mode, int mask, int phase, int stage, int op, bool gs) {
-  return mode == kS8Pair ? mode
+  return mode == kS8Pair || mode == SMX_S8_FP32 ? mode
          : mode == SMX_S8_COMP_BF16 ? (((mask >> (stage - 1)) & 1) ? SMX_S8_COMP_BF16 : kS8HiOnly)
          : (stage <= 2 || gs) ? kS8CompMix
                               : kS8F16;
@@ -1328,7 +1331,9 @@ __device__ __forceinline__ void stage_tile(const StageArgs &args, char *smem, do
   f32x16 acc[kSubM][kSubN];
   // What the epilogue multiplies by; kPair: with the exponents of the FP16
   // pairs (kExpX ...) folded in.
-  constexpr bool kPair = MODE == kS8Pair, kScaled = kPair || MODE == SMX_S8_FP32;  // X0 holds V 2^k (s8_exp0)
+  constexpr bool kPair = MODE == kS8Pair;
+  // The exponent k of X0, which holds V 2^k (s8_pair0_kernel).
+  auto exp0 = [&](double fro2) { return (kPair || MODE == SMX_S8_FP32) && !K.wide ? s8_exp0(fro2) : 0; };
   // X-space pairs: from stage 2 on the Gram is stored as H = G - I and P is
   // formed from it.  The iterate's singular values approach 1, so H is small
   // where G is not: neither the rounding of a diagonal near 1 nor the
@@ -1363,7 +1368,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &args, char *smem, do
   } else if constexpr (PHASE == kGram) {
     if (stage == 1) {
       const double f = M.cst()[kCstFro];
-      scale = f > 0.0 ? static_cast<float>(kScaled ? ldexp(1.0 / f, (kPair ? kExpG : 0) - 2 * s8_exp0(f)) : 1.0 / f) : 0.f;
+      scale = f > 0.0 ? static_cast<float>(ldexp(1.0 / f, (kPair ? kExpG : 0) - 2 * exp0(f))) : 0.f;
     } else if constexpr (kPair) {
       scale = pow2f(kExpG - 2 * kExpX);
     }
@@ -1393,8 +1398,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &args, char *smem, do
     if (stage == 1 || mid) {
       const Stage1Scalars sc = stage1_scalars(M, args.sq_geo, bcast);
       const double inv = sc.ok ? 1.0 / (sqrt(sc.fro2) * static_cast<double>(sc.s)) : 0.0;
-      scale = static_cast<float>(kScaled ? ldexp(inv, (kPair ? kExpX - (mid ? kExpQ : kExpP) : 0) - s8_exp0(sc.fro2))
-                                         : inv);
+      scale = static_cast<float>(ldexp(inv, (kPair ? kExpX - (mid ? kExpQ : kExpP) : 0) - exp0(sc.fro2)));
     } else if constexpr (kPair) {
       // Q2 and Q4 are products of two P (a segment's first Q is its P);
       // the stage-5 results are FP32 without an exponent.
@@ -1900,7 +1904,7 @@ __global__ void __launch_bounds__(256) s8_scan_kernel(StageArgs args) {
   const TileRef ref = tile_of(args);
   const S8Class &K = *ref.k;
   const int64_t tpm = pair_blocks_per_matrix(K);
-  if (ref.L >= tpm * ref.cnt || K.wide) return;
+  if (ref.L >= tpm * ref.cnt) return;
   const S8Mat M{K, ref.slot0 + static_cast<int>(ref.L / tpm)};
   // 16 lanes a piece: load k, lane l the quarter l & 3 of row 4 k + (l >> 2), so
   // that a column's 16 rows are in 4 lanes of one 16-lane row.
@@ -2029,6 +2033,7 @@ struct Seg {
 // The MFMA mode of one product of a launch (gemm_mode under the run's mode
 // and the process-wide compensation mask).
 static int seg_mode(const S8Layout &Lay, int phase, int stage, const Seg &sg) {
+  if (Lay.mode == kS8Pair && Lay.cls[sg.cls].wide) return SMX_S8_FP32;
   return gemm_mode(Lay.mode, g_comp_mask, phase, stage, sg.op, Lay.cls[sg.cls].gs != 0);
 }
 
@@ -2074,9 +2079,10 @@ static std::vector<Seg> launch_segments(const S8Layout &Lay, const SlotSet &set,
 
 // MFMA FLOPs of one launch in MFMA mode `mode`: computed tiles x 2 * TM *
 // TN * K (x3 on compensated operands and FP16 pairs; what a wide matrix of
-// SMX_S8_FP32 issues in its place only the device knows), plus the square phase's one-hot MFMAs: per wave
-// and 32x32 column tile, 2 kSubM window stages of 5 (compensated), 3 (pairs)
-// or 2 (plain BF16: the scalar's hi and lo) 16-deep products, or
+// SMX_S8_FP32 issues in its place only the device knows; a wide class x1), plus
+// the square phase's one-hot MFMAs: per wave
+// and 32x32 column tile, 2 kSubM window stages of 5 (compensated), 3 (pairs), 2
+// (plain BF16: the scalar's hi and lo) or 1 (FP32) 16-deep products, or
 // kSubM stages of 4 (FP16: hi and lo over each 16 K of a 32-deep stage).
 static double launch_flops(int mode, int phase, int stage, int geo, const S8Layout &Lay,
                            const std::vector<Seg> &segs) {
@@ -2087,7 +2093,8 @@ static double launch_flops(int mode, int phase, int stage, int geo, const S8Layo
   // column tiles each (kGeoT: of four waves with half of each)
   const int waves = geo == kGeoT ? 1 : geo == kGeoL ? 8 : 4;
   const int sub_m = geo == kGeoT ? 2 : tm / 64;
-  const double onehot = mode == kS8Pair ? 6.0 * sub_m : is_comp(mode) ? 10.0 * sub_m : 4.0 * sub_m;
+  const double onehot = mode == kS8Pair ? 6.0 * sub_m : is_comp(mode) ? 10.0 * sub_m
+                        : mode == SMX_S8_FP32 ? 2.0 * sub_m : 4.0 * sub_m;
   double f = 0.0;
   for (const Seg &sg : segs) {
     const S8Class &k = Lay.cls[sg.cls];
@@ -2134,7 +2141,9 @@ static int64_t device_cus() {
 // 128 x 128 tiles when they take fewer rounds of the CUs' block slots
 // (three per CU, a round counted 0.9 of one of two 256 x 128 blocks per
 // CU), else 256 x 128 (the cfg4 applies take 128 x 128 tiles: S8 runs 2%
-// shorter than with 256 x 128).
+// shorter than with 256 x 128).  FP16 pairs fit two 128 x 128 blocks a CU;
+// counted as two, a step of nine 768-wide layers takes 2907 us and not 2765,
+// one of nine 912-wide layers 4572 and not 4646: three stays.
 static int pick_geo(const S8Layout &Lay, int phase, const std::vector<Seg> &segs, const std::vector<Seg> &every) {
   if (g_tile_policy == 1) return kGeoL;
   const int64_t cus = device_cus();
@@ -2211,7 +2220,8 @@ static int launch_phase(const S8Layout &Lay, const SlotSet &set, const SlotSet &
     if (static_cast<int>(segs.size()) > kMaxSeg) return fail(SMX_EINVAL, "s8: too many launch segments");
     if (PHASE != kPoly1)
       for (const Seg &sg : segs)
-        if (!form_compiled(mode, PHASE, out_form(Lay.mode, g_comp_mask, PHASE, stage, sg.op, Lay.cls[sg.cls].gs != 0)))
+        if (!form_compiled(mode, PHASE, out_form(mode == SMX_S8_FP32 ? mode : Lay.mode, g_comp_mask, PHASE, stage, sg.op,
+                                                 Lay.cls[sg.cls].gs != 0)))
           return fail(SMX_EINVAL, "s8: no epilogue for the output form of this product");
     const int geo =
         PHASE == kSquare ? sq_geo : PHASE == kPoly1 ? kGeoM
@@ -2238,6 +2248,8 @@ static int launch_phase(const S8Layout &Lay, const SlotSet &set, const SlotSet &
     if constexpr (PHASE == kPoly1) {
       if (mode == kS8Pair)
         hipLaunchKernelGGL(s8_poly1_kernel<kS8Pair>, dim3(off), dim3(256), 0, st, a);
+      else if (mode == SMX_S8_FP32)
+        hipLaunchKernelGGL(s8_poly1_kernel<SMX_S8_FP32>, dim3(off), dim3(256), 0, st, a);
       else
         hipLaunchKernelGGL(s8_poly1_kernel<SMX_S8_COMP_BF16>, dim3(off), dim3(256), 0, st, a);
       rc = check_launch("s8 stage-1 polynomial");
@@ -2246,7 +2258,8 @@ static int launch_phase(const S8Layout &Lay, const SlotSet &set, const SlotSet &
       else if (mode == kS8CompMix) launch_stage<kS8CompMix, PHASE>(geo, off, a, st);
       else if (mode == kS8HiOnly) launch_stage<kS8HiOnly, PHASE>(geo, off, a, st);
       else if (mode == kS8F16) launch_stage<kS8F16, PHASE>(geo, off, a, st);
-      else launch_stage<kS8Pair, PHASE>(geo, off, a, st);
+      else if (mode == kS8Pair) launch_stage<kS8Pair, PHASE>(geo, off, a, st);
+      else launch_stage<SMX_S8_FP32, PHASE>(geo, off, a, st);
       rc = check_launch(PHASE == kGram ? "s8 gram" : PHASE == kSquare ? "s8 square" : PHASE == kSym ? "s8 sym"
                                                                                                   : "s8 apply");
     }
@@ -2344,7 +2357,7 @@ static int run_s8_pair0(const S8Layout &Lay, bool small, hipStream_t st) {
   int32_t off = 0;
   for (int i = 0; i < Lay.n_classes; ++i) {
     const S8Class &k = Lay.cls[i];
-    if (!k.count || (small && s8_small(k))) continue;
+    if (!k.count || k.wide || (small && s8_small(k))) continue;
     a.seg_off[a.n_seg] = off;
     a.seg_cls[a.n_seg] = i;
     a.seg_cnt[a.n_seg++] = k.count;

@@ -131,6 +131,19 @@ def test_fp32_arithmetic_does_not_depend_on_a_narrow_neighbour(device):
         assert ((w0.double() - w.double() - u).norm() / u.norm()).item() <= 1e-4
 
 
+def test_fp32_mma_classes_record_one_product(device):
+    """A class on FP32 MFMAs as a whole (16 x 2304 here) runs in launches of its
+    own, one product per K: two Grams (Gram space: stages 1 and 3) of the upper
+    triangle of 256 x 256 in 128 x 128 tiles or their quadrants."""
+    _native.s8_timing(True)
+    try:
+        _s8_fp32(torch.randn(2, 16, 2304, device=device))
+    finally:
+        _native.s8_timing(False)
+    grams = [f for _, p, f in _native.s8_timing_read() if p == "gram"]
+    assert grams == [2 * 3 * 128 * 128 * 2 * 2304.0] * 2
+
+
 def test_fp32_mode_keeps_non_finite_inputs_visible(device):
     x = torch.randn(2, 40, 50, device=device)
     x[1, 3, 4] = float("inf")
